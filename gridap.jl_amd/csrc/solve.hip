@@ -61,81 +61,76 @@ __device__ __forceinline__ void put_partial(double v, double *part, double *sh) 
   if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
-// Σ part[0..np) in a fixed order, the same in every block.
-__device__ __forceinline__ double sum_partials(const double *__restrict__ part, int np,
-                                               double *sh) {
-  constexpr int kUnroll = 8;
-  const int T = (int)blockDim.x;
-  double a = 0.0;
-  for (int b0 = threadIdx.x; b0 < np; b0 += T * kUnroll) {
-    double w[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int b = b0 + u * T;
-      w[u] = b < np ? part[b] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) a += w[u];
-  }
-  return block_sum(a, sh);
-}
-
 // Grids of the iteration kernels are capped at kPcgGrid blocks (grid-stride loops):
 // every block of a consuming kernel re-reads all partials of its producer, so the
 // partial count, not only the row count, sets the cost of a reduction.
 constexpr int kPcgGrid = 1024;
 static_assert(kPcgGrid <= kMaxParts, "partial slots");
 
-// Σ a[0..np) and Σ b[0..np) in one pass (fixed order, the same in every block).
-__device__ __forceinline__ void sum_partials2(const double *__restrict__ a,
-                                              const double *__restrict__ b, int np, double *sh,
-                                              double &ra, double &rb) {
-  double x = 0.0, y = 0.0;
-  for (int k = threadIdx.x; k < np; k += (int)blockDim.x) {
-    x += a[k];
-    y += b[k];
+// Wave-wide sum (every lane gets it).
+__device__ __forceinline__ double wave_sum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+
+// The loads an iteration kernel starts with, issued together: the stop flag and this
+// thread's share of one or two partial arrays.  The kernel issues its first data loads
+// next, so they are in flight while the reduction below runs: an iteration kernel of a
+// small system is a chain of memory round trips (about 1 µs each), not bandwidth.
+struct StartIn {
+  double a = 0.0, b = 0.0, stop = 0.0;
+};
+
+__device__ __forceinline__ StartIn start_loads(const double *scal, const double *__restrict__ pa,
+                                               const double *__restrict__ pb, int np) {
+  constexpr int kPer = (kPcgGrid + kBlock - 1) / kBlock;  // partials per thread
+  StartIn S;
+  double va[kPer], vb[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int k = (int)threadIdx.x + u * kBlock;
+    va[u] = k < np ? pa[k] : 0.0;
+    vb[u] = pb && k < np ? pb[k] : 0.0;
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    x += __shfl_xor(x, o);
-    y += __shfl_xor(y, o);
+  S.stop = scal[kStop];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    S.a += va[u];
+    S.b += vb[u];
   }
+  return S;
+}
+
+// Σ of both partial arrays (fixed order, the same in every block) into S.a, S.b; true
+// when an earlier kernel stopped the solve.  Thread 0's flag decides for the block.
+// One barrier; sh holds 2 x kBlock/64 + 1 values and is reused by later reductions.
+__device__ __forceinline__ bool start_sums(StartIn &S, double *sh) {
+  constexpr int kW = kBlock / 64;
+  const double a = wave_sum(S.a), b = wave_sum(S.b);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  __syncthreads();
   if (lane == 0) {
-    sh[2 * w] = x;
-    sh[2 * w + 1] = y;
+    sh[2 * w] = a;
+    sh[2 * w + 1] = b;
   }
+  if (threadIdx.x == 0) sh[2 * kW] = S.stop;
   __syncthreads();
-  ra = rb = 0.0;
-  for (int k = 0; k < (int)(blockDim.x >> 6); ++k) {
-    ra += sh[2 * k];
-    rb += sh[2 * k + 1];
+  S.a = S.b = 0.0;
+#pragma unroll
+  for (int k = 0; k < kW; ++k) {
+    S.a += sh[2 * k];
+    S.b += sh[2 * k + 1];
   }
+  return sh[2 * kW] != 0.0;
 }
+constexpr int kStartLds = 2 * (kBlock / 64) + 1;
 
-// True when the solve has stopped (scal[kStop] set by an earlier kernel).  Read once
-// per workgroup and shared, so the whole workgroup returns or none of it does.
-__device__ __forceinline__ bool block_stopped(const double *scal) {
-  __shared__ int flag;
-  if (threadIdx.x == 0) flag = scal[kStop] != 0.0;
-  __syncthreads();
-  return flag != 0;
-}
-
-// Start of an iteration: r·z (for β) and, after the first iteration of a start,
-// r·r of the previous update against thr = (rtol ‖b‖)²; true when the solve stops
-// here (block 0 records why and at which iteration).  Every block sums the same
-// partials in the same order, so every block takes the same decision.
-__device__ __forceinline__ bool iteration_start(double *scal, const double *__restrict__ part_rz,
-                                                const double *__restrict__ part_rr, int np,
-                                                int first, double thr, int it, double *sh,
-                                                double &rz) {
-  double rr = 0.0;
-  if (first) {
-    rz = sum_partials(part_rz, np, sh);
-    return false;
-  }
-  sum_partials2(part_rz, part_rr, np, sh, rz, rr);
+// Convergence at the start of an iteration (after the first of a start): r·r of the
+// previous update against thr = (rtol ‖b‖)²; true when the solve stops here (block 0
+// records why and at which iteration).  Every block has summed the same partials in the
+// same order, so every block takes the same decision.
+__device__ __forceinline__ bool iteration_stops(double *scal, double rr, int first, double thr,
+                                                int it) {
+  if (first) return false;
   const bool stop = !(rr > thr) || !isfinite(rr);
   if (stop && blockIdx.x == 0 && threadIdx.x == 0) {
     scal[kStop] = isfinite(rr) ? 1.0 : 2.0;
@@ -216,11 +211,13 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_kernel(
     double *scal, int par, int first, const double *__restrict__ part_rz,
     const double *__restrict__ part_rr, int np_rz, double thr, int it,
     double *__restrict__ part_pq) {
-  __shared__ double sh[2 * (kBlock / 64)];
-  if (block_stopped(scal)) return;
-  double rz;
-  if (iteration_start(scal, part_rz, part_rr, np_rz, first, thr, it, sh, rz)) return;
-  const double beta = first ? 0.0 : rz / scal[kRz + (par ^ 1)];
+  __shared__ double sh[kStartLds];
+  StartIn S = start_loads(scal, part_rz, first ? nullptr : part_rr, np_rz);
+  const double rz_old = scal[kRz + (par ^ 1)];
+  if (start_sums(S, sh)) return;
+  const double rz = S.a;
+  if (iteration_stops(scal, S.b, first, thr, it)) return;
+  const double beta = first ? 0.0 : rz / rz_old;
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[kRz + par] = rz;
   const int sub = threadIdx.x % kSpmvLanes;
   const int64_t stride = (int64_t)gridDim.x * (kBlock / kSpmvLanes);
@@ -249,25 +246,55 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_kernel(
 }
 
 // α = r·z / p'·q; x += α p'; r -= α q; z = M r (diagonal M or none); partials of
-// r·z and r·r
+// r·z and r·r.  Two consecutive entries per thread (16-byte loads and stores: every
+// vector starts 16-byte aligned); the first pair's loads are issued before the
+// reduction that gives α.  One entry per thread and the reduction first: 6.9 µs at 64³,
+// 24.6 µs at 128³; this form 5.9 and 22.9 µs (131 MB, 5.7 TB/s).
 __global__ __launch_bounds__(kBlock) void update_kernel(
     int64_t n, int par, const double *__restrict__ dinv, double *__restrict__ x,
     double *__restrict__ r, double *__restrict__ z, const double *__restrict__ p,
     const double *__restrict__ q, const double *scal, const double *__restrict__ part_pq,
     int np_pq, double *__restrict__ part_rz, double *__restrict__ part_rr) {
-  __shared__ double sh[kBlock / 64];
-  if (block_stopped(scal)) return;
-  const double alpha = scal[kRz + par] / sum_partials(part_pq, np_pq, sh);
+  __shared__ double sh[kStartLds];
+  const int64_t n2 = n / 2, stride = (int64_t)gridDim.x * kBlock;
+  int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  double2 xi{}, ri{}, pi{}, qi{}, di{1.0, 1.0};
+  auto load = [&](int64_t k) {
+    pi = reinterpret_cast<const double2 *>(p)[k];
+    qi = reinterpret_cast<const double2 *>(q)[k];
+    ri = reinterpret_cast<const double2 *>(r)[k];
+    xi = reinterpret_cast<const double2 *>(x)[k];
+    if (dinv) di = reinterpret_cast<const double2 *>(dinv)[k];
+  };
+  StartIn S = start_loads(scal, part_pq, nullptr, np_pq);
+  const double rz_now = scal[kRz + par];
+  if (i < n2) load(i);
+  if (start_sums(S, sh)) return;
+  const double alpha = rz_now / S.a;
   double rz = 0.0, rr = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * kBlock) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    const double zi = dinv ? ri * dinv[i] : ri;
-    z[i] = zi;
-    rz += ri * zi;
-    rr += ri * ri;
+  auto one = [&](double &xv, double &rv, double pv, double qv, double dv) {
+    xv += alpha * pv;
+    rv -= alpha * qv;
+    const double zv = dinv ? rv * dv : rv;
+    rz += rv * zv;
+    rr += rv * rv;
+    return zv;
+  };
+  while (i < n2) {
+    double2 zi;
+    zi.x = one(xi.x, ri.x, pi.x, qi.x, di.x);
+    zi.y = one(xi.y, ri.y, pi.y, qi.y, di.y);
+    reinterpret_cast<double2 *>(x)[i] = xi;
+    reinterpret_cast<double2 *>(r)[i] = ri;
+    reinterpret_cast<double2 *>(z)[i] = zi;
+    i += stride;
+    if (i < n2) load(i);
+  }
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+    double xv = x[n - 1], rv = r[n - 1];
+    z[n - 1] = one(xv, rv, p[n - 1], q[n - 1], dinv ? dinv[n - 1] : 1.0);
+    x[n - 1] = xv;
+    r[n - 1] = rv;
   }
   put_partial(rz, part_rz, sh);
   put_partial(rr, part_rr, sh);
@@ -285,9 +312,11 @@ __global__ __launch_bounds__(kBlock) void update_lower_kernel(
     const double *__restrict__ p, const double *__restrict__ q, double *__restrict__ y,
     const double *scal, const double *__restrict__ part_pq, int np_pq,
     double *__restrict__ part_rr) {
-  __shared__ double sh[kBlock / 64];
-  if (block_stopped(scal)) return;
-  const double alpha = scal[kRz + par] / sum_partials(part_pq, np_pq, sh);
+  __shared__ double sh[kStartLds];
+  StartIn S = start_loads(scal, part_pq, nullptr, np_pq);
+  const double rz_now = scal[kRz + par];
+  if (start_sums(S, sh)) return;
+  const double alpha = rz_now / S.a;
   const int sub = threadIdx.x % kApplyLanes;
   const int64_t stride = (int64_t)gridDim.x * (kBlock / kApplyLanes);
   double rr = 0.0;
@@ -336,8 +365,9 @@ __global__ __launch_bounds__(kBlock) void upper_rz_kernel(
     int64_t n, const float *__restrict__ ge, const int32_t *__restrict__ gi,
     const double *__restrict__ y, const double *__restrict__ r, double *__restrict__ z,
     const double *scal, double *__restrict__ part_rz) {
-  __shared__ double sh[kBlock / 64];
-  if (block_stopped(scal)) return;
+  __shared__ double sh[kStartLds];
+  StartIn S = start_loads(scal, nullptr, nullptr, 0);
+  if (start_sums(S, sh)) return;
   const int sub = threadIdx.x % kApplyLanes;
   const int64_t stride = (int64_t)gridDim.x * (kBlock / kApplyLanes);
   double rz = 0.0;
@@ -385,7 +415,7 @@ __device__ __forceinline__ uint32_t box_valid(const Box &B, int64_t row) {
   return m;
 }
 
-__device__ __forceinline__ int64_t box_off(const Box &B, int o) {
+__host__ __device__ __forceinline__ int64_t box_off(const Box &B, int o) {
   return (int64_t)(o % 3 - 1) + B.m0 * ((o / 3) % 3 - 1) + B.m0 * B.m1 * (o / 9 - 1);
 }
 
@@ -436,119 +466,269 @@ __global__ void diag_inv_box_kernel(int64_t n, const double *__restrict__ a27,
   dinv[i] = d != 0.0 ? 1.0 / d : 1.0;
 }
 
+// The stencil kernels take tiles of kBlock consecutive rows, one row per thread.  The
+// neighbours of a tile's rows are, per dz, one run of consecutive rows (kBlock +
+// 2 (m0 + 1) of them; long rows, m0 > kBlock, take one run of kBlock + 2 per (dz, dy)),
+// so the vector they multiply goes to LDS once per tile, zero outside [0, N), and each
+// row then reads its neighbours there.  No mask is needed: a stored coefficient is zero
+// where its neighbour leaves the box, and so is the mirrored one of an upper offset (when
+// row j = i + off is a wrapped neighbour, row j's neighbour at -off leaves the box too);
+// beyond the last row the run in LDS is zero, and the coefficient address stays inside
+// the 14 arrays.  All 27 coefficient loads of a row are independent and issued together,
+// ahead of the reduction that gives β.  A row used to load coefficient and vector inside
+// the branch of each neighbour, 27 round trips one after the other: spmv_dir 22.5 µs at
+// 64³ and 181 µs at 128³ (latency), now 11.1 and 70 µs (bandwidth: 294 MB, 4.2 TB/s);
+// update_lower 10.6 -> 7.8 µs, upper_rz 6.5 -> 4.8 µs at 64³.
+// Each XCD sweeps a contiguous slab of the tiles in order, so the mirrored coefficients
+// of the next plane are in its L2 when the plane itself reads them.
+constexpr int kRunUnroll = 2;  // kBlock-strided loads of one run held in registers
+
+// Where the runs of a tile start and how a row finds its neighbours in them.  Z0: the
+// first dz of the runs, NZ: how many dz.
+template <bool WIDE, int Z0, int NZ>
+struct Runs {
+  static constexpr int kRuns = WIDE ? 3 * NZ : NZ;
+  int m0, m01, len;
+  __device__ __forceinline__ explicit Runs(const Box &B)
+      : m0((int)B.m0), m01((int)(B.m0 * B.m1)), len(run_len(B.m0)) {}
+  __host__ __device__ static int run_len(int64_t m0) {
+    return WIDE ? kBlock + 2 : kBlock + 2 * ((int)m0 + 1);
+  }
+  __device__ __forceinline__ int base(int i0, int d) const {
+    return WIDE ? i0 + (Z0 + d / 3) * m01 + (d % 3 - 1) * m0 - 1 : i0 + (Z0 + d) * m01 - m0 - 1;
+  }
+  // LDS position of neighbour (dx, dy, dz) of the tile's row t
+  __device__ __forceinline__ int at(int t, int dx, int dy, int dz) const {
+    return WIDE ? (3 * (dz - Z0) + dy + 1) * len + 1 + dx + t
+                : (dz - Z0) * len + (m0 + 1) + dy * m0 + dx + t;
+  }
+  __device__ __forceinline__ int at(int t, int o) const {
+    return at(t, o % 3 - 1, (o / 3) % 3 - 1, o / 9 - 1);
+  }
+};
+
+// The tiles of this block: first, end of the XCD's slab, step.
+struct TileRange {
+  int t, end, step;
+};
+__device__ __forceinline__ TileRange tile_range(int ntiles) {
+  constexpr int kXcds = 8;
+  const int x = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
+  const int q = ntiles / kXcds, r = ntiles % kXcds;
+  const int beg = x * q + min(x, r);
+  const int nb = ((int)gridDim.x - x + kXcds - 1) / kXcds;
+  return {beg + local, beg + q + (x < r), nb};
+}
+
+// a[j] + c b[j] (b nullptr: a[j]) over the runs of a tile, zero outside [0, n); the loads
+// and the LDS stores are two steps, so that the loads can be issued ahead of the
+// reduction that gives c.
+template <class R>
+struct RunLoads {
+  double va[R::kRuns][kRunUnroll], vb[R::kRuns][kRunUnroll];
+  __device__ __forceinline__ void issue(const R &r, const double *__restrict__ a,
+                                        const double *__restrict__ b, int i0, int n) {
+#pragma unroll
+    for (int d = 0; d < R::kRuns; ++d)
+#pragma unroll
+      for (int u = 0; u < kRunUnroll; ++u) {
+        const int k = (int)threadIdx.x + u * kBlock, j = r.base(i0, d) + k;
+        const bool in = k < r.len && j >= 0 && j < n;
+        va[d][u] = in ? a[j] : 0.0;
+        vb[d][u] = in && b ? b[j] : 0.0;
+      }
+  }
+  __device__ __forceinline__ void store(const R &r, double *dst, const double *__restrict__ a,
+                                        const double *__restrict__ b, double c, int i0, int n) {
+#pragma unroll
+    for (int d = 0; d < R::kRuns; ++d) {
+#pragma unroll
+      for (int u = 0; u < kRunUnroll; ++u) {
+        const int k = (int)threadIdx.x + u * kBlock;
+        if (k < r.len) dst[d * r.len + k] = va[d][u] + c * vb[d][u];
+      }
+      for (int k = (int)threadIdx.x + kRunUnroll * kBlock; k < r.len; k += kBlock) {
+        const int j = r.base(i0, d) + k;
+        const bool in = j >= 0 && j < n;
+        dst[d * r.len + k] = (in ? a[j] : 0.0) + c * (in && b ? b[j] : 0.0);
+      }
+    }
+  }
+};
+
+// Element i of a wave-uniform array: 32-bit byte offset (the box holds < 2^28 rows).
+template <class T>
+__device__ __forceinline__ T at32(const T *p, uint32_t i) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + i * (uint32_t)sizeof(T));
+}
+
 // stencil form of spmv_dir_kernel
+template <bool WIDE>
 __global__ __launch_bounds__(kBlock) void spmv_dir_box_kernel(
-    Box B, const double *__restrict__ a27, const double *__restrict__ z,
+    Box B, int ntiles, const double *__restrict__ a27, const double *__restrict__ z,
     const double *__restrict__ pold, double *__restrict__ pnew, double *__restrict__ q,
     double *scal, int par, int first, const double *__restrict__ part_rz,
     const double *__restrict__ part_rr, int np_rz, double thr, int it,
     double *__restrict__ part_pq) {
-  __shared__ double sh[2 * (kBlock / 64)];
-  if (block_stopped(scal)) return;
-  double rz;
-  if (iteration_start(scal, part_rz, part_rr, np_rz, first, thr, it, sh, rz)) return;
-  const double beta = first ? 0.0 : rz / scal[kRz + (par ^ 1)];
+  extern __shared__ __align__(16) double run[];
+  __shared__ double sh[kStartLds];
+  using R = Runs<WIDE, -1, 3>;
+  const R runs(B);
+  const int n = (int)B.n;
+  const double *pb = first ? nullptr : pold;
+  StartIn S = start_loads(scal, part_rz, first ? nullptr : part_rr, np_rz);
+  const double rz_old = scal[kRz + (par ^ 1)];
+  TileRange T = tile_range(ntiles);
+  RunLoads<R> L;
+  double a[27];
+  auto loads = [&](int t) {
+    const int i0 = t * kBlock;
+    L.issue(runs, z, pb, i0, n);
+    const uint32_t i = (uint32_t)min(i0 + (int)threadIdx.x, n - 1);
+#pragma unroll
+    for (int o = 0; o < 27; ++o)  // an upper offset's entry is row j's at the mirrored one
+      a[o] = o <= 13 ? at32(a27 + (int64_t)o * n, i)
+                     : at32(a27 + (int64_t)(26 - o) * n + box_off(B, o), i);
+  };
+  if (T.t < T.end) loads(T.t);
+  if (start_sums(S, sh)) return;
+  const double rz = S.a;
+  if (iteration_stops(scal, S.b, first, thr, it)) return;
+  const double beta = first ? 0.0 : rz / rz_old;
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[kRz + par] = rz;
   double dot = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < B.n;
-       i += (int64_t)gridDim.x * kBlock) {
-    const uint32_t vm = box_valid(B, i);
+  for (; T.t < T.end;) {
+    const int i0 = T.t * kBlock, i = i0 + (int)threadIdx.x;
+    L.store(runs, run, z, pb, beta, i0, n);
+    __syncthreads();
     double s = 0.0;
-    // (a branch-free form, reading row i for neighbours outside the box, needs 149
-    // VGPRs and ran 28 µs instead of 23 µs at N = 250,047)
 #pragma unroll
-    for (int o = 0; o < 27; ++o) {
-      if (!((vm >> o) & 1u)) continue;
-      const int64_t j = i + box_off(B, o);
-      const double pj = first ? z[j] : z[j] + beta * pold[j];
-      // A(i, j) for an upper offset is A(j, i), row j's lower entry at offset 26 - o
-      const double a = o <= 13 ? a27[(int64_t)o * B.n + i] : a27[(int64_t)(26 - o) * B.n + j];
-      s += a * pj;
+    for (int o = 0; o < 27; ++o) s += a[o] * run[runs.at(threadIdx.x, o)];
+    const double pn = run[runs.at(threadIdx.x, 13)];
+    if (i < n) {
+      pnew[i] = pn;
+      q[i] = s;
+      dot += pn * s;
     }
-    const double pn = first ? z[i] : z[i] + beta * pold[i];
-    pnew[i] = pn;
-    q[i] = s;
-    dot += pn * s;
+    T.t += T.step;
+    if (T.t < T.end) {
+      loads(T.t);
+      __syncthreads();  // the runs are read: the next tile's go in
+    }
   }
   put_partial(dot, part_pq, sh);
 }
 
-// stencil form of update_lower_kernel
+// stencil form of update_lower_kernel; START: y = G r only (start of a solve; rold = r)
+template <bool WIDE, bool START>
 __global__ __launch_bounds__(kBlock) void update_lower_box_kernel(
-    Box B, int par, const float *__restrict__ g14, double *__restrict__ x,
+    Box B, int ntiles, int par, const float *__restrict__ g14, double *__restrict__ x,
     const double *__restrict__ rold, double *__restrict__ rnew, const double *__restrict__ p,
     const double *__restrict__ q, double *__restrict__ y, const double *scal,
     const double *__restrict__ part_pq, int np_pq, double *__restrict__ part_rr) {
-  __shared__ double sh[kBlock / 64];
-  if (block_stopped(scal)) return;
-  const double alpha = scal[kRz + par] / sum_partials(part_pq, np_pq, sh);
+  extern __shared__ __align__(16) double run[];
+  __shared__ double sh[kStartLds];
+  using R = Runs<WIDE, -1, 2>;
+  const R runs(B);
+  const int n = (int)B.n;
+  const double *qb = START ? nullptr : q;
+  StartIn S;
+  double rz_now = 0.0;
+  if (!START) {
+    S = start_loads(scal, part_pq, nullptr, np_pq);
+    rz_now = scal[kRz + par];
+  }
+  TileRange T = tile_range(ntiles);
+  RunLoads<R> L;
+  float g[14];
+  double xi = 0.0, pi = 0.0;
+  auto loads = [&](int t) {
+    const int i0 = t * kBlock;
+    L.issue(runs, rold, qb, i0, n);
+    const uint32_t i = (uint32_t)min(i0 + (int)threadIdx.x, n - 1);
+#pragma unroll
+    for (int o = 0; o < 14; ++o) g[o] = at32(g14 + (int64_t)o * n, i);
+    if (!START) {
+      xi = at32(x, i);
+      pi = at32(p, i);
+    }
+  };
+  if (T.t < T.end) loads(T.t);
+  double alpha = 0.0;
+  if (!START) {
+    if (start_sums(S, sh)) return;
+    alpha = rz_now / S.a;
+  }
   double rr = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < B.n;
-       i += (int64_t)gridDim.x * kBlock) {
-    const uint32_t vm = box_valid(B, i);
+  for (; T.t < T.end;) {
+    const int i0 = T.t * kBlock, i = i0 + (int)threadIdx.x;
+    L.store(runs, run, rold, qb, -alpha, i0, n);
+    __syncthreads();
     double s = 0.0;
 #pragma unroll
-    for (int o = 0; o < 14; ++o) {
-      if (!((vm >> o) & 1u)) continue;
-      const int64_t j = i + box_off(B, o);
-      s += (double)g14[(int64_t)o * B.n + i] * (rold[j] - alpha * q[j]);
+    for (int o = 0; o < 14; ++o) s += (double)g[o] * run[runs.at(threadIdx.x, o)];
+    if (i < n) {
+      y[i] = s;
+      if (!START) {
+        const double ri = run[runs.at(threadIdx.x, 13)];
+        rnew[i] = ri;
+        x[i] = xi + alpha * pi;
+        rr += ri * ri;
+      }
     }
-    y[i] = s;
-    const double ri = rold[i] - alpha * q[i];
-    rnew[i] = ri;
-    x[i] += alpha * p[i];
-    rr += ri * ri;
-  }
-  put_partial(rr, part_rr, sh);
-}
-
-// y = G r (start of a solve), stencil form
-__global__ __launch_bounds__(kBlock) void lower_box_kernel(Box B, const float *__restrict__ g14,
-                                                           const double *__restrict__ r,
-                                                           double *__restrict__ y) {
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < B.n;
-       i += (int64_t)gridDim.x * kBlock) {
-    const uint32_t vm = box_valid(B, i);
-    double s = 0.0;
-#pragma unroll
-    for (int o = 0; o < 14; ++o) {
-      const bool in = (vm >> o) & 1u;
-      const int64_t j = in ? i + box_off(B, o) : i;
-      const double g = (double)g14[(int64_t)o * B.n + i];
-      const double rj = r[j];
-      s += in ? g * rj : 0.0;
+    T.t += T.step;
+    if (T.t < T.end) {
+      loads(T.t);
+      __syncthreads();
     }
-    y[i] = s;
   }
+  if (!START) put_partial(rr, part_rr, sh);
 }
 
 // z = Gᵀ y, partials of r·z; stencil form: entry (j, i) of G with j = i − off(o),
-// o ≤ 13, sits at g14[o·N + j], and j is in the box when the mirrored neighbour
-// 26 − o of i is
+// o ≤ 13, sits at g14[o·N + j]
+template <bool WIDE>
 __global__ __launch_bounds__(kBlock) void upper_rz_box_kernel(
-    Box B, const float *__restrict__ g14, const double *__restrict__ y,
+    Box B, int ntiles, const float *__restrict__ g14, const double *__restrict__ y,
     const double *__restrict__ r, double *__restrict__ z, const double *scal,
     double *__restrict__ part_rz) {
-  __shared__ double sh[kBlock / 64];
-  if (block_stopped(scal)) return;
+  extern __shared__ __align__(16) double run[];
+  __shared__ double sh[kStartLds];
+  using R = Runs<WIDE, 0, 2>;
+  const R runs(B);
+  const int n = (int)B.n;
+  StartIn S = start_loads(scal, nullptr, nullptr, 0);
+  TileRange T = tile_range(ntiles);
+  RunLoads<R> L;
+  float g[14];
+  double ri = 0.0;
+  auto loads = [&](int t) {
+    const int i0 = t * kBlock;
+    L.issue(runs, y, nullptr, i0, n);
+    const uint32_t i = (uint32_t)min(i0 + (int)threadIdx.x, n - 1);
+#pragma unroll
+    for (int o = 0; o < 14; ++o) g[o] = at32(g14 + (int64_t)o * n - box_off(B, o), i);
+    ri = at32(r, i);
+  };
+  if (T.t < T.end) loads(T.t);
+  if (start_sums(S, sh)) return;
   double rz = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < B.n;
-       i += (int64_t)gridDim.x * kBlock) {
-    const uint32_t vm = box_valid(B, i);
+  for (; T.t < T.end;) {
+    const int i0 = T.t * kBlock, i = i0 + (int)threadIdx.x;
+    L.store(runs, run, y, nullptr, 0.0, i0, n);
+    __syncthreads();
     double s = 0.0;
 #pragma unroll
-    for (int o = 13; o >= 0; --o) {
-      // branch-free: a neighbour outside the box reads row i itself (in bounds) and
-      // its product is replaced by 0, so all loads of the row are issued together
-      // (6.4 µs instead of 8.1 µs at N = 250,047)
-      const bool in = (vm >> (26 - o)) & 1u;
-      const int64_t j = in ? i - box_off(B, o) : i;
-      const double g = (double)g14[(int64_t)o * B.n + j];
-      const double yj = y[j];
-      s += in ? g * yj : 0.0;
+    for (int o = 13; o >= 0; --o) s += (double)g[o] * run[runs.at(threadIdx.x, 26 - o)];
+    if (i < n) {
+      z[i] = s;
+      rz += s * ri;
     }
-    z[i] = s;
-    rz += s * r[i];
+    T.t += T.step;
+    if (T.t < T.end) {
+      loads(T.t);
+      __syncthreads();
+    }
   }
   put_partial(rz, part_rz, sh);
 }
@@ -600,11 +780,11 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   }
   double *dinv = nullptr;
   const int factored = precond == GH_PRECOND_FSAI;
-  // box lattice: stencil kernels (A as 27 offset arrays, G as 14), one thread per row
+  // box lattice: stencil kernels (A as 14 offset arrays, G as 14), one thread per row
   // GRIDAP_HIP_STENCIL_PCG=0 runs the general (CSR) kernels on a box lattice too, so
   // the two forms can be compared on the same system
   const char *stencil_env = std::getenv("GRIDAP_HIP_STENCIL_PCG");
-  bool box = allow_box && c.box && n > 0 && n < (int64_t(1) << 31) &&
+  bool box = allow_box && c.box && n > 0 && n < (int64_t(1) << 28) &&
              (!factored || c.g14.get() != nullptr) && !(stencil_env && stencil_env[0] == '0');
   const Box B{n, c.box_m[0], c.box_m[1], c.box_m[2]};
   if (box) {
@@ -637,9 +817,36 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   double *part_rr = part_rz + kMaxParts, *part_bb = part_rr + kMaxParts;
   double *rbuf[2] = {V.r, factored ? V.r2 : V.r};
   double *pbuf[2] = {V.p, V.p2};
-  const unsigned g_vec = grid_rows(n, kBlock);
-  const unsigned g_spmv = box ? g_vec : grid_rows(n, kBlock / kSpmvLanes);
-  const unsigned g_apply = box ? g_vec : grid_rows(n, kBlock / kApplyLanes);
+  const int ntiles = (int)((n + kBlock - 1) / kBlock);
+  const unsigned g_vec = grid_rows((n + 1) / 2, kBlock);  // two entries per thread
+  const unsigned g_box = grid_rows(n, kBlock);            // one tile per block and turn
+  const unsigned g_spmv = box ? g_box : grid_rows(n, kBlock / kSpmvLanes);
+  const unsigned g_apply = box ? g_box : grid_rows(n, kBlock / kApplyLanes);
+  // the stencil kernels' form: one run per dz, or per (dz, dy) for long rows
+  const bool wide = B.m0 > kBlock;
+  const size_t run_bytes =
+      sizeof(double) * (wide ? 3 * Runs<true, 0, 1>::run_len(B.m0) : Runs<false, 0, 1>::run_len(B.m0));
+  auto spmv_dir_box = [&](double *pold, double *pnew, int par, int first, int np_rz, double thr,
+                          int itk) {
+    auto kern = wide ? spmv_dir_box_kernel<true> : spmv_dir_box_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(g_box), dim3(kBlock), 3 * run_bytes, s, B, ntiles, c.a27.get(),
+                       V.z, pold, pnew, V.q, scal, par, first, part_rz, part_rr, np_rz, thr, itk,
+                       part_pq);
+  };
+  auto lower_box = [&](bool start, int par, double *rold, double *rnew, double *pnew) {
+    auto kern = wide ? (start ? update_lower_box_kernel<true, true>
+                              : update_lower_box_kernel<true, false>)
+                     : (start ? update_lower_box_kernel<false, true>
+                              : update_lower_box_kernel<false, false>);
+    hipLaunchKernelGGL(kern, dim3(g_box), dim3(kBlock), 2 * run_bytes, s, B, ntiles, par,
+                       c.g14.get(), V.x, rold, rnew, pnew, V.q, V.y, scal, part_pq, (int)g_box,
+                       part_rr);
+  };
+  auto upper_box = [&](double *r) {
+    auto kern = wide ? upper_rz_box_kernel<true> : upper_rz_box_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3(g_box), dim3(kBlock), 2 * run_bytes, s, B, ntiles,
+                       c.g14.get(), V.y, r, V.z, scal, part_rz);
+  };
   // partial counts of each quantity, by producer
   const int np_rz = factored ? (int)g_apply : (int)g_vec;
   double hrr[kPcgGrid], hbb[kPcgGrid];  // g_vec <= kPcgGrid partials
@@ -654,10 +861,8 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
                        dinv, factored, rbuf[0], V.z, part_rz, part_rr, part_bb);
     hipLaunchKernelGGL(clear_stop_kernel, dim3(1), dim3(64), 0, s, scal);
     if (factored && box) {
-      hipLaunchKernelGGL(lower_box_kernel, dim3(g_apply), dim3(kBlock), 0, s, B, c.g14.get(),
-                         rbuf[0], V.y);
-      hipLaunchKernelGGL(upper_rz_box_kernel, dim3(g_apply), dim3(kBlock), 0, s, B,
-                         c.g14.get(), V.y, rbuf[0], V.z, scal, part_rz);
+      lower_box(true, 0, rbuf[0], nullptr, nullptr);
+      upper_box(rbuf[0]);
     } else if (factored) {
       hipLaunchKernelGGL(lower_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, c.gle.get(),
                          c.gli.get(), rbuf[0], V.y);
@@ -692,9 +897,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
         const int itk = it + m;
         double *pold = pbuf[par], *pnew = pbuf[par ^ 1];
         if (box)
-          hipLaunchKernelGGL(spmv_dir_box_kernel, dim3(g_spmv), dim3(kBlock), 0, s, B,
-                             c.a27.get(), V.z, pold, pnew, V.q, scal, par,
-                             k == 0 ? 1 : 0, part_rz, part_rr, np_rz, thr, itk, part_pq);
+          spmv_dir_box(pold, pnew, par, k == 0 ? 1 : 0, np_rz, thr, itk);
         else
           hipLaunchKernelGGL(spmv_dir_kernel, dim3(g_spmv), dim3(kBlock), 0, s, n,
                              c.colptr.get(), c.rowval.get(), c.nzval.get(), V.z, pold,
@@ -702,11 +905,8 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
                              np_rz, thr, itk, part_pq);
         if (factored && box) {
           double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
-          hipLaunchKernelGGL(update_lower_box_kernel, dim3(g_apply), dim3(kBlock), 0, s, B, par,
-                             c.g14.get(), V.x, rold, rnew, pnew, V.q,
-                             V.y, scal, part_pq, (int)g_spmv, part_rr);
-          hipLaunchKernelGGL(upper_rz_box_kernel, dim3(g_apply), dim3(kBlock), 0, s, B,
-                             c.g14.get(), V.y, rnew, V.z, scal, part_rz);
+          lower_box(false, par, rold, rnew, pnew);
+          upper_box(rnew);
         } else if (factored) {
           double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
           hipLaunchKernelGGL(update_lower_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, par,
