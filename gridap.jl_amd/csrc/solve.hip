@@ -35,7 +35,6 @@ namespace {
 
 constexpr int kBlock = 512;
 constexpr int kMaxParts = 8192;  // partial slots per reduced quantity (max blocks per grid)
-constexpr int kSpmvLanes = 8;    // lanes per matrix row in the SpMV
 constexpr int kApplyLanes = 4;   // lanes per row in the FSAI applications
 
 // scalar slots
@@ -144,42 +143,115 @@ inline unsigned grid_rows(int64_t rows, int rows_per_block) {
       std::max<int64_t>((rows + rows_per_block - 1) / rows_per_block, 1), kPcgGrid);
 }
 
+// ---- CSR rows --------------------------------------------------------------------------
+// L lanes take a row together, U entries per lane and turn (a turn is L·U consecutive
+// entries: coalesced values and column indices, all loads of a turn in flight before the
+// first is used).  L and U follow the mean row length (row_shape): one turn covers most
+// rows, and a wave holds 64 / L rows, so short rows leave few lanes idle and long ones
+// are no chain of dependent turns.  Eight lanes and one entry at a time, as before: 612 µs
+// at 184 entries a row (vector Q2, 32³, 1.81 GB), 50 µs at 28 (P2, 40³ x 6 tetrahedra);
+// now 385 µs (4.7 TB/s) and 31 µs.
+// The SpMV runs one workgroup per tile of rows, however many (vector Q2: 451 µs with 4096
+// workgroups, 385 µs with 50,700); the solver's kernels stay at kPcgGrid, whose partials
+// every block re-reads.  Tiles go round-robin over the XCDs: the numbering puts the
+// vertex dofs, whose rows are the longest, first, and contiguous slabs gave one XCD
+// twice the work (P2: 79 µs).
+template <int L, int U>
+struct RowTurn {
+  int32_t col[U];
+  double v[U];
+  // entries p0 + sub + L·u of [.., p1); past the end: the row's last entry with weight 0
+  __device__ __forceinline__ void load(const int32_t *__restrict__ rv,
+                                       const double *__restrict__ val, int32_t p0, int32_t p1) {
+    const int32_t p = p0 + (int32_t)(threadIdx.x % L), left = p1 - p;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int32_t k = max(p + min(u * L, left - 1), 0);
+      col[u] = rv[k];
+      v[u] = val[k];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u * L >= left) v[u] = 0.0;
+  }
+};
+
+template <int L>
+__device__ __forceinline__ double row_sum(double s) {
+#pragma unroll
+  for (int o = L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  return s;
+}
+
 // y = A x (rows from the CSC of a symmetric A).
-__global__ __launch_bounds__(kBlock) void spmv_kernel(int64_t n, const int32_t *__restrict__ cp,
+template <int L, int U>
+__global__ __launch_bounds__(kBlock) void spmv_kernel(int n,
+                                                      const int32_t *__restrict__ cp,
                                                       const int32_t *__restrict__ rv,
                                                       const double *__restrict__ val,
                                                       const double *__restrict__ x,
                                                       double *__restrict__ y) {
-  const int sub = threadIdx.x % kSpmvLanes;
-  const int64_t stride = (int64_t)gridDim.x * (kBlock / kSpmvLanes);
-  for (int64_t row = (int64_t)blockIdx.x * (kBlock / kSpmvLanes) + threadIdx.x / kSpmvLanes;
-       row < n; row += stride) {
-    double s = 0.0;
-    for (int32_t p = cp[row] + sub; p < cp[row + 1]; p += kSpmvLanes) s += val[p] * x[rv[p]];
+  const int row = blockIdx.x * (kBlock / L) + (int)threadIdx.x / L;
+  double s = 0.0;
+  if (row < n) {
+    const int32_t p1 = cp[row + 1];
+    for (int32_t p = cp[row]; p < p1; p += L * U) {
+      RowTurn<L, U> R;
+      R.load(rv, val, p, p1);
+      double g[U];
 #pragma unroll
-    for (int o = kSpmvLanes / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (sub == 0) y[row] = s;
+      for (int u = 0; u < U; ++u) g[u] = x[R.col[u]];
+#pragma unroll
+      for (int u = 0; u < U; ++u) s += R.v[u] * g[u];
+    }
   }
+  s = row_sum<L>(s);
+  if (row < n && threadIdx.x % L == 0) y[row] = s;
 }
 
+// Lanes per row and entries per lane and turn, by the mean row length (2-D Q1: 9, 3-D Q1
+// and P2: 25-29, scalar Q2: 60, vector Q2: 150-190).  Measured around the choices, in µs:
+// P2 4x8 32, 8x4 31, 8x6 37, 16x2 36, 16x3 42; 3-D Q1 (40³) 4.4, 4.3, 5.5, 5.4, 6.2;
+// vector Q2 16x12 406, 32x4 385, 32x6 415, 32x8 400, 64x3 438, 64x6 518: entries past the
+// row's end cost their issue slots, so a turn that covers every row is not the best.
+// f(L, U) with both as compile-time constants.
+template <class F>
+void row_shape(int64_t nnz, int64_t n, F &&f) {
+  const double m = (double)nnz / (double)std::max<int64_t>(n, 1);
+  auto c = [](auto v) { return v; };
+  using std::integral_constant;
+  if (m <= 12) f(c(integral_constant<int, 4>{}), c(integral_constant<int, 3>{}));
+  else if (m <= 32) f(c(integral_constant<int, 8>{}), c(integral_constant<int, 4>{}));
+  else if (m <= 80) f(c(integral_constant<int, 16>{}), c(integral_constant<int, 5>{}));
+  else f(c(integral_constant<int, 32>{}), c(integral_constant<int, 4>{}));
+}
+
+// The diagonal of a row by binary search (rows are sorted).
 __global__ void diag_inv_kernel(int64_t n, const int32_t *__restrict__ cp,
                                 const int32_t *__restrict__ rv, const double *__restrict__ val,
                                 double *__restrict__ dinv) {
   int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
-  double d = 0.0;
-  for (int32_t p = cp[j]; p < cp[j + 1]; ++p)
-    if (rv[p] == j) d = val[p];
+  int lo = cp[j], hi = cp[j + 1];
+  const int end = hi;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (rv[mid] < j) lo = mid + 1;
+    else hi = mid;
+  }
+  const double d = lo < end && rv[lo] == j ? val[lo] : 0.0;
   dinv[j] = d != 0.0 ? 1.0 / d : 1.0;
 }
 
 // r = b - q; with a diagonal (or no) preconditioner also z = M r; partials of r·z,
-// r·r, b·b.
+// r·r, b·b.  The CSR kernels keep z and p interleaved (zp: z in .x, p in .y): they take
+// {z, 0} here.
 __global__ __launch_bounds__(kBlock) void init_kernel(int64_t n, const double *__restrict__ b,
                                                       const double *__restrict__ q,
                                                       const double *__restrict__ dinv,
                                                       int factored, double *__restrict__ r,
                                                       double *__restrict__ z,
+                                                      double2 *__restrict__ zp,
                                                       double *__restrict__ part_rz,
                                                       double *__restrict__ part_rr,
                                                       double *__restrict__ part_bb) {
@@ -191,7 +263,8 @@ __global__ __launch_bounds__(kBlock) void init_kernel(int64_t n, const double *_
     r[i] = ri;
     if (!factored) {
       const double zi = dinv ? ri * dinv[i] : ri;
-      z[i] = zi;
+      if (zp) zp[i] = make_double2(zi, 0.0);
+      else z[i] = zi;
       rz += ri * zi;
     }
     rr += ri * ri;
@@ -203,46 +276,105 @@ __global__ __launch_bounds__(kBlock) void init_kernel(int64_t n, const double *_
 }
 
 // r·z of this iteration from its partials (published to scal[rz slot] by block 0);
-// p' = z + β p, q = A p', partials of p'·q  (β = 0 on the first iteration of a start)
+// p' = z + β p, q = A p', partials of p'·q  (β = 0 on the first iteration of a start).
+// z and p of a column come from one 16-byte gather, issued for the first row's first turn
+// ahead of the reduction that gives β.
+template <int L, int U>
 __global__ __launch_bounds__(kBlock) void spmv_dir_kernel(
-    int64_t n, const int32_t *__restrict__ cp, const int32_t *__restrict__ rv,
-    const double *__restrict__ val, const double *__restrict__ z,
-    const double *__restrict__ pold, double *__restrict__ pnew, double *__restrict__ q,
-    double *scal, int par, int first, const double *__restrict__ part_rz,
-    const double *__restrict__ part_rr, int np_rz, double thr, int it,
-    double *__restrict__ part_pq) {
+    int n, int ntiles, const int32_t *__restrict__ cp, const int32_t *__restrict__ rv,
+    const double *__restrict__ val, const double2 *__restrict__ zp, double2 *__restrict__ zpnew,
+    double *__restrict__ q, double *scal, int par, int first,
+    const double *__restrict__ part_rz, const double *__restrict__ part_rr, int np_rz, double thr,
+    int it, double *__restrict__ part_pq) {
   __shared__ double sh[kStartLds];
   StartIn S = start_loads(scal, part_rz, first ? nullptr : part_rr, np_rz);
   const double rz_old = scal[kRz + (par ^ 1)];
+  int t = blockIdx.x;
+  RowTurn<L, U> R;
+  double2 g[U], own{};
+  int row = n;
+  int32_t p = 0, p1 = 0;
+  auto gather = [&] {
+    R.load(rv, val, p, p1);
+#pragma unroll
+    for (int u = 0; u < U; ++u) g[u] = zp[R.col[u]];
+  };
+  auto open = [&](int tile) {  // a row's first turn
+    row = tile * (kBlock / L) + (int)threadIdx.x / L;
+    if (row >= n) return;
+    p = cp[row];
+    p1 = cp[row + 1];
+    own = zp[row];
+    gather();
+  };
+  if (t < ntiles) open(t);
   if (start_sums(S, sh)) return;
   const double rz = S.a;
   if (iteration_stops(scal, S.b, first, thr, it)) return;
   const double beta = first ? 0.0 : rz / rz_old;
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[kRz + par] = rz;
-  const int sub = threadIdx.x % kSpmvLanes;
-  const int64_t stride = (int64_t)gridDim.x * (kBlock / kSpmvLanes);
   double dot = 0.0;
-  for (int64_t row = (int64_t)blockIdx.x * (kBlock / kSpmvLanes) + threadIdx.x / kSpmvLanes;
-       row < n; row += stride) {
+  while (t < ntiles) {
     double s = 0.0;
-    if (first) {
-      for (int32_t p = cp[row] + sub; p < cp[row + 1]; p += kSpmvLanes) s += val[p] * z[rv[p]];
-    } else {
-      for (int32_t p = cp[row] + sub; p < cp[row + 1]; p += kSpmvLanes) {
-        const int32_t j = rv[p];
-        s += val[p] * (z[j] + beta * pold[j]);
-      }
-    }
+    if (row < n)
+      for (;;) {
 #pragma unroll
-    for (int o = kSpmvLanes / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (sub == 0) {
-      const double pn = first ? z[row] : z[row] + beta * pold[row];
-      pnew[row] = pn;
+        for (int u = 0; u < U; ++u) s += R.v[u] * (g[u].x + beta * g[u].y);
+        p += L * U;
+        if (p >= p1) break;
+        gather();
+      }
+    s = row_sum<L>(s);
+    if (row < n && threadIdx.x % L == 0) {
+      const double pn = own.x + beta * own.y;
+      zpnew[row].y = pn;
       q[row] = s;
       dot += pn * s;
     }
+    t += gridDim.x;
+    if (t < ntiles) open(t);
   }
   put_partial(dot, part_pq, sh);
+}
+
+// α = r·z / p'·q; x += α p'; r -= α q; z = M r beside p' (diagonal M or none); partials
+// of r·z and r·r: the CSR kernels' form (interleaved z and p), loads ahead of the
+// reduction that gives α
+__global__ __launch_bounds__(kBlock) void update_zp_kernel(
+    int64_t n, int par, const double *__restrict__ dinv, double *__restrict__ x,
+    double *__restrict__ r, double2 *__restrict__ zp, const double *__restrict__ q,
+    const double *scal, const double *__restrict__ part_pq, int np_pq,
+    double *__restrict__ part_rz, double *__restrict__ part_rr) {
+  __shared__ double sh[kStartLds];
+  const int64_t stride = (int64_t)gridDim.x * kBlock;
+  int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  double xi = 0.0, ri = 0.0, pi = 0.0, qi = 0.0, di = 1.0;
+  auto load = [&] {
+    pi = zp[i].y;
+    qi = q[i];
+    ri = r[i];
+    xi = x[i];
+    if (dinv) di = dinv[i];
+  };
+  StartIn S = start_loads(scal, part_pq, nullptr, np_pq);
+  const double rz_now = scal[kRz + par];
+  if (i < n) load();
+  if (start_sums(S, sh)) return;
+  const double alpha = rz_now / S.a;
+  double rz = 0.0, rr = 0.0;
+  while (i < n) {
+    x[i] = xi + alpha * pi;
+    ri -= alpha * qi;
+    r[i] = ri;
+    const double zi = dinv ? ri * di : ri;
+    zp[i] = make_double2(zi, pi);
+    rz += ri * zi;
+    rr += ri * ri;
+    i += stride;
+    if (i < n) load();
+  }
+  put_partial(rz, part_rz, sh);
+  put_partial(rr, part_rr, sh);
 }
 
 // α = r·z / p'·q; x += α p'; r -= α q; z = M r (diagonal M or none); partials of
@@ -309,7 +441,7 @@ static_assert(kSlots == 4 * kApplyLanes, "4 slots per lane");
 __global__ __launch_bounds__(kBlock) void update_lower_kernel(
     int64_t n, int par, const float *__restrict__ ge, const int32_t *__restrict__ gi,
     double *__restrict__ x, const double *__restrict__ rold, double *__restrict__ rnew,
-    const double *__restrict__ p, const double *__restrict__ q, double *__restrict__ y,
+    const double2 *__restrict__ zp, const double *__restrict__ q, double *__restrict__ y,
     const double *scal, const double *__restrict__ part_pq, int np_pq,
     double *__restrict__ part_rr) {
   __shared__ double sh[kStartLds];
@@ -334,7 +466,7 @@ __global__ __launch_bounds__(kBlock) void update_lower_kernel(
       y[row] = s;
       const double ri = rold[row] - alpha * q[row];
       rnew[row] = ri;
-      x[row] += alpha * p[row];
+      x[row] += alpha * zp[row].y;
       rr += ri * ri;
     }
   }
@@ -360,10 +492,11 @@ __global__ __launch_bounds__(kBlock) void lower_kernel(int64_t n, const float *_
   }
 }
 
-// z = Gᵀ y; partials of r·z
+// z = Gᵀ y (beside p); partials of r·z.  START: p becomes 0 (start of a solve)
+template <bool START>
 __global__ __launch_bounds__(kBlock) void upper_rz_kernel(
     int64_t n, const float *__restrict__ ge, const int32_t *__restrict__ gi,
-    const double *__restrict__ y, const double *__restrict__ r, double *__restrict__ z,
+    const double *__restrict__ y, const double *__restrict__ r, double2 *__restrict__ zp,
     const double *scal, double *__restrict__ part_rz) {
   __shared__ double sh[kStartLds];
   StartIn S = start_loads(scal, nullptr, nullptr, 0);
@@ -380,7 +513,8 @@ __global__ __launch_bounds__(kBlock) void upper_rz_kernel(
 #pragma unroll
     for (int o = kApplyLanes / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
     if (sub == 0) {
-      z[row] = s;
+      if (START) zp[row] = make_double2(s, 0.0);
+      else zp[row].x = s;
       rz += s * r[row];
     }
   }
@@ -736,9 +870,12 @@ __global__ __launch_bounds__(kBlock) void upper_rz_box_kernel(
 }  // namespace
 
 void spmv_device(Ctx &c, const double *x, double *y) {
-  hipLaunchKernelGGL(spmv_kernel, dim3(grid_rows(c.nfree, kBlock / kSpmvLanes)), dim3(kBlock), 0,
-                     c.stream, (int64_t)c.nfree, c.colptr.get(), c.rowval.get(), c.nzval.get(),
-                     x, y);
+  row_shape(c.nnz, c.nfree, [&](auto L, auto U) {
+    const int ntiles = (int)((c.nfree + kBlock / L() - 1) / (kBlock / L()));
+    hipLaunchKernelGGL((spmv_kernel<L(), U()>), dim3((unsigned)std::max(ntiles, 1)),
+                       dim3(kBlock), 0, c.stream, (int)c.nfree, c.colptr.get(), c.rowval.get(),
+                       c.nzval.get(), x, y);
+  });
   GH_CHECK_HIP(hipGetLastError());
 }
 
@@ -757,6 +894,7 @@ namespace {
 // vectors, the diagonal inverse, partial sums (4 x kMaxParts) and scalars (8).
 struct PcgBufs {
   double *x, *b, *r, *r2, *z, *p, *p2, *q, *y, *dinv, *part, *scal;
+  double2 *zp, *zp2;  // the CSR form's interleaved z and p (two buffers)
 };
 
 __global__ void clear_stop_kernel(double *scal) {
@@ -817,10 +955,13 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   double *part_rr = part_rz + kMaxParts, *part_bb = part_rr + kMaxParts;
   double *rbuf[2] = {V.r, factored ? V.r2 : V.r};
   double *pbuf[2] = {V.p, V.p2};
+  double2 *zpbuf[2] = {V.zp, V.zp2};
   const int ntiles = (int)((n + kBlock - 1) / kBlock);
-  const unsigned g_vec = grid_rows((n + 1) / 2, kBlock);  // two entries per thread
+  // the vector kernels: two entries per thread, one with the interleaved z and p
+  const unsigned g_vec = grid_rows(box ? (n + 1) / 2 : n, kBlock);
   const unsigned g_box = grid_rows(n, kBlock);            // one tile per block and turn
-  const unsigned g_spmv = box ? g_box : grid_rows(n, kBlock / kSpmvLanes);
+  unsigned g_spmv = g_box;
+  if (!box) row_shape(c.nnz, n, [&](auto L, auto) { g_spmv = grid_rows(n, kBlock / L()); });
   const unsigned g_apply = box ? g_box : grid_rows(n, kBlock / kApplyLanes);
   // the stencil kernels' form: one run per dz, or per (dz, dy) for long rows
   const bool wide = B.m0 > kBlock;
@@ -858,7 +999,8 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
     // (re)start from the true residual r = b - A x
     spmv_device(c, V.x, V.q);
     hipLaunchKernelGGL(init_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, V.b, V.q,
-                       dinv, factored, rbuf[0], V.z, part_rz, part_rr, part_bb);
+                       dinv, factored, rbuf[0], V.z, box ? nullptr : zpbuf[0], part_rz, part_rr,
+                       part_bb);
     hipLaunchKernelGGL(clear_stop_kernel, dim3(1), dim3(64), 0, s, scal);
     if (factored && box) {
       lower_box(true, 0, rbuf[0], nullptr, nullptr);
@@ -866,8 +1008,8 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
     } else if (factored) {
       hipLaunchKernelGGL(lower_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, c.gle.get(),
                          c.gli.get(), rbuf[0], V.y);
-      hipLaunchKernelGGL(upper_rz_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, c.gue.get(),
-                         c.gui.get(), V.y, rbuf[0], V.z, scal, part_rz);
+      hipLaunchKernelGGL(upper_rz_kernel<true>, dim3(g_apply), dim3(kBlock), 0, s, n,
+                         c.gue.get(), c.gui.get(), V.y, rbuf[0], zpbuf[0], scal, part_rz);
     }
     GH_CHECK_HIP(hipGetLastError());
     GH_CHECK_HIP(hipMemcpyAsync(hrr, part_rr, sizeof(double) * g_vec,
@@ -896,13 +1038,17 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
         const int par = k & 1;
         const int itk = it + m;
         double *pold = pbuf[par], *pnew = pbuf[par ^ 1];
+        double2 *zpold = zpbuf[par], *zpnew = zpbuf[par ^ 1];
         if (box)
           spmv_dir_box(pold, pnew, par, k == 0 ? 1 : 0, np_rz, thr, itk);
         else
-          hipLaunchKernelGGL(spmv_dir_kernel, dim3(g_spmv), dim3(kBlock), 0, s, n,
-                             c.colptr.get(), c.rowval.get(), c.nzval.get(), V.z, pold,
-                             pnew, V.q, scal, par, k == 0 ? 1 : 0, part_rz, part_rr,
-                             np_rz, thr, itk, part_pq);
+          row_shape(c.nnz, n, [&](auto L, auto U) {
+            const int nt = (int)((n + kBlock / L() - 1) / (kBlock / L()));
+            hipLaunchKernelGGL((spmv_dir_kernel<L(), U()>), dim3(g_spmv), dim3(kBlock), 0, s,
+                               (int)n, nt, c.colptr.get(), c.rowval.get(), c.nzval.get(), zpold,
+                               zpnew, V.q, scal, par, k == 0 ? 1 : 0, part_rz, part_rr, np_rz,
+                               thr, itk, part_pq);
+          });
         if (factored && box) {
           double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
           lower_box(false, par, rold, rnew, pnew);
@@ -910,10 +1056,14 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
         } else if (factored) {
           double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
           hipLaunchKernelGGL(update_lower_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, par,
-                             c.gle.get(), c.gli.get(), V.x, rold, rnew, pnew, V.q,
+                             c.gle.get(), c.gli.get(), V.x, rold, rnew, zpnew, V.q,
                              V.y, scal, part_pq, (int)g_spmv, part_rr);
-          hipLaunchKernelGGL(upper_rz_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, c.gue.get(),
-                             c.gui.get(), V.y, rnew, V.z, scal, part_rz);
+          hipLaunchKernelGGL(upper_rz_kernel<false>, dim3(g_apply), dim3(kBlock), 0, s, n,
+                             c.gue.get(), c.gui.get(), V.y, rnew, zpnew, scal, part_rz);
+        } else if (!box) {
+          hipLaunchKernelGGL(update_zp_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, par, dinv,
+                             V.x, rbuf[0], zpnew, V.q, scal, part_pq, (int)g_spmv, part_rz,
+                             part_rr);
         } else {
           hipLaunchKernelGGL(update_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, par, dinv,
                              V.x, rbuf[0], V.z, pnew, V.q, scal, part_pq,
@@ -954,7 +1104,9 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
 
 void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st) {
   const size_t nn = (size_t)std::max<int64_t>(c.nfree, 1);
-  for (auto *bf : {&c.s_r, &c.s_z, &c.s_p, &c.s_p2, &c.s_q}) bf->resize(nn);
+  for (auto *bf : {&c.s_r, &c.s_z, &c.s_q}) bf->resize(nn);
+  // p and its second buffer, or the interleaved z and p of the CSR kernels
+  for (auto *bf : {&c.s_p, &c.s_p2}) bf->resize(2 * nn);
   c.s_part.resize(4 * kMaxParts);
   c.s_scal.resize(8);
   if (precond == GH_PRECOND_JACOBI) c.s_dinv.resize(nn);
@@ -964,19 +1116,21 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
   }
   const PcgBufs V{c.s_x.get(), c.s_b.get(), c.s_r.get(), c.s_r2.get(), c.s_z.get(),
                   c.s_p.get(), c.s_p2.get(), c.s_q.get(), c.s_y.get(), c.s_dinv.get(),
-                  c.s_part.get(), c.s_scal.get()};
+                  c.s_part.get(), c.s_scal.get(), (double2 *)c.s_p.get(),
+                  (double2 *)c.s_p2.get()};
   pcg_run(c, V, precond, rtol, maxit, true, true, st);
 }
 
 // ---- the solve that allocates nothing (gh_pcg_noalloc) ------------------------------
 // Its vectors live in one fixed device array, `scratch`, which every GPU the library
-// runs on holds until the process ends: x, b, r, z, p, p', q, D^-1 of at most
-// GH_NOALLOC_MAX_N entries each, then the partial sums and the scalars.  Every call on
+// runs on holds until the process ends: x, b, r, q, D^-1 and two interleaved {z, p}, of
+// at most GH_NOALLOC_MAX_N entries each (nine vectors), then the partial sums and the scalars.  Every call on
 // one GPU shares that GPU's copy (calls that overlap on one GPU race), and nothing in
 // it is read before the call writes it.
 namespace {
 constexpr size_t kNoAllocVec = (size_t)GH_NOALLOC_MAX_N;
-constexpr size_t kScratchDoubles = 8 * kNoAllocVec + 4 * (size_t)kMaxParts + 8;
+constexpr size_t kNoAllocVecs = 9;
+constexpr size_t kScratchDoubles = kNoAllocVecs * kNoAllocVec + 4 * (size_t)kMaxParts + 8;
 __device__ __align__(256) double scratch[kScratchDoubles];
 
 constexpr int kMaxDevices = 64;
@@ -1011,9 +1165,10 @@ void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, i
   GH_REQUIRE(base, GH_ERR_STATE, "scratch address not set up for this device");
   const size_t n = (size_t)c.nfree;
   const size_t L = kNoAllocVec;
-  const PcgBufs V{base, base + L, base + 2 * L, nullptr, base + 3 * L, base + 4 * L,
-                  base + 5 * L, base + 6 * L, nullptr, base + 7 * L, base + 8 * L,
-                  base + 8 * L + 4 * (size_t)kMaxParts};
+  double *part = base + kNoAllocVecs * L;
+  const PcgBufs V{base, base + L, base + 2 * L, nullptr, nullptr, nullptr, nullptr, base + 3 * L,
+                  nullptr, base + 4 * L, part, part + 4 * (size_t)kMaxParts,
+                  (double2 *)(base + 5 * L), (double2 *)(base + 7 * L)};
   const auto t0 = std::chrono::steady_clock::now();
   GH_CHECK_HIP(hipMemcpyAsync(V.x, x, sizeof(double) * n, hipMemcpyHostToDevice, c.stream));
   if (b)
