@@ -26,8 +26,6 @@ namespace gh {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kMlpCellsPerBlock = 256;  // backward / weight-gradient partials
-constexpr int kMlpFwdCells = 32;        // forward: small blocks, many waves in flight
 constexpr int kEllSlots = kFsaiEllSlots;
 
 inline unsigned grid_for(int64_t n, int block = kBlock) {
@@ -78,21 +76,22 @@ __device__ __forceinline__ void node_xyz(const Lat3 &L, int n, int *xi) {
 
 // ---- set-up --------------------------------------------------------------
 
-__global__ void diag_setup_kernel(int64_t n, const int32_t *__restrict__ cp,
-                                  const int32_t *__restrict__ rv,
-                                  const double *__restrict__ val, int32_t *__restrict__ dpos,
+// Per free node: the position and value of its diagonal entry (the number of free
+// stencil neighbours below it, from the mask, past the column start) and D^-1/2.
+__global__ void diag_setup_kernel(int nnodes, const int32_t *__restrict__ node_dof,
+                                  const uint32_t *__restrict__ fmask,
+                                  const int32_t *__restrict__ cp, const double *__restrict__ val,
+                                  int32_t *__restrict__ dpos, double *__restrict__ diag,
                                   double *__restrict__ fs) {
-  int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  int lo = cp[j], hi = cp[j + 1];
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (rv[mid] < j) lo = mid + 1;
-    else hi = mid;
-  }
-  dpos[j] = lo;  // the diagonal is in the pattern of every free column
-  const double d = val[lo];
-  fs[j] = d > 0.0 ? 1.0 / sqrt(d) : 1.0;
+  const int node = blockIdx.x * blockDim.x + threadIdx.x;
+  if (node >= nnodes) return;
+  const int d = node_dof[node];
+  if (d <= 0) return;
+  const int p = cp[d - 1] + __popc(fmask[node] & ((1u << 13) - 1u));
+  const double v = val[p];
+  dpos[d - 1] = p;
+  diag[d - 1] = v;
+  fs[d - 1] = v > 0.0 ? 1.0 / sqrt(v) : 1.0;
 }
 
 __global__ void grf_kappa_kernel(Lat3 L, int64_t ncells, double ox, double oy, double oz,
@@ -114,54 +113,38 @@ __global__ void grf_kappa_kernel(Lat3 L, int64_t ncells, double ox, double oy, d
 
 // ---- network inputs --------------------------------------------------------
 
+// The diagonal comes from its own array, the 8 nodes' loads together: through positions into
+// nzval, one node after the other, 62 µs at 64³; now 11 µs.
 __global__ void features_kernel(Lat3 L, int64_t ncells, const double *__restrict__ kappa,
                                 const int32_t *__restrict__ node_dof,
-                                const int32_t *__restrict__ dpos,
-                                const double *__restrict__ nzval, double kdiag, float logh,
+                                const double *__restrict__ diag, double kdiag, float logh,
                                 float *__restrict__ feat) {
   int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= ncells) return;
-  const int cx = (int)(c % L.nc[0]);
-  const int cy = (int)((c / L.nc[0]) % L.nc[1]);
-  const int cz = (int)(c / ((int64_t)L.nc[0] * L.nc[1]));
+  const int ci = (int)c;
+  const int cx = ci % L.nc[0];
+  const int cy = (ci / L.nc[0]) % L.nc[1];
+  const int cz = ci / (L.nc[0] * L.nc[1]);
   const double k = kappa ? kappa[c] : 1.0;
-  float *f = feat + c * kMlpInPad;
+  int d[8];
+  double dg[8];
 #pragma unroll
-  for (int a = 0; a < 8; ++a) {
-    const int node = (cx + (a & 1)) + L.nn[0] * ((cy + ((a >> 1) & 1)) + L.nn[1] * (cz + (a >> 2)));
-    const int d = node_dof[node];
-    f[a] = d > 0 ? (float)(k * kdiag / nzval[dpos[d - 1]]) : 0.0f;
-  }
+  for (int a = 0; a < 8; ++a)
+    d[a] = node_dof[(cx + (a & 1)) + L.nn[0] * ((cy + ((a >> 1) & 1)) + L.nn[1] * (cz + (a >> 2)))];
+#pragma unroll
+  for (int a = 0; a < 8; ++a) dg[a] = diag[max(d[a], 1) - 1];  // all in flight
+  float f[kMlpInPad] = {};
+#pragma unroll
+  for (int a = 0; a < 8; ++a) f[a] = d[a] > 0 ? (float)(k * kdiag / dg[a]) : 0.0f;
   f[8] = (float)log(k);
   f[9] = logh;
+  float4 *out = reinterpret_cast<float4 *>(feat + c * kMlpInPad);
 #pragma unroll
-  for (int a = 10; a < kMlpInPad; ++a) f[a] = 0.0f;
+  for (int q = 0; q < kMlpInPad / 4; ++q)
+    out[q] = make_float4(f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]);
 }
 
-// ---- MLP: lane = output unit, one cell row (uniform) at a time ---------------
-
-template <int NIN, int NINP, int NOUT, int NOUTP, bool GELU, bool SOA = false>
-__global__ __launch_bounds__(64) void mlp_fwd(const float *__restrict__ in,
-                                              const uint16_t *__restrict__ wq, int woff,
-                                              int boff, float *__restrict__ zout,
-                                              float *__restrict__ hout, int C, int cpb) {
-  const int j = threadIdx.x;
-  float w[NIN];
-#pragma unroll
-  for (int k = 0; k < NIN; ++k) w[k] = j < NOUT ? bf16_to_f32(wq[woff + j * NIN + k]) : 0.0f;
-  const float bias = j < NOUT ? bf16_to_f32(wq[boff + j]) : 0.0f;
-  const int c0 = blockIdx.x * cpb, c1 = min(c0 + cpb, C);
-  for (int c = c0; c < c1; ++c) {
-    const float *row = in + (size_t)c * NINP;
-    float acc = bias;
-#pragma unroll
-    for (int k = 0; k < NIN; ++k) acc = fmaf(w[k], row[k], acc);
-    if (j < NOUT) {
-      zout[SOA ? (size_t)j * C + c : (size_t)c * NOUTP + j] = acc;
-      if (GELU) hout[(size_t)c * NOUTP + j] = gelu(acc);
-    }
-  }
-}
+// ---- MLP ---------------------------------------------------------------------------
 
 // Inference forward of the whole network on the matrix cores
 // (v_mfma_f32_16x16x32_bf16): a wave owns 16-cell tiles; layer inputs are rounded
@@ -312,67 +295,351 @@ __global__ __launch_bounds__(kFwdWaves * 64) void mlp_fwd_mfma(const float *__re
   }
 }
 
-// dz_in = (Wᵀ dz_out) ⊙ gelu'(z_in); lane = input unit
-template <int NOUT, int NOUTP, int NIN, int NINP>
-__global__ __launch_bounds__(64) void mlp_bwd(const float *__restrict__ dzout,
-                                              const uint16_t *__restrict__ wq, int woff,
-                                              const float *__restrict__ zin,
-                                              float *__restrict__ dzin, int C, int cpb) {
-  const int k = threadIdx.x;
-  float w[NOUT];
+// Training: forward, and forward + backward, on the FP32 matrix cores
+// (v_mfma_f32_16x16x4_f32: FP32 operands and accumulators; lane l supplies A[l%16][k],
+// B[k][l%16] with k of its lane group l/16, and holds D[4(l/16)+j][l%16]).  A workgroup
+// takes tiles of 64 cells; a wave owns 16 of them in the forward and the
+// back-propagated products (cells are the rows, the layer's units the columns) and 16
+// output units in the weight gradients (units are the rows, the 64 cells the
+// contraction).  The order of a contraction is free, so group g takes k = 16 g + kk: each
+// lane's 16 operands are contiguous, in LDS and in the BF16 weights (read from L1).
+// The backward kernel recomputes the activations from the features: it reads 64 B
+// of features and 160 B of output gradient per cell and keeps the rest in LDS, and each
+// workgroup writes one partial of every gradient.  Bound by the matrix cores at large
+// C (560 instructions of 32 cycles per tile and wave), by the number of tiles below
+// 256 tiles.  One lane per unit and 256 cells in turn left 128 waves for the whole chip:
+// 32³ cells 1,480 µs for forward, backward, gradients and their sums; now 20 + 58 + 9 µs.
+constexpr int kTrainCells = 64;
+constexpr int kTrainLd = kMlpHidden + 4;   // row stride of activations: conflict-free b128
+constexpr int kTrainGrid = 256;            // most workgroups of the backward (partials)
+
+struct TrainLds {
+  float h[3][kTrainCells][kTrainLd];   // activations, then (backward) pre-activation gradients
+  float dy[kTrainCells][48 + 4];       // output gradient, zero from 36 on
+  float ft[kTrainCells][kMlpInPad + 4];  // features; column 10 is 1 (the bias gradient)
+};
+
+__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int N>
+__device__ __forceinline__ void load_row(const float *p, float (&v)[N]) {
 #pragma unroll
-  for (int j = 0; j < NOUT; ++j) w[j] = k < NIN ? bf16_to_f32(wq[woff + j * NIN + k]) : 0.0f;
-  const int c0 = blockIdx.x * cpb, c1 = min(c0 + cpb, C);
-  for (int c = c0; c < c1; ++c) {
-    const float *row = dzout + (size_t)c * NOUTP;
-    float s = 0.0f;
-#pragma unroll
-    for (int j = 0; j < NOUT; ++j) s = fmaf(w[j], row[j], s);
-    if (k < NIN) dzin[(size_t)c * NINP + k] = s * gelu_d(zin[(size_t)c * NINP + k]);
+  for (int i = 0; i < N / 4; ++i) {
+    const float4 q = reinterpret_cast<const float4 *>(p)[i];
+    v[4 * i] = q.x;
+    v[4 * i + 1] = q.y;
+    v[4 * i + 2] = q.z;
+    v[4 * i + 3] = q.w;
   }
 }
 
-// Per-block partial of dW = Σ_c dz_c h_cᵀ and db = Σ_c dz_c; lane = output unit.
-template <int NIN, int NINP, int NOUT, int NOUTP>
-__global__ __launch_bounds__(64) void mlp_wgrad(const float *__restrict__ dz,
-                                                const float *__restrict__ hin,
-                                                float *__restrict__ part, int C, int cpb) {
-  const int j = threadIdx.x;
-  float acc[NIN];
+// 16 consecutive BF16 weights as FP32 (16-byte aligned)
+__device__ __forceinline__ void load_weights16(const uint16_t *w, float (&v)[16]) {
 #pragma unroll
-  for (int k = 0; k < NIN; ++k) acc[k] = 0.0f;
-  float accb = 0.0f;
-  const int c0 = blockIdx.x * cpb, c1 = min(c0 + cpb, C);
-  for (int c = c0; c < c1; ++c) {
-    const float d = j < NOUT ? dz[(size_t)c * NOUTP + j] : 0.0f;
-    const float *row = hin + (size_t)c * NINP;
+  for (int i = 0; i < 2; ++i) {
+    const uint4 u = reinterpret_cast<const uint4 *>(w)[i];
+    const uint32_t d[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-    for (int k = 0; k < NIN; ++k) acc[k] = fmaf(d, row[k], acc[k]);
-    accb += d;
-  }
-  float *pp = part + (size_t)blockIdx.x * (NOUT * NIN + NOUT);
-  if (j < NOUT) {
-#pragma unroll
-    for (int k = 0; k < NIN; ++k) pp[j * NIN + k] = acc[k];
-    pp[NOUT * NIN + j] = accb;
+    for (int j = 0; j < 4; ++j) {
+      v[8 * i + 2 * j] = __uint_as_float(d[j] << 16);
+      v[8 * i + 2 * j + 1] = __uint_as_float(d[j] & 0xffff0000u);
+    }
   }
 }
 
-__global__ void reduce_parts(const float *__restrict__ part, int nblocks, int len,
-                             float *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= len) return;
+// The three hidden layers of the wave's 16 cells: activations to S.h, gelu' of the
+// pre-activations to gd (BWD).
+template <bool BWD>
+__device__ __forceinline__ void hidden_layers(TrainLds &S, const uint16_t *__restrict__ wq,
+                                              int wave, int lane, float (&gd)[3][16]) {
+  const int l16 = lane & 15, g = lane >> 4, row = 16 * wave + l16;
+#pragma unroll
+  for (int layer = 0; layer < 3; ++layer) {
+    const int woff = layer == 0 ? kMlpW1 : layer == 1 ? kMlpW2 : kMlpW3;
+    const int boff = layer == 0 ? kMlpB1 : layer == 1 ? kMlpB2 : kMlpB3;
+    float a[16];
+    if (layer == 0) {
+      float f[4];
+      load_row(&S.ft[row][4 * g], f);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a[k] = f[k];
+    } else {
+      load_row(&S.h[layer - 1][row][16 * g], a);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int unit = 16 * t + l16;
+      v4f acc{0.0f, 0.0f, 0.0f, 0.0f};
+      if (layer == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          acc = mfma4(a[k], 4 * g + k < kMlpIn
+                                ? bf16_to_f32(wq[kMlpW1 + unit * kMlpIn + 4 * g + k]) : 0.0f, acc);
+      } else {
+        float w[16];
+        load_weights16(wq + woff + unit * kMlpHidden + 16 * g, w);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) acc = mfma4(a[k], w[k], acc);
+      }
+      const float bias = bf16_to_f32(wq[boff + unit]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float z = acc[j] + bias;
+        S.h[layer][16 * wave + 4 * g + j][unit] = gelu(z);
+        if (BWD) gd[layer][4 * t + j] = gelu_d(z);
+      }
+    }
+    wave_sync();  // the wave reads its own 16 rows next
+  }
+}
+
+// features of a tile to LDS (rows past the last cell are zero)
+__device__ __forceinline__ void load_features(TrainLds &S, const float *__restrict__ feat, int c0,
+                                              int C) {
+  const int r = threadIdx.x >> 2, q = threadIdx.x & 3;  // 64 rows x 4 quads
+  float4 v{0.0f, 0.0f, 0.0f, 0.0f};
+  if (c0 + r < C) v = reinterpret_cast<const float4 *>(feat + (size_t)(c0 + r) * kMlpInPad)[q];
+  if (q == 2) v.z = 1.0f;
+  *reinterpret_cast<float4 *>(&S.ft[r][4 * q]) = v;
+}
+
+// network output yo[n][cell] of every cell
+__global__ __launch_bounds__(256) void mlp_train_fwd(const float *__restrict__ feat,
+                                                     const uint16_t *__restrict__ wq, int C,
+                                                     float *__restrict__ yo) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  TrainLds &S = *reinterpret_cast<TrainLds *>(lds_raw);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
+  float gd[3][16];
+  for (int c0 = blockIdx.x * kTrainCells; c0 < C; c0 += gridDim.x * kTrainCells) {
+    __syncthreads();
+    load_features(S, feat, c0, C);
+    __syncthreads();
+    hidden_layers<false>(S, wq, wave, lane, gd);
+    float a[16];
+    load_row(&S.h[2][16 * wave + l16][16 * g], a);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const int n = 16 * t + l16;
+      float w[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) w[k] = 0.0f;
+      if (n < kMlpOut) load_weights16(wq + kMlpW4 + n * kMlpHidden + 16 * g, w);
+      v4f acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc = mfma4(a[k], w[k], acc);
+      if (n < kMlpOut) {
+        const float bias = bf16_to_f32(wq[kMlpB4 + n]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c = c0 + 16 * wave + 4 * g + j;
+          if (c < C) yo[(size_t)n * C + c] = acc[j] + bias;
+        }
+      }
+    }
+  }
+}
+
+// Weights in input-major order (the backward product's B operand), in LDS
+constexpr int kWtLd = kMlpHidden + 8;      // BF16; 16-byte rows, conflict-free b128
+constexpr int kWt4Ld = 56;                 // 36 outputs padded to 48
+struct TrainWeights {
+  uint16_t w2t[kMlpHidden][kWtLd], w3t[kMlpHidden][kWtLd], w4t[kMlpHidden][kWt4Ld];
+};
+
+// Partial gradients of every weight: one kMlpParams run per workgroup.
+__global__ __launch_bounds__(256) void mlp_train_bwd(const float *__restrict__ feat,
+                                                     const uint16_t *__restrict__ wq,
+                                                     const float *__restrict__ dy, int C,
+                                                     float *__restrict__ part) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  TrainLds &S = *reinterpret_cast<TrainLds *>(lds_raw);
+  TrainWeights &W = *reinterpret_cast<TrainWeights *>(lds_raw + sizeof(TrainLds));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g = lane >> 4;
+  const int row = 16 * wave + l16;
+  for (int t = threadIdx.x; t < kMlpHidden * kMlpHidden; t += 256) {
+    const int o = t / kMlpHidden, i = t % kMlpHidden;
+    W.w2t[i][o] = wq[kMlpW2 + t];
+    W.w3t[i][o] = wq[kMlpW3 + t];
+    if (o < 48) W.w4t[i][o] = o < kMlpOut ? wq[kMlpW4 + o * kMlpHidden + i] : (uint16_t)0;
+  }
+  // this wave's gradient tiles: W2, W3 rows 16 wave.. x all inputs; W4 all outputs x inputs
+  // 16 wave..; W1 rows 16 wave.. x the (padded) inputs
+  v4f aw1{0.0f, 0.0f, 0.0f, 0.0f}, aw2[4], aw3[4], aw4[3];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    aw2[t] = aw3[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    if (t < 3) aw4[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  float ab2 = 0.0f, ab3 = 0.0f, ab4[3] = {0.0f, 0.0f, 0.0f};
+  float gd[3][16];
+  // contraction step s of a weight gradient: the cell of lane group g (rows four apart,
+  // so the groups of a half-wave read different banks)
+  auto cell_of = [&](int s) { return 4 * g + (s & 3) + 16 * (s >> 2); };
+  // pre-activation gradient of a hidden layer: rows a (the layer above's gradient), its
+  // weights input-major, times gelu'; written over the activations
+  auto back16 = [&](int from, int to, const uint16_t (*wt)[kWtLd]) {
+    float a[16], d[16];
+    load_row(&S.h[from][row][16 * g], a);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float w[16];
+      load_weights16(&wt[16 * t + l16][16 * g], w);
+      v4f acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc = mfma4(a[k], w[k], acc);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[4 * t + j] = acc[j] * gd[to][4 * t + j];
+    }
+    __syncthreads();  // every wave has read the activations
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) S.h[to][16 * wave + 4 * g + j][16 * t + l16] = d[4 * t + j];
+    __syncthreads();
+  };
+  for (int c0 = blockIdx.x * kTrainCells; c0 < C; c0 += gridDim.x * kTrainCells) {
+    __syncthreads();
+    load_features(S, feat, c0, C);
+    for (int t = threadIdx.x; t < kTrainCells * 12; t += 256) {  // 12 quads, 9 of them stored
+      const int r = t / 12, q = t % 12;
+      float4 v{0.0f, 0.0f, 0.0f, 0.0f};
+      if (c0 + r < C && q < kMlpOut / 4)
+        v = reinterpret_cast<const float4 *>(dy + (size_t)(c0 + r) * kMlpOutPad)[q];
+      *reinterpret_cast<float4 *>(&S.dy[r][4 * q]) = v;
+    }
+    __syncthreads();
+    hidden_layers<true>(S, wq, wave, lane, gd);
+    __syncthreads();
+    // output layer: dW4 = dyᵀ h3, db4, and dz3
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int c = cell_of(s);
+      const float b = S.h[2][c][16 * wave + l16];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const float a = S.dy[c][16 * t + l16];
+        aw4[t] = mfma4(a, b, aw4[t]);
+        ab4[t] += a;
+      }
+    }
+    {
+      float a[12], d[16];
+      load_row(&S.dy[row][12 * g], a);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const uint2 *wp = reinterpret_cast<const uint2 *>(&W.w4t[16 * t + l16][12 * g]);
+        v4f acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const uint2 u = wp[q];
+          acc = mfma4(a[4 * q], __uint_as_float(u.x << 16), acc);
+          acc = mfma4(a[4 * q + 1], __uint_as_float(u.x & 0xffff0000u), acc);
+          acc = mfma4(a[4 * q + 2], __uint_as_float(u.y << 16), acc);
+          acc = mfma4(a[4 * q + 3], __uint_as_float(u.y & 0xffff0000u), acc);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[4 * t + j] = acc[j] * gd[2][4 * t + j];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S.h[2][16 * wave + 4 * g + j][16 * t + l16] = d[4 * t + j];
+      __syncthreads();
+    }
+    // hidden layer 3: dW3 = dz3ᵀ h2; hidden layer 2: dW2 = dz2ᵀ h1
+    auto wgrad = [&](int layer, v4f (&aw)[4], float &ab) {
+#pragma unroll
+      for (int s = 0; s < 16; ++s) {
+        const int c = cell_of(s);
+        const float a = S.h[layer][c][16 * wave + l16];
+        ab += a;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) aw[t] = mfma4(a, S.h[layer - 1][c][16 * t + l16], aw[t]);
+      }
+    };
+    wgrad(2, aw3, ab3);
+    back16(2, 1, W.w3t);
+    wgrad(1, aw2, ab2);
+    back16(1, 0, W.w2t);
+    // input layer: dW1 = dz1ᵀ features (column 10 of the features is 1: db1)
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int c = cell_of(s);
+      aw1 = mfma4(S.h[0][c][16 * wave + l16], S.ft[c][l16], aw1);
+    }
+  }
+  // bias sums over the lane groups
+  auto groups = [](float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+  };
+  ab2 = groups(ab2);
+  ab3 = groups(ab3);
+#pragma unroll
+  for (int t = 0; t < 3; ++t) ab4[t] = groups(ab4[t]);
+  float *pp = part + (size_t)blockIdx.x * kMlpParams;
+  if (g == 0) {
+    pp[kMlpB2 + 16 * wave + l16] = ab2;
+    pp[kMlpB3 + 16 * wave + l16] = ab3;
+    if (wave == 0)
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+        if (16 * t + l16 < kMlpOut) pp[kMlpB4 + 16 * t + l16] = ab4[t];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int o = 16 * wave + 4 * g + j;
+    if (l16 < kMlpIn) pp[kMlpW1 + o * kMlpIn + l16] = aw1[j];
+    else if (l16 == kMlpIn) pp[kMlpB1 + o] = aw1[j];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      pp[kMlpW2 + o * kMlpHidden + 16 * t + l16] = aw2[t][j];
+      pp[kMlpW3 + o * kMlpHidden + 16 * t + l16] = aw3[t][j];
+    }
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const int n = 16 * t + 4 * g + j;
+      if (n < kMlpOut) pp[kMlpW4 + n * kMlpHidden + 16 * wave + l16] = aw4[t][j];
+    }
+  }
+}
+
+// Gradient of every parameter: its partials summed in FP64 in a fixed order (16 threads
+// a parameter), then the Adam step (lr > 0).
+constexpr int kReduceLanes = 16;
+__global__ __launch_bounds__(256) void reduce_adam_kernel(
+    const float *__restrict__ part, int nblocks, float *__restrict__ g, float lr, float b1t,
+    float b2t, float *__restrict__ w, float *__restrict__ m, float *__restrict__ v,
+    uint16_t *__restrict__ wq) {
+  constexpr int P = 256 / kReduceLanes;  // parameters per workgroup: 64-byte runs of a partial
+  __shared__ double sh[kReduceLanes][P];
+  const int col = threadIdx.x % P, lane = threadIdx.x / P;
+  const int t = blockIdx.x * P + col;
   double s = 0.0;
-  for (int b = 0; b < nblocks; ++b) s += part[(size_t)b * len + t];
-  out[t] = (float)s;
-}
-
-__global__ void adam_kernel(int n, float *__restrict__ w, const float *__restrict__ g,
-                            float *__restrict__ m, float *__restrict__ v, float lr, float b1t,
-                            float b2t, uint16_t *__restrict__ wq) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float gi = g[t];
+  if (t < kMlpParams) {
+    constexpr int U = kTrainGrid / kReduceLanes;  // partials per thread, all in flight
+    float x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int b = lane + u * kReduceLanes;
+      x[u] = b < nblocks ? part[(size_t)b * kMlpParams + t] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) s += x[u];
+  }
+  sh[lane][col] = s;
+  __syncthreads();
+  if (lane != 0 || t >= kMlpParams) return;
+  s = 0.0;
+#pragma unroll
+  for (int k = 0; k < kReduceLanes; ++k) s += sh[k][col];
+  const float gi = (float)s;
+  g[t] = gi;
+  if (!(lr > 0.0f)) return;
   const float mi = 0.9f * m[t] + 0.1f * gi;
   const float vi = 0.999f * v[t] + 0.001f * gi * gi;
   m[t] = mi;
@@ -393,53 +660,22 @@ __device__ __forceinline__ int pair_index(int a, int b) {  // a > b, local numbe
   return 8 + a * (a - 1) / 2 + b;
 }
 
-// Ĝ entry of node n and its stencil neighbour m = n + (DX, DY, DZ) (the diagonal for
-// 0, 0, 0): Σ over the cells holding both, in ascending cell order, so that both
-// endpoints compute the same bits.  Along an axis with offset 0 the cell index is
-// x-1 or x, else min(x, x+D); cells outside the lattice are skipped.
-template <int DX, int DY, int DZ>
-__device__ __forceinline__ float pair_sum(const Lat3 &L, const int *xn,
-                                          const float *__restrict__ yo, size_t C) {
-  constexpr int NX = DX == 0 ? 2 : 1, NY = DY == 0 ? 2 : 1, NZ = DZ == 0 ? 2 : 1;
-  float s = 0.0f;
-#pragma unroll
-  for (int kz = 0; kz < NZ; ++kz)
-#pragma unroll
-    for (int ky = 0; ky < NY; ++ky)
-#pragma unroll
-      for (int kx = 0; kx < NX; ++kx) {
-        const int cx = DX == 0 ? xn[0] - 1 + kx : xn[0] + min(DX, 0);
-        const int cy = DY == 0 ? xn[1] - 1 + ky : xn[1] + min(DY, 0);
-        const int cz = DZ == 0 ? xn[2] - 1 + kz : xn[2] + min(DZ, 0);
-        if (cx < 0 || cx >= L.nc[0] || cy < 0 || cy >= L.nc[1] || cz < 0 || cz >= L.nc[2])
-          continue;
-        const size_t cell = (size_t)cx + (size_t)L.nc[0] * (cy + (size_t)L.nc[1] * cz);
-        const int ln = (xn[0] - cx) | ((xn[1] - cy) << 1) | ((xn[2] - cz) << 2);
-        const int lm = (xn[0] + DX - cx) | ((xn[1] + DY - cy) << 1) | ((xn[2] + DZ - cz) << 2);
-        const int idx = ln == lm ? ln : (ln > lm ? pair_index(ln, lm) : pair_index(lm, ln));
-        s += yo[(size_t)idx * C + cell];
-      }
-  return s;
-}
-
-template <int O>
-__device__ __forceinline__ float pair_sum_o(const Lat3 &L, const int *xn,
-                                            const float *__restrict__ yo, size_t C) {
-  return pair_sum<O % 3 - 1, (O / 3) % 3 - 1, O / 9 - 1>(L, xn, yo, C);
-}
-
-// One thread per lattice node n (row i of G): the column-i prefix (gl, rows of G)
-// and suffix (gu, rows of Gᵀ) of Ĝ in CSC positions, and the solver's copy of
-// G = Ĝ D^-1/2 in 16-slot rows: gle[i] = G(i, j ≤ i), gue[i] = G(j ≥ i, i).
+// One thread per lattice node n (row i of G).  The entry of n and its neighbour at offset
+// o is Σ over the cells holding both, in ascending cell order (both endpoints compute the
+// same bits); n is local node 7 ^ e of its e-th cell, so its 8 cells give 8 values each:
+// 64 loads, all in flight (cells outside the lattice read cell 0 and count 0).  Summed
+// inside a branch per neighbour and cell, as before, every load waited for the one
+// before (64³: 75 µs, now 51; 32³ with the CSC copies 36 µs, now 8).
+// Written: the column-i prefix (gl, rows of G) and suffix (gu, rows of Gᵀ) of Ĝ in CSC
+// positions (CSC), and (solver) the solver's copy of G = Ĝ D^-1/2 in 16-slot rows:
+// gle[i] = G(i, j ≤ i), gue[i] = G(j ≥ i, i).
 template <bool CSC>
-__global__ void g_assemble_kernel(Lat3 L, int nnodes, const int32_t *__restrict__ node_dof,
-                                  const uint32_t *__restrict__ fmask,
-                                  const int32_t *__restrict__ colptr,
-                                  const float *__restrict__ yo, const double *__restrict__ fs,
-                                  float *__restrict__ gl, float *__restrict__ gu,
-                                  float *__restrict__ gle, float *__restrict__ gue,
-                                  int64_t nfree, float *__restrict__ g14) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64) void g_assemble_kernel(
+    Lat3 L, int nnodes, const int32_t *__restrict__ node_dof, const uint32_t *__restrict__ fmask,
+    const int32_t *__restrict__ colptr, const float *__restrict__ yo,
+    const double *__restrict__ fs, float *__restrict__ gl, float *__restrict__ gu, bool solver,
+    float *__restrict__ gle, float *__restrict__ gue, int64_t nfree, float *__restrict__ g14) {
+  const int n = blockIdx.x * 64 + threadIdx.x;
   if (n >= nnodes) return;
   const int d0 = node_dof[n];
   if (d0 <= 0) return;
@@ -447,48 +683,81 @@ __global__ void g_assemble_kernel(Lat3 L, int nnodes, const int32_t *__restrict_
   node_xyz(L, n, xi);
   const uint32_t fm = fmask[n];
   const int p0 = colptr[d0 - 1];
+  const int C = L.nc[0] * L.nc[1] * L.nc[2];
+  float v[8][8];  // v[e][b]: cell e's value of the pair (n, its local node b)
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int cx = xi[0] - 1 + (e & 1), cy = xi[1] - 1 + ((e >> 1) & 1), cz = xi[2] - 1 + (e >> 2);
+    const bool in = cx >= 0 && cx < L.nc[0] && cy >= 0 && cy < L.nc[1] && cz >= 0 && cz < L.nc[2];
+    const int cell = in ? cx + L.nc[0] * (cy + L.nc[1] * cz) : 0;
+    const int a = 7 ^ e;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const int idx = a == b ? a : (a > b ? pair_index(a, b) : pair_index(b, a));
+      const float y = yo[(size_t)idx * C + cell];
+      v[e][b] = in ? y : 0.0f;
+    }
+  }
   const double sn = fs[d0 - 1];
+  // D^-1/2 of the lower neighbours (the node itself where there is none)
+  double sm[13];
+  if (solver) {
+    int dm[13];
+#pragma unroll
+    for (int o = 0; o < 13; ++o)
+      dm[o] = node_dof[(fm >> o) & 1u ? n + (o % 3 - 1) + L.nn[0] * (((o / 3) % 3 - 1) +
+                                                                   L.nn[1] * (o / 9 - 1))
+                                      : n];
+#pragma unroll
+    for (int o = 0; o < 13; ++o) sm[o] = fs[dm[o] - 1];
+  }
   float *el = gle + (size_t)(d0 - 1) * kEllSlots, *eu = gue + (size_t)(d0 - 1) * kEllSlots;
   int kl = 0, ku = 0;
-  float sums[27];
-  const size_t C = (size_t)L.nc[0] * L.nc[1] * L.nc[2];
-#define GH_PAIR(O) sums[O] = ((fm >> (O)) & 1u) ? pair_sum_o<O>(L, xi, yo, C) : 0.0f;
-  GH_PAIR(0) GH_PAIR(1) GH_PAIR(2) GH_PAIR(3) GH_PAIR(4) GH_PAIR(5) GH_PAIR(6) GH_PAIR(7)
-  GH_PAIR(8) GH_PAIR(9) GH_PAIR(10) GH_PAIR(11) GH_PAIR(12) GH_PAIR(13) GH_PAIR(14)
-  GH_PAIR(15) GH_PAIR(16) GH_PAIR(17) GH_PAIR(18) GH_PAIR(19) GH_PAIR(20) GH_PAIR(21)
-  GH_PAIR(22) GH_PAIR(23) GH_PAIR(24) GH_PAIR(25) GH_PAIR(26)
-#undef GH_PAIR
 #pragma unroll
   for (int o = 0; o < 27; ++o) {
-    if (!((fm >> o) & 1u)) continue;
+    const int dx = o % 3 - 1, dy = (o / 3) % 3 - 1, dz = o / 9 - 1;
+    float sum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int a = 7 ^ e;
+      const int bx = (a & 1) + dx, by = ((a >> 1) & 1) + dy, bz = (a >> 2) + dz;
+      if (bx >= 0 && bx <= 1 && by >= 0 && by <= 1 && bz >= 0 && bz <= 1)
+        sum += v[e][bx | (by << 1) | (bz << 2)];
+    }
+    if (!((fm >> o) & 1u)) {
+      // lower offsets whose neighbour is not free (outside the box): zero
+      if (o < 13 && solver && g14) g14[o * nfree + (d0 - 1)] = 0.0f;
+      continue;
+    }
     const int pos = p0 + __popc(fm & ((1u << o) - 1u));
-    const float sum = sums[o];
     if (o == 13) {
       const float g = expf(sum);
       if (CSC) {
         gl[pos] = g;
         gu[pos] = g;
       }
-      const float ge = (float)((double)g * sn);
-      el[kl++] = ge;
-      eu[ku++] = ge;
-      if (g14) g14[13 * nfree + (d0 - 1)] = ge;
+      if (solver) {
+        const float ge = (float)((double)g * sn);
+        el[kl++] = ge;
+        eu[ku++] = ge;
+        if (g14) g14[13 * nfree + (d0 - 1)] = ge;
+      }
     } else if (o < 13) {
       if (CSC) gl[pos] = sum;  // Ĝ(n, m), m < n
-      const int m = (xi[0] + o % 3 - 1) + L.nn[0] * ((xi[1] + (o / 3) % 3 - 1) +
-                                                     L.nn[1] * (xi[2] + o / 9 - 1));
-      el[kl++] = (float)((double)sum * fs[node_dof[m] - 1]);
-      if (g14) g14[o * nfree + (d0 - 1)] = el[kl - 1];
+      if (solver) {
+        const float ge = (float)((double)sum * sm[o]);
+        el[kl++] = ge;
+        if (g14) g14[o * nfree + (d0 - 1)] = ge;
+      }
     } else {
       if (CSC) gu[pos] = sum;  // Ĝ(m, n), m > n
-      eu[ku++] = (float)((double)sum * sn);
+      if (solver) eu[ku++] = (float)((double)sum * sn);
     }
   }
-  for (; kl < kEllSlots; ++kl) el[kl] = 0.0f;
-  for (; ku < kEllSlots; ++ku) eu[ku] = 0.0f;
-  if (g14)  // lower offsets whose neighbour is not free (outside the box): zero
-    for (int o = 0; o < 13; ++o)
-      if (!((fm >> o) & 1u)) g14[o * nfree + (d0 - 1)] = 0.0f;
+  if (solver) {
+    for (; kl < kEllSlots; ++kl) el[kl] = 0.0f;
+    for (; ku < kEllSlots; ++ku) eu[ku] = 0.0f;
+  }
 }
 
 // Column indices of the 16-slot rows (from the pattern; padding points at the row
@@ -507,135 +776,207 @@ __global__ void ell_index_kernel(int64_t n, const int32_t *__restrict__ cp,
   }
 }
 
-// ∂L/∂y_c from the pattern gradient (the transpose of g_assemble).
-__global__ void cell_grad_kernel(Lat3 L, int64_t ncells, const int32_t *__restrict__ node_dof,
-                                 const uint32_t *__restrict__ fmask,
-                                 const int32_t *__restrict__ colptr,
-                                 const int32_t *__restrict__ dpos,
-                                 const float *__restrict__ gG, const float *__restrict__ gl,
-                                 float *__restrict__ dy) {
-  int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// ∂L/∂y_c from the pattern gradient (the transpose of g_assemble).  The 36 gradient
+// loads of a cell are independent (a pair with a Dirichlet node reads entry 0 and
+// counts 0): 21 -> 7 µs at 32³.
+__global__ __launch_bounds__(64) void cell_grad_kernel(
+    Lat3 L, int ncells, const int32_t *__restrict__ node_dof, const uint32_t *__restrict__ fmask,
+    const int32_t *__restrict__ colptr, const float *__restrict__ gG,
+    const float *__restrict__ gl, float *__restrict__ dy) {
+  const int c = blockIdx.x * 64 + threadIdx.x;
   if (c >= ncells) return;
-  const int cx = (int)(c % L.nc[0]);
-  const int cy = (int)((c / L.nc[0]) % L.nc[1]);
-  const int cz = (int)(c / ((int64_t)L.nc[0] * L.nc[1]));
-  int dof[8];
+  const int cx = c % L.nc[0];
+  const int cy = (c / L.nc[0]) % L.nc[1];
+  const int cz = c / (L.nc[0] * L.nc[1]);
+  int dof[8], cp[8];
   uint32_t fm[8];
 #pragma unroll
   for (int a = 0; a < 8; ++a) {
     const int node = (cx + (a & 1)) + L.nn[0] * ((cy + ((a >> 1) & 1)) + L.nn[1] * (cz + (a >> 2)));
     dof[a] = node_dof[node];
-    fm[a] = dof[a] > 0 ? fmask[node] : 0u;
+    fm[a] = fmask[node];
   }
-  float *out = dy + c * kMlpOutPad;
+#pragma unroll
+  for (int a = 0; a < 8; ++a) cp[a] = colptr[max(dof[a], 1) - 1];
+  float out[kMlpOutPad] = {};
+  float gd[8];
 #pragma unroll
   for (int a = 0; a < 8; ++a) {
-    float g = 0.0f;
-    if (dof[a] > 0) {
-      const int pd = dpos[dof[a] - 1];
-      g = gG[pd] * gl[pd];
-    }
-    out[a] = g;
+    const int pd = dof[a] > 0 ? cp[a] + __popc(fm[a] & ((1u << 13) - 1u)) : 0;
+    out[a] = gG[pd];
+    gd[a] = gl[pd];
   }
 #pragma unroll
   for (int a = 1; a < 8; ++a)
 #pragma unroll
     for (int b = 0; b < a; ++b) {
-      float g = 0.0f;
-      if (dof[a] > 0 && dof[b] > 0) {
-        const int dx = (b & 1) - (a & 1), dyy = ((b >> 1) & 1) - ((a >> 1) & 1),
-                  dz = (b >> 2) - (a >> 2);
-        const int o = (dx + 1) + 3 * (dyy + 1) + 9 * (dz + 1);
-        const int pos = colptr[dof[a] - 1] + __popc(fm[a] & ((1u << o) - 1u));
-        g = gG[pos];
-      }
-      out[pair_index(a, b)] = g;
+      const int o = ((b & 1) - (a & 1) + 1) + 3 * (((b >> 1) & 1) - ((a >> 1) & 1) + 1) +
+                    9 * ((b >> 2) - (a >> 2) + 1);
+      const bool in = dof[a] > 0 && dof[b] > 0;
+      const float g = gG[in ? cp[a] + __popc(fm[a] & ((1u << o) - 1u)) : 0];
+      out[pair_index(a, b)] = in ? g : 0.0f;
     }
 #pragma unroll
-  for (int k = kMlpOut; k < kMlpOutPad; ++k) out[k] = 0.0f;
+  for (int a = 0; a < 8; ++a) out[a] = dof[a] > 0 ? out[a] * gd[a] : 0.0f;
+  float4 *p = reinterpret_cast<float4 *>(dy + (size_t)c * kMlpOutPad);
+#pragma unroll
+  for (int q = 0; q < kMlpOutPad / 4; ++q)
+    p[q] = make_float4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
 }
 
-// ---- applications of G and Gᵀ ------------------------------------------------
+// ---- probes -----------------------------------------------------------------------------
+// NB probes at a time, their vectors interleaved ([row][NB]), so that the matrix and the
+// factor are read once per batch and a column is one gather of NB values.  A row's
+// entries are spread over its lanes, all of a turn's loads in flight (four kernels per
+// probe with one entry at a time: 40 µs and 8 launches a probe at 32³; now 31 µs and 7
+// launches for four).
 
-constexpr int kApplyLanes = 4;
+constexpr int kApplyLanes = 4, kApplyTurn = 4;   // a half row: at most 14 entries of 16
+constexpr int kMultiLanes = 8, kMultiTurn = 4;   // a full row: at most 27 of 32
 
-// y_i = Σ_{j <= i} Ĝ_ij s_j r_j  (column-i prefix)
-__global__ __launch_bounds__(256) void apply_lower_kernel(int64_t n, const int32_t *__restrict__ cp,
-                                                          const int32_t *__restrict__ rv,
-                                                          const int32_t *__restrict__ dpos,
-                                                          const float *__restrict__ gl,
-                                                          const double *__restrict__ fs,
-                                                          const double *__restrict__ r,
-                                                          double *__restrict__ y) {
-  const int sub = threadIdx.x % kApplyLanes;
+// bit k of sg[i]: the sign of probe first + k at i (set: +1)
+__global__ void rademacher_kernel(int64_t n, uint64_t seed, uint64_t first, int nb,
+                                  uint8_t *__restrict__ sg) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  uint32_t m = 0;
+  for (int k = 0; k < nb; ++k)
+    m |= (rademacher(seed, first + (uint64_t)k, (uint64_t)i) > 0.0 ? 1u : 0u) << k;
+  sg[i] = (uint8_t)m;
+}
+
+template <int NB>
+struct Vals {
+  double v[NB];
+};
+template <int NB>
+__device__ __forceinline__ Vals<NB> signs(const uint8_t *__restrict__ sg, int64_t i) {
+  const uint32_t m = sg[i];
+  Vals<NB> r;
+#pragma unroll
+  for (int k = 0; k < NB; ++k) r.v[k] = (m >> k) & 1u ? 1.0 : -1.0;
+  return r;
+}
+template <int NB>
+__device__ __forceinline__ Vals<NB> load_vals(const double *__restrict__ x, int64_t i) {
+  Vals<NB> r;
+  if constexpr (NB % 2 == 0) {
+#pragma unroll
+    for (int k = 0; k < NB; k += 2) {
+      const double2 d = *reinterpret_cast<const double2 *>(x + i * NB + k);
+      r.v[k] = d.x;
+      r.v[k + 1] = d.y;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < NB; ++k) r.v[k] = x[i * NB + k];
+  }
+  return r;
+}
+
+// s_k += Σ over entries [p0, p1) of the row, L lanes and U entries each: wt(p) f(rv[p])
+template <int L, int U, int NB, class Wt, class F>
+__device__ __forceinline__ void row_dot(int p0, int p1, const int32_t *__restrict__ rv, Wt wt,
+                                        F f, double (&s)[NB]) {
+  const int sub = threadIdx.x % L;
+  for (int p = p0; p < p1; p += L * U) {
+    int j[U];
+    double w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = min(p + sub + u * L, p1 - 1);
+      j[u] = rv[q];
+      w[u] = wt(q);
+    }
+    Vals<NB> g[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) g[u] = f(j[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (p + sub + u * L < p1)
+#pragma unroll
+        for (int k = 0; k < NB; ++k) s[k] += w[u] * g[u].v[k];
+  }
+#pragma unroll
+  for (int k = 0; k < NB; ++k)
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) s[k] += __shfl_xor(s[k], o);
+}
+
+// z_j = s_j Σ_{i >= j} Ĝ_ij y_i  (column-j suffix); SIGNS: y are the probes themselves
+template <int NB, bool SIGNS>
+__global__ __launch_bounds__(256) void apply_upper_kernel(
+    int64_t n, const int32_t *__restrict__ cp, const int32_t *__restrict__ rv,
+    const int32_t *__restrict__ dpos, const float *__restrict__ gu,
+    const double *__restrict__ fs, const uint8_t *__restrict__ sg, const double *__restrict__ y,
+    double *__restrict__ z) {
   const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kApplyLanes;
-  double s = 0.0;
-  if (row < n) {
-    for (int p = cp[row] + sub; p <= dpos[row]; p += kApplyLanes) {
-      const int j = rv[p];
-      s += (double)gl[p] * fs[j] * r[j];
-    }
-  }
+  double s[NB] = {};
+  if (row < n)
+    row_dot<kApplyLanes, kApplyTurn, NB>(
+        dpos[row], cp[row + 1], rv, [&](int p) { return (double)gu[p]; },
+        [&](int j) {
+          if constexpr (SIGNS) return signs<NB>(sg, j);
+          else return load_vals<NB>(y, j);
+        },
+        s);
+  if (row < n && threadIdx.x % kApplyLanes == 0) {
+    const double f = fs[row];
 #pragma unroll
-  for (int o = kApplyLanes / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (row < n && sub == 0) y[row] = s;
+    for (int k = 0; k < NB; ++k) z[row * NB + k] = f * s[k];
+  }
 }
 
-// z_j = s_j Σ_{i >= j} Ĝ_ij y_i  (column-j suffix); optional block partials of z·d
-__global__ __launch_bounds__(256) void apply_upper_kernel(int64_t n, const int32_t *__restrict__ cp,
-                                                          const int32_t *__restrict__ rv,
-                                                          const int32_t *__restrict__ dpos,
-                                                          const float *__restrict__ gu,
-                                                          const double *__restrict__ fs,
-                                                          const double *__restrict__ y,
-                                                          double *__restrict__ z,
-                                                          const double *__restrict__ d,
-                                                          double *__restrict__ part) {
-  __shared__ double sh[4];
-  const int sub = threadIdx.x % kApplyLanes;
-  double dot = 0.0;
-  const int64_t rows_per_iter = (int64_t)gridDim.x * (blockDim.x / kApplyLanes);
-  for (int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kApplyLanes; row < n;
-       row += rows_per_iter) {
-    double s = 0.0;
-    for (int p = dpos[row] + sub; p < cp[row + 1]; p += kApplyLanes) s += (double)gu[p] * y[rv[p]];
+// y = A x
+template <int NB>
+__global__ __launch_bounds__(256) void spmv_multi_kernel(
+    int64_t n, const int32_t *__restrict__ cp, const int32_t *__restrict__ rv,
+    const double *__restrict__ val, const double *__restrict__ x, double *__restrict__ y) {
+  const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kMultiLanes;
+  double s[NB] = {};
+  if (row < n)
+    row_dot<kMultiLanes, kMultiTurn, NB>(
+        cp[row], cp[row + 1], rv, [&](int p) { return val[p]; },
+        [&](int j) { return load_vals<NB>(x, j); }, s);
+  if (row < n && threadIdx.x % kMultiLanes == 0)
 #pragma unroll
-    for (int o = kApplyLanes / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if (sub == 0) {
-      const double zj = fs[row] * s;
-      z[row] = zj;
-      if (d) dot += zj * d[row];
-    }
-  }
-  if (part) {
-    for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) sh[w] = dot;
-    __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
-  }
+    for (int k = 0; k < NB; ++k) y[row * NB + k] = s[k];
 }
 
-// ---- training pieces -------------------------------------------------------------
-
-__global__ void rademacher_kernel(int64_t n, uint64_t seed, uint64_t probe,
-                                  double *__restrict__ z) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) z[i] = rademacher(seed, probe, (uint64_t)i);
-}
-
-// r = z - u; block partials of r·r added to lpart (one slot per block)
-__global__ __launch_bounds__(256) void residual_kernel(int64_t n, const double *__restrict__ z,
-                                                       const double *__restrict__ u,
-                                                       double *__restrict__ r,
-                                                       double *__restrict__ lpart) {
+// r = z − u, u_i = Σ_{j <= i} Ĝ_ij s_j v_j (column-i prefix); block partials of r·r over
+// the probes, added to lpart (one slot per block)
+template <int NB>
+__global__ __launch_bounds__(256) void residual_kernel(
+    int64_t n, const int32_t *__restrict__ cp, const int32_t *__restrict__ rv,
+    const int32_t *__restrict__ dpos, const float *__restrict__ gl,
+    const double *__restrict__ fs, const uint8_t *__restrict__ sg, const double *__restrict__ v,
+    double *__restrict__ r, double *__restrict__ lpart) {
   __shared__ double sh[4];
   double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double ri = z[i] - u[i];
-    r[i] = ri;
-    acc += ri * ri;
+  const int64_t step = (int64_t)gridDim.x * (256 / kApplyLanes);
+  for (int64_t r0 = (int64_t)blockIdx.x * (256 / kApplyLanes); r0 < n; r0 += step) {
+    const int64_t row = r0 + threadIdx.x / kApplyLanes;
+    double s[NB] = {};
+    if (row < n)
+      row_dot<kApplyLanes, kApplyTurn, NB>(
+          cp[row], dpos[row] + 1, rv, [&](int p) { return (double)gl[p]; },
+          [&](int j) {
+            Vals<NB> x = load_vals<NB>(v, j);
+            const double f = fs[j];
+#pragma unroll
+            for (int k = 0; k < NB; ++k) x.v[k] *= f;
+            return x;
+          },
+          s);
+    if (row < n && threadIdx.x % kApplyLanes == 0) {
+      const Vals<NB> z = signs<NB>(sg, row);
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const double ri = z.v[k] - s[k];
+        r[row * NB + k] = ri;
+        acc += ri * ri;
+      }
+    }
   }
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -644,20 +985,40 @@ __global__ __launch_bounds__(256) void residual_kernel(int64_t n, const double *
   if (threadIdx.x == 0) lpart[blockIdx.x] += sh[0] + sh[1] + sh[2] + sh[3];
 }
 
-// gĜ_ij += coef (r_i v_j + z_i q_j) s_j on the lower pattern (column-i prefix)
-__global__ void pattern_grad_kernel(int64_t n, const int32_t *__restrict__ cp,
-                                    const int32_t *__restrict__ rv,
-                                    const int32_t *__restrict__ dpos,
-                                    const double *__restrict__ fs, const double *__restrict__ r,
-                                    const double *__restrict__ v, const double *__restrict__ z,
-                                    const double *__restrict__ q, double coef,
-                                    float *__restrict__ gG) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double ri = r[i], zi = z[i];
-  for (int p = cp[i]; p <= dpos[i]; ++p) {
-    const int j = rv[p];
-    gG[p] += (float)(coef * (ri * v[j] + zi * q[j]) * fs[j]);
+// gĜ_ij (+)= coef Σ_k (r_i v_j + z_i q_j) s_j on the lower pattern (column-i prefix); the
+// first batch writes
+template <int NB>
+__global__ __launch_bounds__(256) void pattern_grad_kernel(
+    int64_t n, const int32_t *__restrict__ cp, const int32_t *__restrict__ rv,
+    const int32_t *__restrict__ dpos, const double *__restrict__ fs,
+    const double *__restrict__ r, const double *__restrict__ v, const uint8_t *__restrict__ sg,
+    const double *__restrict__ q, double coef, bool add, float *__restrict__ gG) {
+  const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kApplyLanes;
+  if (row >= n) return;
+  const Vals<NB> ri = load_vals<NB>(r, row), zi = signs<NB>(sg, row);
+  const int p0 = cp[row] + threadIdx.x % kApplyLanes, p1 = dpos[row];
+  for (int p = p0; p <= p1; p += kApplyLanes * kApplyTurn) {
+    int j[kApplyTurn];
+    double f[kApplyTurn];
+    Vals<NB> vj[kApplyTurn], qj[kApplyTurn];
+#pragma unroll
+    for (int u = 0; u < kApplyTurn; ++u) j[u] = rv[min(p + u * kApplyLanes, p1)];
+#pragma unroll
+    for (int u = 0; u < kApplyTurn; ++u) {
+      vj[u] = load_vals<NB>(v, j[u]);
+      qj[u] = load_vals<NB>(q, j[u]);
+      f[u] = fs[j[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < kApplyTurn; ++u) {
+      const int at = p + u * kApplyLanes;
+      if (at > p1) continue;
+      double t = 0.0;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) t += ri.v[k] * vj[u].v[k] + zi.v[k] * qj[u].v[k];
+      const float d = (float)(coef * t * f[u]);
+      gG[at] = add ? gG[at] + d : d;
+    }
   }
 }
 
@@ -673,6 +1034,7 @@ Lat3 lattice_of(const Ctx &c) {
 }
 
 constexpr int kResidualBlocks = 512;
+constexpr int kProbeBatch = 4;
 
 }  // namespace
 
@@ -683,26 +1045,18 @@ void fsai_prepare(Ctx &c) {
   const int64_t n = c.nfree, C = c.ncells;
   if (!c.fsai_ready) {
     c.diagpos.resize(std::max<int64_t>(n, 1));
+    c.diag.resize(std::max<int64_t>(n, 1));
     c.fs.resize(std::max<int64_t>(n, 1));
     c.gl.resize(std::max<int64_t>(c.nnz, 1));
     c.gu.resize(std::max<int64_t>(c.nnz, 1));
-    c.gG.resize(std::max<int64_t>(c.nnz, 1));
     c.feat.resize(C * kMlpInPad);
-    for (auto *b : {&c.z1, &c.h1, &c.z2, &c.h2, &c.z3, &c.h3, &c.dz1, &c.dz2, &c.dz3})
-      b->resize(C * kMlpHidden);
     c.yo.resize(C * kMlpOut);  // output-major: yo[n * C + cell]
-    c.dy.resize(C * kMlpOutPad);
-    const int nb = (int)((C + kMlpCellsPerBlock - 1) / kMlpCellsPerBlock);
-    c.wpart.resize((size_t)nb * (kMlpHidden * kMlpHidden + kMlpHidden));
-    for (auto *b : {&c.pz, &c.pw, &c.pv, &c.pu, &c.pr, &c.pt, &c.pq})
-      b->resize(std::max<int64_t>(n, 1));
-    c.lpart.resize(kResidualBlocks);
     for (auto *b : {&c.gle, &c.gue}) b->resize((size_t)std::max<int64_t>(n, 1) * kEllSlots);
     for (auto *b : {&c.gli, &c.gui}) b->resize((size_t)std::max<int64_t>(n, 1) * kEllSlots);
   }
-  hipLaunchKernelGGL(diag_setup_kernel, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n,
-                     c.colptr.get(), c.rowval.get(), c.nzval.get(), c.diagpos.get(),
-                     c.fs.get());
+  hipLaunchKernelGGL(diag_setup_kernel, dim3(grid_for(c.nnodes)), dim3(kBlock), 0, c.stream,
+                     (int)c.nnodes, c.node_dof.get(), c.node_fmask.get(), c.colptr.get(),
+                     c.nzval.get(), c.diagpos.get(), c.diag.get(), c.fs.get());
   GH_CHECK_HIP(hipGetLastError());
   if (!c.fsai_ready) {
     DBuf<int> ovf;
@@ -726,7 +1080,7 @@ void mlp_sync_bf16(Ctx &c) {
   GH_CHECK_HIP(hipGetLastError());
 }
 
-void fsai_forward_build(Ctx &c, bool inference) {
+void fsai_forward_build(Ctx &c, bool inference, bool solver) {
   GH_REQUIRE(c.have_mlp, GH_ERR_STATE, "no network weights: call gh_mlp_init or gh_mlp_set");
   fsai_prepare(c);
   const Lat3 L = lattice_of(c);
@@ -747,8 +1101,8 @@ void fsai_forward_build(Ctx &c, bool inference) {
   const float logh = (float)(std::log(c.sizes[0] * c.sizes[1] * c.sizes[2]) / 3.0);
   hipStream_t s = c.stream;
   hipLaunchKernelGGL(features_kernel, dim3(grid_for(C)), dim3(kBlock), 0, s, L, (int64_t)C,
-                     c.have_kappa ? c.kappa.get() : nullptr, c.node_dof.get(), c.diagpos.get(),
-                     c.nzval.get(), kdiag, logh, c.feat.get());
+                     c.have_kappa ? c.kappa.get() : nullptr, c.node_dof.get(), c.diag.get(),
+                     kdiag, logh, c.feat.get());
   if (inference) {
     const int ntiles = (C + 15) / 16;
     const unsigned grid =
@@ -756,20 +1110,9 @@ void fsai_forward_build(Ctx &c, bool inference) {
     hipLaunchKernelGGL(mlp_fwd_mfma, dim3(grid), dim3(kFwdWaves * 64), 0, s, c.feat.get(),
                        c.params_bf16.get(), C, c.yo.get());
   } else {
-    const int nb = (C + kMlpFwdCells - 1) / kMlpFwdCells;
-    const uint16_t *wq = c.params_bf16.get();
-    hipLaunchKernelGGL((mlp_fwd<kMlpIn, kMlpInPad, kMlpHidden, kMlpHidden, true>), dim3(nb),
-                       dim3(64), 0, s, c.feat.get(), wq, kMlpW1, kMlpB1, c.z1.get(), c.h1.get(), C,
-                       kMlpFwdCells);
-    hipLaunchKernelGGL((mlp_fwd<kMlpHidden, kMlpHidden, kMlpHidden, kMlpHidden, true>), dim3(nb),
-                       dim3(64), 0, s, c.h1.get(), wq, kMlpW2, kMlpB2, c.z2.get(), c.h2.get(), C,
-                       kMlpFwdCells);
-    hipLaunchKernelGGL((mlp_fwd<kMlpHidden, kMlpHidden, kMlpHidden, kMlpHidden, true>), dim3(nb),
-                       dim3(64), 0, s, c.h2.get(), wq, kMlpW3, kMlpB3, c.z3.get(), c.h3.get(), C,
-                       kMlpFwdCells);
-    hipLaunchKernelGGL((mlp_fwd<kMlpHidden, kMlpHidden, kMlpOut, kMlpOutPad, false, true>), dim3(nb),
-                       dim3(64), 0, s, c.h3.get(), wq, kMlpW4, kMlpB4, c.yo.get(),
-                       (float *)nullptr, C, kMlpFwdCells);
+    const unsigned grid = (unsigned)std::min((C + kTrainCells - 1) / kTrainCells, 2 * kTrainGrid);
+    hipLaunchKernelGGL(mlp_train_fwd, dim3(grid), dim3(256), sizeof(TrainLds), s, c.feat.get(),
+                       c.params_bf16.get(), C, c.yo.get());
   }
   // box lattice: also the 14 lower-offset arrays of G for the stencil PCG kernels
   float *g14 = nullptr;
@@ -777,109 +1120,95 @@ void fsai_forward_build(Ctx &c, bool inference) {
     c.g14.resize((size_t)14 * std::max<int64_t>(c.nfree, 1));
     g14 = c.g14.get();
   }
-  if (inference)
-    hipLaunchKernelGGL(g_assemble_kernel<false>, dim3(grid_for(c.nnodes)), dim3(kBlock), 0, s, L,
-                       (int)c.nnodes, c.node_dof.get(), c.node_fmask.get(), c.colptr.get(),
-                       c.yo.get(), c.fs.get(), c.gl.get(), c.gu.get(), c.gle.get(), c.gue.get(),
-                       c.nfree, g14);
-  else
-    hipLaunchKernelGGL(g_assemble_kernel<true>, dim3(grid_for(c.nnodes)), dim3(kBlock), 0, s, L,
-                       (int)c.nnodes, c.node_dof.get(), c.node_fmask.get(), c.colptr.get(),
-                       c.yo.get(), c.fs.get(), c.gl.get(), c.gu.get(), c.gle.get(), c.gue.get(),
-                       c.nfree, g14);
+  auto g_kern = inference ? g_assemble_kernel<false> : g_assemble_kernel<true>;
+  hipLaunchKernelGGL(g_kern, dim3(grid_for(c.nnodes, 64)), dim3(64), 0, s, L, (int)c.nnodes,
+                     c.node_dof.get(), c.node_fmask.get(), c.colptr.get(), c.yo.get(),
+                     c.fs.get(), c.gl.get(), c.gu.get(), solver, c.gle.get(), c.gue.get(),
+                     c.nfree, g14);
   GH_CHECK_HIP(hipGetLastError());
-  c.fsai_built = true;
+  c.fsai_built = solver;
 }
 
-void fsai_apply_lower(Ctx &c, const double *r, double *y) {
+namespace {
+
+// One batch of NB probes from probe `first` on: loss partials and gĜ.
+template <int NB>
+void probe_batch(Ctx &c, uint64_t seed, int first, double coef) {
+  hipStream_t s = c.stream;
   const int64_t n = c.nfree;
-  const unsigned grid = (unsigned)((n * kApplyLanes + 255) / 256);
-  hipLaunchKernelGGL(apply_lower_kernel, dim3(std::max(grid, 1u)), dim3(256), 0, c.stream, n,
-                     c.colptr.get(), c.rowval.get(), c.diagpos.get(), c.gl.get(), c.fs.get(),
-                     r, y);
+  const int32_t *cp = c.colptr.get(), *rv = c.rowval.get(), *dp = c.diagpos.get();
+  const double *fs = c.fs.get();
+  const uint8_t *sg = c.psign.get();
+  const dim3 half(grid_for(n * kApplyLanes)), full(grid_for(n * kMultiLanes)), block(256);
+  hipLaunchKernelGGL(rademacher_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, n, seed,
+                     (uint64_t)first, NB, c.psign.get());
+  // w = Gᵀ z, v = A w, r = z − G v, t = Gᵀ r, q = A t
+  hipLaunchKernelGGL((apply_upper_kernel<NB, true>), half, block, 0, s, n, cp, rv, dp, c.gu.get(),
+                     fs, sg, (const double *)nullptr, c.pw.get());
+  hipLaunchKernelGGL(spmv_multi_kernel<NB>, full, block, 0, s, n, cp, rv, c.nzval.get(),
+                     c.pw.get(), c.pv.get());
+  hipLaunchKernelGGL(residual_kernel<NB>, dim3(kResidualBlocks), block, 0, s, n, cp, rv, dp,
+                     c.gl.get(), fs, sg, c.pv.get(), c.pr.get(), c.lpart.get());
+  hipLaunchKernelGGL((apply_upper_kernel<NB, false>), half, block, 0, s, n, cp, rv, dp,
+                     c.gu.get(), fs, sg, c.pr.get(), c.pw.get());
+  hipLaunchKernelGGL(spmv_multi_kernel<NB>, full, block, 0, s, n, cp, rv, c.nzval.get(),
+                     c.pw.get(), c.pq.get());
+  hipLaunchKernelGGL(pattern_grad_kernel<NB>, half, block, 0, s, n, cp, rv, dp, fs, c.pr.get(),
+                     c.pv.get(), sg, c.pq.get(), coef, first > 0, c.gG.get());
   GH_CHECK_HIP(hipGetLastError());
 }
 
-// grid of the upper apply: `parts` blocks when partials are requested (the PCG
-// reduction expects exactly that many), else one row group per thread group.
-void fsai_apply_upper_grid(Ctx &c, const double *y, double *z, const double *d, double *part,
-                           int parts) {
-  const int64_t n = c.nfree;
-  unsigned grid = part ? (unsigned)parts : (unsigned)((n * kApplyLanes + 255) / 256);
-  hipLaunchKernelGGL(apply_upper_kernel, dim3(std::max(grid, 1u)), dim3(256), 0, c.stream, n,
-                     c.colptr.get(), c.rowval.get(), c.diagpos.get(), c.gu.get(), c.fs.get(),
-                     y, z, d, part);
-  GH_CHECK_HIP(hipGetLastError());
+__global__ void clear_kernel(int n, double *v) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) v[i] = 0.0;
 }
+
+}  // namespace
 
 double fsai_train_step(Ctx &c, int nprobes, uint64_t seed, float lr) {
   GH_REQUIRE(nprobes >= 1 && nprobes <= 1024, GH_ERR_ARG, "nprobes must be in 1..1024");
-  fsai_forward_build(c, false);
+  // a step that changes the weights leaves no factor for the solver: its copy is not written
+  fsai_forward_build(c, false, !(lr > 0.0f));
   hipStream_t s = c.stream;
   const int64_t n = c.nfree;
   const int C = (int)c.ncells;
   const Lat3 L = lattice_of(c);
-  GH_CHECK_HIP(hipMemsetAsync(c.gG.get(), 0, sizeof(float) * std::max<int64_t>(c.nnz, 1), s));
-  GH_CHECK_HIP(hipMemsetAsync(c.lpart.get(), 0, sizeof(double) * kResidualBlocks, s));
+  // workspace of the training step, at its first one
+  const size_t nv = (size_t)std::max<int64_t>(n, 1) * kProbeBatch;
+  for (auto *b : {&c.pw, &c.pv, &c.pr, &c.pq}) b->resize(nv);
+  c.psign.resize(std::max<int64_t>(n, 1));
+  c.gG.resize(std::max<int64_t>(c.nnz, 1));
+  c.lpart.resize(kResidualBlocks);
+  c.dy.resize((size_t)C * kMlpOutPad);
+  const int nb = std::min((C + kTrainCells - 1) / kTrainCells, kTrainGrid);
+  c.wpart.resize((size_t)nb * kMlpParams);
+  hipLaunchKernelGGL(clear_kernel, dim3(2), dim3(256), 0, s, kResidualBlocks, c.lpart.get());
   const double coef = -2.0 / ((double)nprobes * (double)std::max<int64_t>(n, 1));
-  for (int k = 0; k < nprobes; ++k) {
-    hipLaunchKernelGGL(rademacher_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, n, seed,
-                       (uint64_t)k, c.pz.get());
-    fsai_apply_upper_grid(c, c.pz.get(), c.pw.get(), nullptr, nullptr, 0);   // w = Gᵀ z
-    spmv_device(c, c.pw.get(), c.pv.get());                                  // v = A w
-    fsai_apply_lower(c, c.pv.get(), c.pu.get());                             // u = G v
-    hipLaunchKernelGGL(residual_kernel, dim3(kResidualBlocks), dim3(256), 0, s, n, c.pz.get(),
-                       c.pu.get(), c.pr.get(), c.lpart.get());               // r = z - u
-    fsai_apply_upper_grid(c, c.pr.get(), c.pt.get(), nullptr, nullptr, 0);   // t = Gᵀ r
-    spmv_device(c, c.pt.get(), c.pq.get());                                  // q = A t
-    hipLaunchKernelGGL(pattern_grad_kernel, dim3(grid_for(n)), dim3(kBlock), 0, s, n,
-                       c.colptr.get(), c.rowval.get(), c.diagpos.get(), c.fs.get(), c.pr.get(),
-                       c.pv.get(), c.pz.get(), c.pq.get(), coef, c.gG.get());
+  int k = 0;
+  for (; k + 4 <= nprobes; k += 4) probe_batch<4>(c, seed, k, coef);
+  if (k + 2 <= nprobes) {
+    probe_batch<2>(c, seed, k, coef);
+    k += 2;
   }
-  hipLaunchKernelGGL(cell_grad_kernel, dim3(grid_for(C)), dim3(kBlock), 0, s, L, (int64_t)C,
-                     c.node_dof.get(), c.node_fmask.get(), c.colptr.get(), c.diagpos.get(),
-                     c.gG.get(), c.gl.get(), c.dy.get());
+  if (k < nprobes) probe_batch<1>(c, seed, k, coef);
+  hipLaunchKernelGGL(cell_grad_kernel, dim3(grid_for(C, 64)), dim3(64), 0, s, L, C,
+                     c.node_dof.get(), c.node_fmask.get(), c.colptr.get(), c.gG.get(),
+                     c.gl.get(), c.dy.get());
   GH_CHECK_HIP(hipGetLastError());
-  // back-propagation (weights are the BF16 values the forward pass used)
-  const int nb = (C + kMlpCellsPerBlock - 1) / kMlpCellsPerBlock;
-  const uint16_t *wq = c.params_bf16.get();
-  float *gr = c.grads.get();
-  auto wgrad_reduce = [&](int off, int len) {
-    hipLaunchKernelGGL(reduce_parts, dim3(grid_for(len)), dim3(kBlock), 0, s, c.wpart.get(), nb,
-                       len, gr + off);
-  };
-  hipLaunchKernelGGL((mlp_wgrad<kMlpHidden, kMlpHidden, kMlpOut, kMlpOutPad>), dim3(nb),
-                     dim3(64), 0, s, c.dy.get(), c.h3.get(), c.wpart.get(), C, kMlpCellsPerBlock);
-  wgrad_reduce(kMlpW4, kMlpOut * kMlpHidden + kMlpOut);
-  hipLaunchKernelGGL((mlp_bwd<kMlpOut, kMlpOutPad, kMlpHidden, kMlpHidden>), dim3(nb), dim3(64),
-                     0, s, c.dy.get(), wq, kMlpW4, c.z3.get(), c.dz3.get(), C, kMlpCellsPerBlock);
-  hipLaunchKernelGGL((mlp_wgrad<kMlpHidden, kMlpHidden, kMlpHidden, kMlpHidden>), dim3(nb),
-                     dim3(64), 0, s, c.dz3.get(), c.h2.get(), c.wpart.get(), C,
-                     kMlpCellsPerBlock);
-  wgrad_reduce(kMlpW3, kMlpHidden * kMlpHidden + kMlpHidden);
-  hipLaunchKernelGGL((mlp_bwd<kMlpHidden, kMlpHidden, kMlpHidden, kMlpHidden>), dim3(nb),
-                     dim3(64), 0, s, c.dz3.get(), wq, kMlpW3, c.z2.get(), c.dz2.get(), C,
-                     kMlpCellsPerBlock);
-  hipLaunchKernelGGL((mlp_wgrad<kMlpHidden, kMlpHidden, kMlpHidden, kMlpHidden>), dim3(nb),
-                     dim3(64), 0, s, c.dz2.get(), c.h1.get(), c.wpart.get(), C,
-                     kMlpCellsPerBlock);
-  wgrad_reduce(kMlpW2, kMlpHidden * kMlpHidden + kMlpHidden);
-  hipLaunchKernelGGL((mlp_bwd<kMlpHidden, kMlpHidden, kMlpHidden, kMlpHidden>), dim3(nb),
-                     dim3(64), 0, s, c.dz2.get(), wq, kMlpW2, c.z1.get(), c.dz1.get(), C,
-                     kMlpCellsPerBlock);
-  hipLaunchKernelGGL((mlp_wgrad<kMlpIn, kMlpInPad, kMlpHidden, kMlpHidden>), dim3(nb), dim3(64),
-                     0, s, c.dz1.get(), c.feat.get(), c.wpart.get(), C, kMlpCellsPerBlock);
-  wgrad_reduce(kMlpW1, kMlpHidden * kMlpIn + kMlpHidden);
-  GH_CHECK_HIP(hipGetLastError());
+  // back-propagation (weights are the BF16 values the forward pass used), Adam
+  hipLaunchKernelGGL(mlp_train_bwd, dim3(nb), dim3(256), sizeof(TrainLds) + sizeof(TrainWeights),
+                     s, c.feat.get(), c.params_bf16.get(), c.dy.get(), C, c.wpart.get());
+  float b1t = 0.0f, b2t = 0.0f;
   if (lr > 0.0f) {
     ++c.adam_t;
-    const float b1t = (float)std::pow(0.9, c.adam_t), b2t = (float)std::pow(0.999, c.adam_t);
-    hipLaunchKernelGGL(adam_kernel, dim3(grid_for(kMlpParams)), dim3(kBlock), 0, s, kMlpParams,
-                       c.params.get(), c.grads.get(), c.adam_m.get(), c.adam_v.get(), lr, b1t,
-                       b2t, c.params_bf16.get());
-    GH_CHECK_HIP(hipGetLastError());
-    c.fsai_built = false;  // G still holds the factor of the weights before the step
+    b1t = (float)std::pow(0.9, c.adam_t);
+    b2t = (float)std::pow(0.999, c.adam_t);
   }
+  hipLaunchKernelGGL(reduce_adam_kernel,
+                     dim3(grid_for(kMlpParams, 256 / kReduceLanes)), dim3(256), 0, s,
+                     c.wpart.get(), nb, c.grads.get(), lr, b1t, b2t, c.params.get(),
+                     c.adam_m.get(), c.adam_v.get(), c.params_bf16.get());
+  GH_CHECK_HIP(hipGetLastError());
   double lp[kResidualBlocks];
   GH_CHECK_HIP(hipMemcpyAsync(lp, c.lpart.get(), sizeof(lp), hipMemcpyDeviceToHost, s));
   GH_CHECK_HIP(hipStreamSynchronize(s));

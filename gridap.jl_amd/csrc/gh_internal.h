@@ -305,19 +305,19 @@ struct Ctx {
   bool fsai_ready = false;   // structures allocated for the current pattern
   bool fsai_built = false;   // G holds the factor of the current matrix
   DBuf<int32_t> diagpos;     // N: nzval position of each column's diagonal
+  DBuf<double> diag;         // N: diag(A)
   DBuf<double> fs;           // N: diag(A)^(-1/2)
   DBuf<float> gl, gu;        // NNZ: Ĝ in column-prefix (rows of G) and suffix (rows of Gᵀ) layout
   DBuf<float> gG;            // NNZ: loss gradient w.r.t. Ĝ, prefix layout
   DBuf<float> gle, gue;      // N x 16: rows of G = Ĝ D^-1/2 and of Gᵀ (solver copy)
   DBuf<int32_t> gli, gui;    // N x 16: their column indices (padding: the row itself)
   DBuf<float> feat;          // C x 16 (10 used)
-  DBuf<float> z1, h1, z2, h2, z3, h3;  // C x 64 pre-/post-activations
   DBuf<float> yo, dy;        // C x 40 (36 used): network output and its gradient
-  DBuf<float> dz1, dz2, dz3; // C x 64
   DBuf<float> params, grads, adam_m, adam_v;  // NPARAM, FP32 master copy and Adam state
   DBuf<uint16_t> params_bf16;                 // the weights the kernels use
   DBuf<float> wpart;         // per-block weight-gradient partials
-  DBuf<double> pz, pw, pv, pu, pr, pt, pq, lpart;  // probe vectors, loss partials
+  DBuf<double> pw, pv, pr, pq, lpart;         // probe vectors (N x batch), loss partials
+  DBuf<uint8_t> psign;                        // signs of a batch of probes
   int adam_t = 0;
   bool have_mlp = false;
 };
@@ -377,11 +377,10 @@ constexpr int kMlpIn = 10, kMlpInPad = 16, kMlpHidden = 64, kMlpOut = 36, kMlpOu
 constexpr int kMlpW1 = 0, kMlpB1 = 640, kMlpW2 = 704, kMlpB2 = 4800, kMlpW3 = 4864,
               kMlpB3 = 8960, kMlpW4 = 9024, kMlpB4 = 11328, kMlpParams = 11364;
 void fsai_prepare(Ctx &c);                       // diag positions, D^-1/2, buffers
-// features -> MLP -> Ĝ; inference: the BF16 matrix-core forward (no stored
-// activations), else the FP32 forward that keeps the activations for training
-void fsai_forward_build(Ctx &c, bool inference);
+// features -> MLP -> Ĝ; inference: the BF16 matrix-core forward, else the FP32 forward of
+// training (Ĝ also in CSC positions); solver: write the solver's copy of G
+void fsai_forward_build(Ctx &c, bool inference, bool solver = true);
 double fsai_train_step(Ctx &c, int nprobes, uint64_t seed, float lr);
-void fsai_apply_lower(Ctx &c, const double *r, double *y);   // y = Ĝ (D^-1/2 r)
 void mlp_sync_bf16(Ctx &c);
 void grf_kappa(Ctx &c, int nmodes, const double *omega, const double *phase, double amp);
 
