@@ -1210,8 +1210,9 @@ double fsai_train_step(Ctx &c, int nprobes, uint64_t seed, float lr) {
                      c.adam_m.get(), c.adam_v.get(), c.params_bf16.get());
   GH_CHECK_HIP(hipGetLastError());
   double lp[kResidualBlocks];
-  GH_CHECK_HIP(hipMemcpyAsync(lp, c.lpart.get(), sizeof(lp), hipMemcpyDeviceToHost, s));
-  GH_CHECK_HIP(hipStreamSynchronize(s));
+  HostCopy copy(c);
+  copy.down(lp, c.lpart.get(), sizeof(lp));
+  copy.finish();
   double loss = 0.0;
   for (int b = 0; b < kResidualBlocks; ++b) loss += lp[b];
   return loss / ((double)nprobes * (double)std::max<int64_t>(n, 1));

@@ -249,10 +249,10 @@ int gh_mesh_upload(gh_ctx *ctx, int dim, int64_t nnodes, const double *xyz, int6
     c.nv = nv;
     c.xyz.resize(size_t(nnodes) * dim);
     c.cell_nodes.resize(cn.size());
-    GH_CHECK_HIP(hipMemcpy(c.xyz.get(), xyz, sizeof(double) * nnodes * dim,
-                           hipMemcpyHostToDevice));
-    GH_CHECK_HIP(hipMemcpy(c.cell_nodes.get(), cn.data(), sizeof(int32_t) * cn.size(),
-                           hipMemcpyHostToDevice));
+    gh::HostCopy copy(c);
+    copy.up(c.xyz, xyz, (size_t)nnodes * dim);
+    copy.up(c.cell_nodes, cn.data(), cn.size());
+    copy.finish();
     invalidate_space(c);
     invalidate_pattern(c);
   });
@@ -292,8 +292,9 @@ int gh_space_upload(gh_ctx *ctx, int reffe_kind, int order, int ncomp, const int
     c.nfree = nfree;
     c.ndiri = ndiri;
     c.cell_dofs.resize(cd.size());
-    GH_CHECK_HIP(hipMemcpy(c.cell_dofs.get(), cd.data(), sizeof(int32_t) * cd.size(),
-                           hipMemcpyHostToDevice));
+    gh::HostCopy copy(c);
+    copy.up(c.cell_dofs, cd.data(), cd.size());
+    copy.finish();
     c.h_cell_dofs.swap(cd);
     c.have_space = true;
     c.have_trial = false;  // a new test space ends the previous rectangular pair
@@ -346,8 +347,9 @@ int gh_trial_space_upload(gh_ctx *ctx, int reffe_kind, int order, int ncomp,
     c.tnfree = nfree;
     c.tndiri = ndiri;
     c.tcell_dofs.resize(cd.size());
-    GH_CHECK_HIP(hipMemcpy(c.tcell_dofs.get(), cd.data(), sizeof(int32_t) * cd.size(),
-                           hipMemcpyHostToDevice));
+    gh::HostCopy copy(c);
+    copy.up(c.tcell_dofs, cd.data(), cd.size());
+    copy.finish();
     c.tshp.clear();
     c.tgrad.clear();
     c.tnq = 0;
@@ -464,20 +466,20 @@ int gh_boundary_upload(gh_ctx *ctx, int64_t nfaces, const int32_t *face_cells,
     }
     c.bface_cell.resize(nfaces);
     c.bface_side.resize(nfaces);
-    GH_CHECK_HIP(hipMemcpy(c.bface_cell.get(), fc.data(), sizeof(int32_t) * nfaces,
-                           hipMemcpyHostToDevice));
-    GH_CHECK_HIP(hipMemcpy(c.bface_side.get(), fs.data(), sizeof(int32_t) * nfaces,
-                           hipMemcpyHostToDevice));
+    gh::HostCopy copy(c);
+    copy.up(c.bface_cell, fc.data(), fc.size());
+    copy.up(c.bface_side, fs.data(), fs.size());
     auto up = [&](gh::DBuf<double> &buf, bool &flag, const double *src, size_t n) {
       flag = src != nullptr;
       if (!flag) return;
       buf.resize(n);
-      GH_CHECK_HIP(hipMemcpy(buf.get(), src, sizeof(double) * n, hipMemcpyHostToDevice));
+      copy.up(buf, src, n);
     };
     up(c.balpha, c.have_balpha, alpha, nfaces);
     up(c.bbeta, c.have_bbeta, beta, nfaces);
     up(c.bg, c.have_bg, gq, (size_t)nfaces * c.nqf * c.ncomp);
     up(c.bh, c.have_bh, hq, (size_t)nfaces * c.nqf * c.ncomp);
+    copy.finish();
     c.h_face_cell.swap(fc);
     c.nbfaces = nfaces;
   });
@@ -509,17 +511,10 @@ int gh_symbolic(gh_ctx *ctx, int64_t *nnz_out) {
 int gh_pattern_get(gh_ctx *ctx, int64_t *colptr, int64_t *rowval) {
   return guarded(ctx, [&](gh::Ctx &c) {
     GH_REQUIRE(c.have_pattern, GH_ERR_STATE, "no pattern: call gh_symbolic first");
-    std::vector<int32_t> cp((c.have_trial ? c.tnfree : c.nfree) + 1), rv(c.nnz);
-    GH_CHECK_HIP(hipMemcpyAsync(cp.data(), c.colptr.get(), sizeof(int32_t) * cp.size(),
-                                hipMemcpyDeviceToHost, c.stream));
-    if (c.nnz)
-      GH_CHECK_HIP(hipMemcpyAsync(rv.data(), c.rowval.get(), sizeof(int32_t) * rv.size(),
-                                  hipMemcpyDeviceToHost, c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
-    if (colptr)
-      for (size_t k = 0; k < cp.size(); ++k) colptr[k] = int64_t(cp[k]) + 1;
-    if (rowval)
-      for (size_t k = 0; k < rv.size(); ++k) rowval[k] = int64_t(rv[k]) + 1;
+    gh::HostCopy copy(c);
+    if (colptr) copy.down_ids(colptr, c.colptr.get(), (c.have_trial ? c.tnfree : c.nfree) + 1);
+    if (rowval) copy.down_ids(rowval, c.rowval.get(), c.nnz);
+    copy.finish();
   });
 }
 
@@ -527,18 +522,18 @@ int gh_coef_upload(gh_ctx *ctx, const double *kappa, const double *fsrc,
                    const double *dirichlet_vals) {
   return guarded(ctx, [&](gh::Ctx &c) {
     GH_REQUIRE(c.have_space, GH_ERR_STATE, "upload the FE space before coefficients");
+    gh::HostCopy copy(c);
     auto up = [&](gh::DBuf<double> &buf, bool &flag, const double *src, int64_t n) {
       flag = src != nullptr && n > 0;
       if (!flag) return;
       buf.resize(n);
-      GH_CHECK_HIP(hipMemcpyAsync(buf.get(), src, sizeof(double) * n, hipMemcpyHostToDevice,
-                                  c.stream));
+      copy.up(buf, src, n);
     };
     up(c.kappa, c.have_kappa, kappa, c.ncells);
     up(c.fsrc, c.have_fsrc, fsrc, c.ncells);
     // Dirichlet values of the trial space (the test space's own for a square pair)
     up(c.dvals, c.have_dvals, dirichlet_vals, c.have_trial ? c.tndiri : c.ndiri);
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.finish();
   });
 }
 
@@ -554,9 +549,9 @@ int gh_mass_upload(gh_ctx *ctx, const double *sigma) {
     GH_REQUIRE(c.reffe_kind == GH_REFFE_QK && c.ncomp == 1 && (c.order == 1 || c.order == 2),
                GH_ERR_UNSUPPORTED, "the cell mass term is provided for scalar Q1 and Q2 spaces");
     c.sigma.resize(c.ncells);
-    GH_CHECK_HIP(hipMemcpyAsync(c.sigma.get(), sigma, sizeof(double) * c.ncells,
-                                hipMemcpyHostToDevice, c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    gh::HostCopy copy(c);
+    copy.up(c.sigma, sigma, c.ncells);
+    copy.finish();
   });
 }
 
@@ -580,7 +575,9 @@ int gh_source_qp_upload(gh_ctx *ctx, const double *fq) {
                "vector spaces of the general n-cube path (fq[(cell*nq + q)*ncomp + i])");
     const size_t n = (size_t)c.ncells * c.nq * c.ncomp;
     c.fq.resize(n);
-    GH_CHECK_HIP(hipMemcpy(c.fq.get(), fq, sizeof(double) * n, hipMemcpyHostToDevice));
+    gh::HostCopy copy(c);
+    copy.up(c.fq, fq, n);
+    copy.finish();
   });
 }
 
@@ -656,16 +653,14 @@ int gh_fefunction_upload(gh_ctx *ctx, const double *free_vals, const double *dir
     GH_REQUIRE(c.have_space, GH_ERR_STATE, "upload the FE space first");
     GH_REQUIRE(free_vals || c.nfree == 0, GH_ERR_ARG, "NULL free values");
     c.ustate.resize(std::max<int64_t>(c.nfree, 1));
-    if (c.nfree)
-      GH_CHECK_HIP(hipMemcpyAsync(c.ustate.get(), free_vals, sizeof(double) * c.nfree,
-                                  hipMemcpyHostToDevice, c.stream));
+    gh::HostCopy copy(c);
+    copy.up(c.ustate, free_vals, c.nfree);
     c.have_dvals = dirichlet_vals != nullptr && c.ndiri > 0;
     if (c.have_dvals) {
       c.dvals.resize(c.ndiri);
-      GH_CHECK_HIP(hipMemcpyAsync(c.dvals.get(), dirichlet_vals, sizeof(double) * c.ndiri,
-                                  hipMemcpyHostToDevice, c.stream));
+      copy.up(c.dvals, dirichlet_vals, c.ndiri);
     }
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.finish();
     c.have_state = true;
   });
 }
@@ -680,13 +675,10 @@ int gh_plaplacian_params(gh_ctx *ctx, double p) {
 int gh_values_get(gh_ctx *ctx, double *nzval, double *b) {
   return guarded(ctx, [&](gh::Ctx &c) {
     GH_REQUIRE(c.have_values, GH_ERR_STATE, "no assembled values: call gh_assemble first");
-    if (nzval && c.nnz)
-      GH_CHECK_HIP(hipMemcpyAsync(nzval, c.nzval.get(), sizeof(double) * c.nnz,
-                                  hipMemcpyDeviceToHost, c.stream));
-    if (b && c.nfree)
-      GH_CHECK_HIP(hipMemcpyAsync(b, c.b.get(), sizeof(double) * c.nfree,
-                                  hipMemcpyDeviceToHost, c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    gh::HostCopy copy(c);
+    if (nzval) copy.down(nzval, c.nzval.get(), sizeof(double) * c.nnz);
+    if (b) copy.down(b, c.b.get(), sizeof(double) * c.nfree);
+    copy.finish();
   });
 }
 
@@ -716,16 +708,15 @@ int gh_compose_block(gh_ctx *ctx, gh_ctx *src, const int64_t *dst, int64_t n, in
     blk->src = &src->c;
     blk->n = n;
     blk->dst.resize((size_t)n);
-    if (n)
-      GH_CHECK_HIP(hipMemcpyAsync(blk->dst.get(), d.data(), sizeof(int32_t) * n,
-                                  hipMemcpyHostToDevice, c.stream));
+    gh::HostCopy copy(c);
+    copy.up(blk->dst, d.data(), (size_t)n);
     if (c.comp_nnz < 0) {
       // positions no block covers read as stored zeros
       c.comp_nz.resize((size_t)nnz);
       if (nnz)
         GH_CHECK_HIP(hipMemsetAsync(c.comp_nz.get(), 0, sizeof(double) * nnz, c.stream));
     }
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.finish();
     c.comp.push_back(std::move(blk));
     c.comp_taken.swap(taken);
     c.comp_nnz = nnz;
@@ -741,10 +732,9 @@ int gh_compose_values_get(gh_ctx *ctx, double *nzval) {
     GH_REQUIRE(c.comp_nnz >= 0, GH_ERR_STATE, "no composite blocks: call gh_compose_block");
     GH_REQUIRE(nzval || c.comp_nnz == 0, GH_ERR_ARG, "NULL nzval");
     for (const auto &blk : c.comp) GH_CHECK_HIP(hipStreamSynchronize(blk->src->stream));
-    if (c.comp_nnz)
-      GH_CHECK_HIP(hipMemcpyAsync(nzval, c.comp_nz.get(), sizeof(double) * c.comp_nnz,
-                                  hipMemcpyDeviceToHost, c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    gh::HostCopy copy(c);
+    copy.down(nzval, c.comp_nz.get(), sizeof(double) * c.comp_nnz);
+    copy.finish();
   });
 }
 
@@ -762,13 +752,10 @@ int gh_values_set(gh_ctx *ctx, const double *nzval, const double *b) {
     GH_REQUIRE(c.have_pattern, GH_ERR_STATE, "no pattern: call gh_symbolic first");
     GH_REQUIRE(nzval || c.have_values, GH_ERR_STATE,
                "no matrix on the device: pass nzval or assemble first");
-    if (nzval && c.nnz)
-      GH_CHECK_HIP(hipMemcpyAsync(c.nzval.get(), nzval, sizeof(double) * c.nnz,
-                                  hipMemcpyHostToDevice, c.stream));
-    if (b && c.nfree)
-      GH_CHECK_HIP(hipMemcpyAsync(c.b.get(), b, sizeof(double) * c.nfree,
-                                  hipMemcpyHostToDevice, c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    gh::HostCopy copy(c);
+    if (nzval) copy.up(c.nzval, nzval, c.nnz);
+    if (b) copy.up(c.b, b, c.nfree);
+    copy.finish();
     c.have_values = true;
     if (nzval) c.fsai_built = false;
   });
@@ -809,12 +796,11 @@ int gh_spmv(gh_ctx *ctx, const double *x, double *y) {
     GH_REQUIRE(x && y, GH_ERR_ARG, "NULL vector");
     c.s_x.resize(c.nfree);
     c.s_q.resize(c.nfree);
-    GH_CHECK_HIP(hipMemcpyAsync(c.s_x.get(), x, sizeof(double) * c.nfree,
-                                hipMemcpyHostToDevice, c.stream));
+    gh::HostCopy copy(c);
+    copy.up(c.s_x, x, c.nfree);
     gh::spmv_device(c, c.s_x.get(), c.s_q.get());
-    GH_CHECK_HIP(hipMemcpyAsync(y, c.s_q.get(), sizeof(double) * c.nfree,
-                                hipMemcpyDeviceToHost, c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.down(y, c.s_q.get(), sizeof(double) * c.nfree);
+    copy.finish();
   });
 }
 
@@ -831,11 +817,10 @@ int gh_pcg(gh_ctx *ctx, int precond, const double *b, double *x, double rtol, in
     size_t n = c.nfree;
     c.s_x.resize(std::max<size_t>(n, 1));
     c.s_b.resize(std::max<size_t>(n, 1));
-    GH_CHECK_HIP(hipMemcpyAsync(c.s_x.get(), x, sizeof(double) * n, hipMemcpyHostToDevice,
-                                c.stream));
+    gh::HostCopy copy(c);
+    copy.up(c.s_x, x, n);
     if (b)
-      GH_CHECK_HIP(hipMemcpyAsync(c.s_b.get(), b, sizeof(double) * n, hipMemcpyHostToDevice,
-                                  c.stream));
+      copy.up(c.s_b, b, n);
     else
       GH_CHECK_HIP(hipMemcpyAsync(c.s_b.get(), c.b.get(), sizeof(double) * n,
                                   hipMemcpyDeviceToDevice, c.stream));
@@ -848,16 +833,14 @@ int gh_pcg(gh_ctx *ctx, int precond, const double *b, double *x, double rtol, in
       // preconditioner; the reported time covers both attempts.
       const double first_ms = local.device_ms;
       const int first_it = local.iterations;
-      GH_CHECK_HIP(hipMemcpyAsync(c.s_x.get(), x, sizeof(double) * n, hipMemcpyHostToDevice,
-                                  c.stream));
+      copy.up(c.s_x, x, n);
       gh::pcg_device(c, GH_PRECOND_JACOBI, rtol, maxit, &local);
       local.precond_used = GH_PRECOND_JACOBI;
       local.device_ms += first_ms;
       local.iterations += first_it;
     }
-    GH_CHECK_HIP(hipMemcpyAsync(x, c.s_x.get(), sizeof(double) * n, hipMemcpyDeviceToHost,
-                                c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.down(x, c.s_x.get(), sizeof(double) * n);
+    copy.finish();
     if (stats) *stats = local;
     if (!local.converged)
       throw gh::Error(GH_ERR_NOCONV, "PCG did not reach the requested tolerance");
@@ -938,11 +921,11 @@ int gh_mlp_set(gh_ctx *ctx, const float *params, int64_t n) {
     for (int64_t k = 0; k < n; ++k)
       GH_REQUIRE(std::isfinite(params[k]), GH_ERR_ARG, "non-finite network weight");
     mlp_alloc(c);
-    GH_CHECK_HIP(hipMemcpyAsync(c.params.get(), params, sizeof(float) * n, hipMemcpyHostToDevice,
-                                c.stream));
+    gh::HostCopy copy(c);
+    copy.up(c.params, params, n);
     mlp_reset_optimizer(c);
     gh::mlp_sync_bf16(c);
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.finish();
     c.have_mlp = true;
     c.fsai_built = false;
   });
@@ -952,9 +935,9 @@ int gh_mlp_get(gh_ctx *ctx, float *params, int64_t n) {
   return guarded(ctx, [&](gh::Ctx &c) {
     GH_REQUIRE(c.have_mlp, GH_ERR_STATE, "no network weights");
     GH_REQUIRE(params && n == gh::kMlpParams, GH_ERR_ARG, "expected gh_mlp_nparams() weights");
-    GH_CHECK_HIP(hipMemcpyAsync(params, c.params.get(), sizeof(float) * n, hipMemcpyDeviceToHost,
-                                c.stream));
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    gh::HostCopy copy(c);
+    copy.down(params, c.params.get(), sizeof(float) * n);
+    copy.finish();
   });
 }
 
@@ -990,8 +973,9 @@ int gh_fsai_train_step(gh_ctx *ctx, int nprobes, uint64_t seed, float lr, double
 int gh_fsai_get(gh_ctx *ctx, float *feat, float *yout, float *gl, float *gu, float *grad) {
   return guarded(ctx, [&](gh::Ctx &c) {
     GH_REQUIRE(c.fsai_ready && c.have_mlp, GH_ERR_STATE, "no FSAI state: build or train first");
+    gh::HostCopy copy(c);
     auto cp = [&](void *dst, const void *src, size_t bytes) {
-      if (dst) GH_CHECK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
+      if (dst) copy.down(dst, src, bytes);
     };
     const size_t C = (size_t)c.ncells;
     std::vector<float> yt(yout ? C * gh::kMlpOut : 0);
@@ -1000,7 +984,7 @@ int gh_fsai_get(gh_ctx *ctx, float *feat, float *yout, float *gl, float *gu, flo
     cp(gl, c.gl.get(), sizeof(float) * c.nnz);
     cp(gu, c.gu.get(), sizeof(float) * c.nnz);
     cp(grad, c.grads.get(), sizeof(float) * gh::kMlpParams);
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.finish();
     if (yout)  // device layout is output-major; hand back cells x kMlpOutPad
       for (size_t cell = 0; cell < C; ++cell)
         for (int n = 0; n < gh::kMlpOutPad; ++n)
@@ -1012,14 +996,15 @@ int gh_fsai_factor_get(gh_ctx *ctx, float *gle, int32_t *gli, float *gue, int32_
   return guarded(ctx, [&](gh::Ctx &c) {
     GH_REQUIRE(c.fsai_built, GH_ERR_STATE, "no FSAI factor: call gh_fsai_build");
     const size_t n = (size_t)c.nfree * gh::kFsaiEllSlots;
+    gh::HostCopy copy(c);
     auto cp = [&](void *dst, const void *src, size_t bytes) {
-      if (dst) GH_CHECK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
+      if (dst) copy.down(dst, src, bytes);
     };
     cp(gle, c.gle.get(), sizeof(float) * n);
     cp(gli, c.gli.get(), sizeof(int32_t) * n);
     cp(gue, c.gue.get(), sizeof(float) * n);
     cp(gui, c.gui.get(), sizeof(int32_t) * n);
-    GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+    copy.finish();
   });
 }
 

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <stdexcept>
 #include <string>
 #include <memory>
@@ -108,7 +109,7 @@ __host__ __device__ inline double det_inv(const double *J, double *Ji) {
   }
 }
 
-// Pinned host memory (small read-backs of the symbolic phase).
+// Pinned host memory (small read-backs).
 template <class T>
 struct HBuf {
   T *p = nullptr;
@@ -131,10 +132,31 @@ struct HBuf {
   }
 };
 
+// Timing events and the events of the staged host copies, created at their first use.
+struct Events {
+  static constexpr int kCopy = 4, kAll = kCopy + 2;
+  hipEvent_t e[kAll] = {};
+  Events() = default;
+  Events(const Events &) = delete;
+  Events &operator=(const Events &) = delete;
+  ~Events() {
+    for (hipEvent_t v : e)
+      if (v) (void)hipEventDestroy(v);
+  }
+  hipEvent_t *get(int first, int n, unsigned flags) {
+    for (int k = first; k < first + n; ++k)
+      if (!e[k]) GH_CHECK_HIP(hipEventCreateWithFlags(&e[k], flags));
+    return e + first;
+  }
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
+  Events events;
+  hipEvent_t *copy_events() { return events.get(0, Events::kCopy, hipEventDisableTiming); }
+  hipEvent_t *timing_events() { return events.get(Events::kCopy, 2, hipEventDefault); }
   // workspace of the lattice symbolic phase, kept between calls (it is rebuilt for
   // every pattern, so reusing it saves the allocations, not any result)
   DBuf<int32_t> ws_f, ws_scan, ws_count, ws_start, ws_flag;
@@ -320,6 +342,37 @@ struct Ctx {
   DBuf<uint8_t> psign;                        // signs of a batch of probes
   int adam_t = 0;
   bool have_mlp = false;
+};
+
+// hostcopy.hip: copies between pageable host arrays and the device through pinned staging,
+// ordered on the context's stream.  up returns with the host array read (the device copy
+// is enqueued), down with the host array written.  finish waits for the stream; a HostCopy
+// that ends without it waits before its staging is reused.
+class HostCopy {
+ public:
+  explicit HostCopy(Ctx &c);
+  ~HostCopy();
+  HostCopy(const HostCopy &) = delete;
+  HostCopy &operator=(const HostCopy &) = delete;
+  void up(void *dev, const void *host, size_t bytes);
+  void down(void *host, const void *dev, size_t bytes);
+  // 0-based 32-bit ids on the device to 1-based 64-bit ids on the host
+  void down_ids(int64_t *host, const int32_t *dev, size_t count);
+  void finish();
+  template <class T>
+  void up(DBuf<T> &dev, const T *host, size_t count) {
+    up(dev.get(), host, sizeof(T) * count);
+  }
+
+ private:
+  void wait_slot(int k);
+  void down_chunks(const void *dev, size_t bytes, size_t unit,
+                   const std::function<void(const char *, size_t, size_t)> &take);
+  hipStream_t s_;
+  hipEvent_t *ev_ = nullptr;
+  char *buf_ = nullptr;
+  bool used_[Events::kCopy] = {}, busy_ = false;
+  int next_ = 0;
 };
 
 // pattern.hip

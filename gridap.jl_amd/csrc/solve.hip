@@ -912,10 +912,11 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   // included
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (timed) {
-    GH_CHECK_HIP(hipEventCreate(&e0));
-    GH_CHECK_HIP(hipEventCreate(&e1));
+    e0 = c.timing_events()[0];
+    e1 = c.timing_events()[1];
     GH_CHECK_HIP(hipEventRecord(e0, s));
   }
+  HostCopy copy(c);
   double *dinv = nullptr;
   const int factored = precond == GH_PRECOND_FSAI;
   // box lattice: stencil kernels (A as 14 offset arrays, G as 14), one thread per row
@@ -1012,11 +1013,8 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
                          c.gue.get(), c.gui.get(), V.y, rbuf[0], zpbuf[0], scal, part_rz);
     }
     GH_CHECK_HIP(hipGetLastError());
-    GH_CHECK_HIP(hipMemcpyAsync(hrr, part_rr, sizeof(double) * g_vec,
-                                hipMemcpyDeviceToHost, s));
-    GH_CHECK_HIP(hipMemcpyAsync(hbb, part_bb, sizeof(double) * g_vec,
-                                hipMemcpyDeviceToHost, s));
-    GH_CHECK_HIP(hipStreamSynchronize(s));
+    copy.down(hrr, part_rr, sizeof(double) * g_vec);
+    copy.down(hbb, part_bb, sizeof(double) * g_vec);
     const double bb = host_sum(hbb, (int)g_vec);
     bnorm = std::sqrt(bb) > 0 ? std::sqrt(bb) : 1.0;
     relres = std::sqrt(host_sum(hrr, (int)g_vec)) / bnorm;
@@ -1072,8 +1070,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
       }
       GH_CHECK_HIP(hipGetLastError());
       double st2[2] = {0.0, 0.0};
-      GH_CHECK_HIP(hipMemcpyAsync(st2, scal + kStop, sizeof(st2), hipMemcpyDeviceToHost, s));
-      GH_CHECK_HIP(hipStreamSynchronize(s));
+      copy.down(st2, scal + kStop, sizeof(st2));
       if (st2[0] != 0.0) {
         it = (int)st2[1];  // iterations completed before the stop
         stopped = true;
@@ -1089,8 +1086,6 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
     GH_CHECK_HIP(hipEventRecord(e1, s));
     GH_CHECK_HIP(hipEventSynchronize(e1));
     GH_CHECK_HIP(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
   } else {
     GH_CHECK_HIP(hipStreamSynchronize(s));
   }
@@ -1170,15 +1165,16 @@ void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, i
                   nullptr, base + 4 * L, part, part + 4 * (size_t)kMaxParts,
                   (double2 *)(base + 5 * L), (double2 *)(base + 7 * L)};
   const auto t0 = std::chrono::steady_clock::now();
-  GH_CHECK_HIP(hipMemcpyAsync(V.x, x, sizeof(double) * n, hipMemcpyHostToDevice, c.stream));
+  HostCopy copy(c);
+  copy.up(V.x, x, sizeof(double) * n);
   if (b)
-    GH_CHECK_HIP(hipMemcpyAsync(V.b, b, sizeof(double) * n, hipMemcpyHostToDevice, c.stream));
+    copy.up(V.b, b, sizeof(double) * n);
   else
     GH_CHECK_HIP(hipMemcpyAsync(V.b, c.b.get(), sizeof(double) * n, hipMemcpyDeviceToDevice,
                                 c.stream));
   pcg_run(c, V, precond, rtol, maxit, false, false, st);
-  GH_CHECK_HIP(hipMemcpyAsync(x, V.x, sizeof(double) * n, hipMemcpyDeviceToHost, c.stream));
-  GH_CHECK_HIP(hipStreamSynchronize(c.stream));
+  copy.down(x, V.x, sizeof(double) * n);
+  copy.finish();
   st->device_ms =
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   st->precond_used = precond;

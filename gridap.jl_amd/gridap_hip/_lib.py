@@ -261,8 +261,8 @@ class Context:
         return nnz.value
 
     def pattern_get(self):
-        colptr = np.zeros(self.ncols + 1, dtype=np.int64)
-        rowval = np.zeros(max(self.nnz, 1), dtype=np.int64)
+        colptr = np.empty(self.ncols + 1, dtype=np.int64)
+        rowval = np.empty(max(self.nnz, 1), dtype=np.int64)
         self.check(lib().gh_pattern_get(self.h, ptr(colptr), ptr(rowval)))
         return colptr, rowval[:self.nnz]
 
@@ -299,15 +299,15 @@ class Context:
                                   not b.flags.c_contiguous or b.shape != (self.nfree,)):
                 raise ValueError("b must be a contiguous float64 array of %d entries"
                                  % self.nfree)
-            bo = b if b is not None and self.nfree > 0 else np.zeros(max(self.nfree, 1))
+            bo = b if b is not None and self.nfree > 0 else np.empty(max(self.nfree, 1))
             self.check(lib().gh_values_get(self.h, None, ptr(bo)))
             return None, (b if b is not None else bo[:self.nfree])
         for name, a, n in (("nz", nz, self.nnz), ("b", b, self.nfree)):
             if a is not None and (not isinstance(a, np.ndarray) or a.dtype != np.float64 or
                                   not a.flags.c_contiguous or a.shape != (n,)):
                 raise ValueError("%s must be a contiguous float64 array of %d entries" % (name, n))
-        nzo = nz if nz is not None and self.nnz > 0 else np.zeros(max(self.nnz, 1))
-        bo = b if b is not None and self.nfree > 0 else np.zeros(max(self.nfree, 1))
+        nzo = nz if nz is not None and self.nnz > 0 else np.empty(max(self.nnz, 1))
+        bo = b if b is not None and self.nfree > 0 else np.empty(max(self.nfree, 1))
         self.check(lib().gh_values_get(self.h, ptr(nzo), ptr(bo)))
         return (nz if nz is not None else nzo[:self.nnz]), (b if b is not None else bo[:self.nfree])
 
@@ -379,8 +379,8 @@ class Context:
         for name, a, n in (("cell_coef", k, self.ncells), ("cell_source", f, self.ncells)):
             if a is not None and a.shape != (n,):
                 raise ValueError("%s must have one value per cell" % name)
-        nz = np.zeros(max(self.nnz, 1))
-        b = np.zeros(max(self.nfree, 1))
+        nz = np.empty(max(self.nnz, 1))
+        b = np.empty(max(self.nfree, 1))
         self.check(lib().gh_numeric(self.h, int(form), ptr(k), ptr(f), int(precision), ptr(nz),
                                     ptr(b), ptr(g)))
         return nz[:self.nnz], b[:self.nfree]
@@ -389,7 +389,7 @@ class Context:
         x = np.ascontiguousarray(x, dtype=np.float64)
         if x.shape != (self.nfree,):
             raise ValueError("x must have num_free_dofs entries")
-        y = np.zeros_like(x)
+        y = np.empty_like(x)
         self.check(lib().gh_spmv(self.h, ptr(x), ptr(y)))
         return y
 
