@@ -32,6 +32,36 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// v of the lane that DPP control C selects (0 where it selects none or the row is masked).
+template <int C, int ROWS = 0xf>
+__device__ __forceinline__ double dpp_mov(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, C, ROWS, 0xf, ROWS == 0xf);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), C, ROWS, 0xf, ROWS == 0xf);
+  return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {  // uniform
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// Sum over each row of 16 lanes, in its last lane.  Moves between lanes inside the vector
+// unit: a sum through LDS permutes is six dependent LDS round trips a value.
+__device__ __forceinline__ double row16_sum(double v) {
+  v += dpp_mov<0x111>(v);  // row_shr:1, 2, 4, 8
+  v += dpp_mov<0x112>(v);
+  v += dpp_mov<0x114>(v);
+  return v + dpp_mov<0x118>(v);
+}
+// Sum over the wave, the same in every lane (all 64 lanes active).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = row16_sum(v);
+  v += dpp_mov<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += dpp_mov<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return lane_value(v, 63);
+}
+
 // Error carried from the point of failure to the ABI boundary, where it becomes a
 // status code plus gh_last_error() text.
 struct Error : std::runtime_error {

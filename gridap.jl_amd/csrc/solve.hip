@@ -43,21 +43,30 @@ constexpr int kRz = 0;  // [0..1]: r·z, double-buffered by iteration parity
 // 2 (r·r not finite); kStopIt = the iteration at whose start it was decided
 constexpr int kStop = 5, kStopIt = 6;
 
-__device__ __forceinline__ double block_sum(double v, double *sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+// One partial per block: part[blockIdx.x] = Σ_block v, for up to four quantities with one
+// barrier (wave sums inside the vector unit, the wave sums by the first wave).
+template <int N>
+__device__ __forceinline__ void put_partials(const double (&v)[N], double *const (&part)[N]) {
+  static_assert(N <= 4 && kBlock / 64 <= 16, "a row of 16 lanes per quantity");
+  __shared__ double sums[N][16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const double s = wave_sum(v[k]);
+    if (lane == 0) sums[k][w] = s;
+  }
   __syncthreads();
-  if (lane == 0) sh[w] = v;
-  __syncthreads();
-  double r = 0.0;
-  for (int k = 0; k < (int)(blockDim.x >> 6); ++k) r += sh[k];
-  return r;
+  if (w != 0) return;
+  const int q = lane >> 4, i = lane & 15;
+  const double s = row16_sum(q < N && i < kBlock / 64 ? sums[q < N ? q : 0][i] : 0.0);
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    if (lane == 16 * k + 15) part[k][blockIdx.x] = s;
 }
-
-// One partial per block: part[blockIdx.x] = Σ_block v.
-__device__ __forceinline__ void put_partial(double v, double *part, double *sh) {
-  v = block_sum(v, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = v;
+__device__ __forceinline__ void put_partial(double v, double *part) {
+  const double a[1] = {v};
+  double *const p[1] = {part};
+  put_partials(a, p);
 }
 
 // Grids of the iteration kernels are capped at kPcgGrid blocks (grid-stride loops):
@@ -65,12 +74,6 @@ __device__ __forceinline__ void put_partial(double v, double *part, double *sh) 
 // partial count, not only the row count, sets the cost of a reduction.
 constexpr int kPcgGrid = 1024;
 static_assert(kPcgGrid <= kMaxParts, "partial slots");
-
-// Wave-wide sum (every lane gets it).
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
 
 // The loads an iteration kernel starts with, issued together: the stop flag and this
 // thread's share of one or two partial arrays.  The kernel issues its first data loads
@@ -105,20 +108,19 @@ __device__ __forceinline__ StartIn start_loads(const double *scal, const double 
 // One barrier; sh holds 2 x kBlock/64 + 1 values and is reused by later reductions.
 __device__ __forceinline__ bool start_sums(StartIn &S, double *sh) {
   constexpr int kW = kBlock / 64;
+  static_assert(kW <= 16, "a row of 16 lanes per quantity");
   const double a = wave_sum(S.a), b = wave_sum(S.b);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   if (lane == 0) {
-    sh[2 * w] = a;
-    sh[2 * w + 1] = b;
+    sh[w] = a;
+    sh[kW + w] = b;
   }
   if (threadIdx.x == 0) sh[2 * kW] = S.stop;
   __syncthreads();
-  S.a = S.b = 0.0;
-#pragma unroll
-  for (int k = 0; k < kW; ++k) {
-    S.a += sh[2 * k];
-    S.b += sh[2 * k + 1];
-  }
+  const int q = lane >> 4, i = lane & 15;
+  const double v = row16_sum(q < 2 && i < kW ? sh[kW * (q & 1) + i] : 0.0);
+  S.a = lane_value(v, 15);
+  S.b = lane_value(v, 31);
   return sh[2 * kW] != 0.0;
 }
 constexpr int kStartLds = 2 * (kBlock / 64) + 1;
@@ -255,7 +257,6 @@ __global__ __launch_bounds__(kBlock) void init_kernel(int64_t n, const double *_
                                                       double *__restrict__ part_rz,
                                                       double *__restrict__ part_rr,
                                                       double *__restrict__ part_bb) {
-  __shared__ double sh[kBlock / 64];
   double rz = 0.0, rr = 0.0, bb = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kBlock) {
@@ -270,9 +271,10 @@ __global__ __launch_bounds__(kBlock) void init_kernel(int64_t n, const double *_
     rr += ri * ri;
     bb += b[i] * b[i];
   }
-  if (!factored) put_partial(rz, part_rz, sh);
-  put_partial(rr, part_rr, sh);
-  put_partial(bb, part_bb, sh);
+  if (factored)
+    put_partials({rr, bb}, {part_rr, part_bb});
+  else
+    put_partials({rr, bb, rz}, {part_rr, part_bb, part_rz});
 }
 
 // r·z of this iteration from its partials (published to scal[rz slot] by block 0);
@@ -334,7 +336,7 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_kernel(
     t += gridDim.x;
     if (t < ntiles) open(t);
   }
-  put_partial(dot, part_pq, sh);
+  put_partial(dot, part_pq);
 }
 
 // α = r·z / p'·q; x += α p'; r -= α q; z = M r beside p' (diagonal M or none); partials
@@ -373,8 +375,7 @@ __global__ __launch_bounds__(kBlock) void update_zp_kernel(
     i += stride;
     if (i < n) load();
   }
-  put_partial(rz, part_rz, sh);
-  put_partial(rr, part_rr, sh);
+  put_partials({rz, rr}, {part_rz, part_rr});
 }
 
 // α = r·z / p'·q; x += α p'; r -= α q; z = M r (diagonal M or none); partials of
@@ -428,8 +429,7 @@ __global__ __launch_bounds__(kBlock) void update_kernel(
     x[n - 1] = xv;
     r[n - 1] = rv;
   }
-  put_partial(rz, part_rz, sh);
-  put_partial(rr, part_rr, sh);
+  put_partials({rz, rr}, {part_rz, part_rr});
 }
 
 // G and Gᵀ are 16-slot rows (kFsaiEllSlots): 4 lanes per row, 4 slots per lane, one
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(kBlock) void update_lower_kernel(
       rr += ri * ri;
     }
   }
-  put_partial(rr, part_rr, sh);
+  put_partial(rr, part_rr);
 }
 
 // y = G r (start of a solve)
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kBlock) void upper_rz_kernel(
       rz += s * r[row];
     }
   }
-  put_partial(rz, part_rz, sh);
+  put_partial(rz, part_rz);
 }
 
 // ---- box lattice: stencil kernels ---------------------------------------------------
@@ -750,7 +750,7 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_box_kernel(
       __syncthreads();  // the runs are read: the next tile's go in
     }
   }
-  put_partial(dot, part_pq, sh);
+  put_partial(dot, part_pq);
 }
 
 // stencil form of update_lower_kernel; START: y = G r only (start of a solve; rold = r)
@@ -816,7 +816,7 @@ __global__ __launch_bounds__(kBlock) void update_lower_box_kernel(
       __syncthreads();
     }
   }
-  if (!START) put_partial(rr, part_rr, sh);
+  if (!START) put_partial(rr, part_rr);
 }
 
 // z = Gᵀ y, partials of r·z; stencil form: entry (j, i) of G with j = i − off(o),
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(kBlock) void upper_rz_box_kernel(
       __syncthreads();
     }
   }
-  put_partial(rz, part_rz, sh);
+  put_partial(rz, part_rz);
 }
 
 }  // namespace
@@ -1119,9 +1119,9 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
 // ---- the solve that allocates nothing (gh_pcg_noalloc) ------------------------------
 // Its vectors live in one fixed device array, `scratch`, which every GPU the library
 // runs on holds until the process ends: x, b, r, q, D^-1 and two interleaved {z, p}, of
-// at most GH_NOALLOC_MAX_N entries each (nine vectors), then the partial sums and the scalars.  Every call on
-// one GPU shares that GPU's copy (calls that overlap on one GPU race), and nothing in
-// it is read before the call writes it.
+// at most GH_NOALLOC_MAX_N entries each (nine vectors), then the partial sums and the
+// scalars.  Every call on one GPU shares that GPU's copy (calls that overlap on one GPU
+// race), and nothing in it is read before the call writes it.
 namespace {
 constexpr size_t kNoAllocVec = (size_t)GH_NOALLOC_MAX_N;
 constexpr size_t kNoAllocVecs = 9;
