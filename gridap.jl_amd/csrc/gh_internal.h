@@ -343,6 +343,7 @@ struct Ctx {
   // ---- solver scratch ----
   DBuf<double> s_r, s_z, s_p, s_q, s_x, s_dinv, s_b, s_part, s_scal, s_y;
   DBuf<double> s_r2, s_p2;          // second buffers of r (factored M) and p
+  DBuf<unsigned char> s_small;      // workspace of the one-workgroup solve
   // box lattice: the free dofs are all nodes of a box of box_m[0] x box_m[1] x box_m[2]
   // lattice nodes, numbered in node order (Q1, every boundary node outside the box
   // Dirichlet), so A is a 27-point stencil in dof space and PCG runs the stencil
@@ -450,6 +451,13 @@ void q2lattice_assemble(Ctx &c, bool f32, bool vlap = false);
 // solve.hip
 void spmv_device(Ctx &c, const double *x, double *y);
 void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st);
+// solve_small.hip: the whole solve in one workgroup (Jacobi or no preconditioner); x, b on
+// the device, ws kSmallWs bytes there.  False: declined, x unchanged.
+constexpr int kSmallMaxN = 4096;
+constexpr int kSmallStream = 1 << 17;  // streamed entries (10 bytes each)
+constexpr size_t kSmallWs = (size_t)kSmallStream * 10 + 8 * (16 + 2 * kSmallMaxN);
+bool pcg_small(Ctx &c, int precond, double rtol, int maxit, double *x, const double *b,
+               unsigned char *ws, gh_solve_stats *st);
 // the allocation-free solve: vectors in the library's fixed device array
 void scratch_init(int device);
 void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, int maxit,

@@ -1097,7 +1097,38 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
 
 }  // namespace
 
+// Systems that the one-workgroup solve takes: at most 4096 rows, 49,152 entries and 64
+// entries a row on average.  Past the entries one compute unit streams too much of the
+// matrix (µs an iteration, one workgroup and general kernels: 3-D Q1 39,304 entries 7.5 and
+// 16.2, 50,653 14.6 and 16.3, 64,000 15.6 and 15.2); with longer rows a thread's serial
+// share is too long (3-D Q2 of 41 a row 9.8 and 14.2; vector Q2 of 110 a row and 38,124
+// entries 11.5 and 10.0).  GRIDAP_HIP_SMALL_PCG=0 switches it off, and so does choosing
+// between the other forms (GRIDAP_HIP_STENCIL_PCG).
+constexpr int64_t kSmallMaxNnz = 49152, kSmallMaxRow = 64;
+bool small_system(const Ctx &c, int precond) {
+  const char *off = std::getenv("GRIDAP_HIP_SMALL_PCG");
+  return (precond == GH_PRECOND_NONE || precond == GH_PRECOND_JACOBI) && c.nfree > 0 &&
+         c.nfree <= kSmallMaxN && c.nnz <= kSmallMaxNnz &&
+         c.nnz <= kSmallMaxRow * c.nfree && !(off && off[0] == '0') &&
+         !std::getenv("GRIDAP_HIP_STENCIL_PCG");
+}
+
 void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st) {
+  if (small_system(c, precond)) {
+    c.s_small.resize(kSmallWs);
+    hipEvent_t *ev = c.timing_events();
+    GH_CHECK_HIP(hipEventRecord(ev[0], c.stream));
+    const bool done = pcg_small(c, precond, rtol, maxit, c.s_x.get(), c.s_b.get(),
+                                c.s_small.get(), st);
+    if (done) {
+      float ms = 0.f;
+      GH_CHECK_HIP(hipEventRecord(ev[1], c.stream));
+      GH_CHECK_HIP(hipEventSynchronize(ev[1]));
+      GH_CHECK_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
+      st->device_ms = ms;
+      return;
+    }
+  }
   const size_t nn = (size_t)std::max<int64_t>(c.nfree, 1);
   for (auto *bf : {&c.s_r, &c.s_z, &c.s_q}) bf->resize(nn);
   // p and its second buffer, or the interleaved z and p of the CSR kernels
@@ -1172,7 +1203,11 @@ void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, i
   else
     GH_CHECK_HIP(hipMemcpyAsync(V.b, c.b.get(), sizeof(double) * n, hipMemcpyDeviceToDevice,
                                 c.stream));
-  pcg_run(c, V, precond, rtol, maxit, false, false, st);
+  // the one-workgroup solve's workspace: the two {z, p}, which it does not need
+  static_assert(kSmallWs <= 4 * kNoAllocVec * sizeof(double), "workspace");
+  if (!(small_system(c, precond) &&
+        pcg_small(c, precond, rtol, maxit, V.x, V.b, (unsigned char *)V.zp, st)))
+    pcg_run(c, V, precond, rtol, maxit, false, false, st);
   copy.down(x, V.x, sizeof(double) * n);
   copy.finish();
   st->device_ms =
