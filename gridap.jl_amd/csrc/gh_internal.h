@@ -62,6 +62,31 @@ __device__ __forceinline__ double wave_sum(double v) {
   return lane_value(v, 63);
 }
 
+// Box of the 27-point stencil solves: rows in node order, offset o = (dx+1) + 3 (dy+1) +
+// 9 (dz+1).
+struct Box {
+  int64_t n, m0, m1, m2;
+};
+
+__device__ __forceinline__ uint32_t box_valid(const Box &B, int64_t row) {
+  // bit o set when neighbour o of row i lies in the box (32-bit: N < 2^31)
+  const int i = (int)row, m0 = (int)B.m0, m1 = (int)B.m1;
+  const int x = i % m0, y = (i / m0) % m1, z = i / (m0 * m1);
+  const uint32_t vx = (x > 0 ? 1u : 0u) | 2u | (x < B.m0 - 1 ? 4u : 0u);
+  const uint32_t vy = (y > 0 ? 1u : 0u) | 2u | (y < B.m1 - 1 ? 4u : 0u);
+  const uint32_t vz = (z > 0 ? 1u : 0u) | 2u | (z < B.m2 - 1 ? 4u : 0u);
+  uint32_t m = 0;
+#pragma unroll
+  for (int o = 0; o < 27; ++o)
+    if (((vx >> (o % 3)) & 1u) && ((vy >> ((o / 3) % 3)) & 1u) && ((vz >> (o / 9)) & 1u))
+      m |= 1u << o;
+  return m;
+}
+
+__host__ __device__ __forceinline__ int64_t box_off(const Box &B, int o) {
+  return (int64_t)(o % 3 - 1) + B.m0 * ((o / 3) % 3 - 1) + B.m0 * B.m1 * (o / 9 - 1);
+}
+
 // Error carried from the point of failure to the ABI boundary, where it becomes a
 // status code plus gh_last_error() text.
 struct Error : std::runtime_error {
@@ -343,7 +368,7 @@ struct Ctx {
   // ---- solver scratch ----
   DBuf<double> s_r, s_z, s_p, s_q, s_x, s_dinv, s_b, s_part, s_scal, s_y;
   DBuf<double> s_r2, s_p2;          // second buffers of r (factored M) and p
-  DBuf<unsigned char> s_small;      // workspace of the one-workgroup solve
+  DBuf<unsigned char> s_small;      // workspace of the one-launch solves
   // box lattice: the free dofs are all nodes of a box of box_m[0] x box_m[1] x box_m[2]
   // lattice nodes, numbered in node order (Q1, every boundary node outside the box
   // Dirichlet), so A is a 27-point stencil in dof space and PCG runs the stencil
@@ -458,6 +483,14 @@ constexpr int kSmallStream = 1 << 17;  // streamed entries (10 bytes each)
 constexpr size_t kSmallWs = (size_t)kSmallStream * 10 + 8 * (16 + 2 * kSmallMaxN);
 bool pcg_small(Ctx &c, int precond, double rtol, int maxit, double *x, const double *b,
                unsigned char *ws, gh_solve_stats *st);
+// solve_resident.hip: the whole solve of a box system in one launch of workgroups that stay
+// on their compute units.  state: r, p, z of a solve that takes several launches; pub 2n
+// and ws kResidentWs bytes.  False: not taken (st untouched), x a valid initial guess.
+constexpr size_t kResidentWs = 32768;
+bool resident_system(const Ctx &c, const Box &B, int precond);
+bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, double *x,
+                  const double *b, double *const (&state)[3], double *pub, unsigned char *ws,
+                  gh_solve_stats *st);
 // the allocation-free solve: vectors in the library's fixed device array
 void scratch_init(int device);
 void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, int maxit,

@@ -530,29 +530,6 @@ __global__ __launch_bounds__(kBlock) void upper_rz_kernel(
 // at offset 26 − o.  G is g14[o·N + i] for o ≤ 13 (lower offsets); Gᵀ row i collects
 // g14[o·N + i − off(o)] from the mirrored neighbours.
 
-struct Box {
-  int64_t n, m0, m1, m2;
-};
-
-__device__ __forceinline__ uint32_t box_valid(const Box &B, int64_t row) {
-  // bit o set when neighbour o of row i lies in the box (32-bit: N < 2^31)
-  const int i = (int)row, m0 = (int)B.m0, m1 = (int)B.m1;
-  const int x = i % m0, y = (i / m0) % m1, z = i / (m0 * m1);
-  const uint32_t vx = (x > 0 ? 1u : 0u) | 2u | (x < B.m0 - 1 ? 4u : 0u);
-  const uint32_t vy = (y > 0 ? 1u : 0u) | 2u | (y < B.m1 - 1 ? 4u : 0u);
-  const uint32_t vz = (z > 0 ? 1u : 0u) | 2u | (z < B.m2 - 1 ? 4u : 0u);
-  uint32_t m = 0;
-#pragma unroll
-  for (int o = 0; o < 27; ++o)
-    if (((vx >> (o % 3)) & 1u) && ((vy >> ((o / 3) % 3)) & 1u) && ((vz >> (o / 9)) & 1u))
-      m |= 1u << o;
-  return m;
-}
-
-__host__ __device__ __forceinline__ int64_t box_off(const Box &B, int o) {
-  return (int64_t)(o % 3 - 1) + B.m0 * ((o / 3) % 3 - 1) + B.m0 * B.m1 * (o / 9 - 1);
-}
-
 // a27 (lower half, o ≤ 13) from the CSR rows of the box-lattice matrix.  A lattice
 // row holds exactly the neighbours that lie in the box, in ascending column order (the
 // symbolic phase has verified the pattern), which is ascending offset order: the
@@ -1114,21 +1091,23 @@ bool small_system(const Ctx &c, int precond) {
 }
 
 void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st) {
-  if (small_system(c, precond)) {
-    c.s_small.resize(kSmallWs);
+  // a solve in one launch, timed like the general one; false: not taken
+  auto timed = [&](auto &&solve) {
+    float ms = 0.f;
     hipEvent_t *ev = c.timing_events();
     GH_CHECK_HIP(hipEventRecord(ev[0], c.stream));
-    const bool done = pcg_small(c, precond, rtol, maxit, c.s_x.get(), c.s_b.get(),
-                                c.s_small.get(), st);
-    if (done) {
-      float ms = 0.f;
-      GH_CHECK_HIP(hipEventRecord(ev[1], c.stream));
-      GH_CHECK_HIP(hipEventSynchronize(ev[1]));
-      GH_CHECK_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
-      st->device_ms = ms;
-      return;
-    }
-  }
+    if (!solve()) return false;
+    GH_CHECK_HIP(hipEventRecord(ev[1], c.stream));
+    GH_CHECK_HIP(hipEventSynchronize(ev[1]));
+    GH_CHECK_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
+    st->device_ms = ms;
+    return true;
+  };
+  c.s_small.resize(std::max(kSmallWs, kResidentWs));
+  if (small_system(c, precond) && timed([&] {
+        return pcg_small(c, precond, rtol, maxit, c.s_x.get(), c.s_b.get(), c.s_small.get(), st);
+      }))
+    return;
   const size_t nn = (size_t)std::max<int64_t>(c.nfree, 1);
   for (auto *bf : {&c.s_r, &c.s_z, &c.s_q}) bf->resize(nn);
   // p and its second buffer, or the interleaved z and p of the CSR kernels
@@ -1144,6 +1123,13 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
                   c.s_p.get(), c.s_p2.get(), c.s_q.get(), c.s_y.get(), c.s_dinv.get(),
                   c.s_part.get(), c.s_scal.get(), (double2 *)c.s_p.get(),
                   (double2 *)c.s_p2.get()};
+  const Box B{c.nfree, c.box_m[0], c.box_m[1], c.box_m[2]};
+  if (c.box && resident_system(c, B, precond) &&
+      (precond != GH_PRECOND_FSAI || (c.fsai_built && c.g14.get())) && timed([&] {
+        return pcg_resident(c, B, precond, rtol, maxit, V.x, V.b, {V.r, V.p, V.z}, V.p2,
+                            c.s_small.get(), st);
+      }))
+    return;
   pcg_run(c, V, precond, rtol, maxit, true, true, st);
 }
 

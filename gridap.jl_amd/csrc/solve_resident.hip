@@ -1,0 +1,501 @@
+// PCG on a box lattice in one launch: the workgroups stay on their compute units for the
+// whole solve and keep their rows' matrix in registers.
+//
+// The two kernels of an iteration (solve.hip) read the stencil again every time, 28 MB at
+// 64³, and pay two launches.  Here a workgroup owns rb consecutive rows, one per thread, with
+// the 27 coefficients of the row in registers and x, r, z and D^-1 too (FSAI's G, 14 FP32
+// values a row, comes from L2); per iteration only the vector that the stencil multiplies crosses
+// workgroups.  It is published to memory, and every workgroup reads the runs its rows need
+// (three of rb + 2 (m0 + 1) rows) into LDS, where the direction p of the runs is kept, so
+// that z alone is exchanged: p = z + β p is formed for the neighbours' rows as well.
+//
+// Workgroups meet in exchanges: each stores its partial sums in its own slots, and every
+// workgroup polls all slots and adds them in the same order: a barrier and the dot products in one, and every workgroup takes the
+// same decisions.  Two a Jacobi iteration (p·q; r·z and r·r, with z published), four with
+// FSAI (r, y = G r and z = Gᵀ y published).  Published data and slots are relaxed
+// agent-scope atomics, which the L2s of the eight XCDs keep coherent; a workgroup's stores
+// have completed (s_waitcnt) before its slot is written.  Publications alternate between
+// two buffers: when a workgroup writes one, all have passed the exchange after its last
+// reading.
+//
+// Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.6, 31³
+// 12.1 and 7.1; FSAI 24.9 and 16.6, 18.1 and 11.2.  What bounds it: the exchanges, 4.2 µs
+// each with 245 workgroups and 2.3 with 14 (a store and a load through the fabric, and
+// the slots' lines polled by all); the neighbours' rows take 1 µs.  Hence the largest
+// workgroups that fit (512 rows at least: 31³ with 256 8.3, 512 7.1, 1024 7.3).
+//
+// Every wait ends: a workgroup that waits longer than kArrive for the first exchange (some
+// workgroups are not on the device: other work holds it) or kLost for a later one sets the
+// abort word, which every waiting workgroup polls, and the general kernels solve the
+// system.  One launch runs at most kPause iterations.
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <cstdlib>
+#include <cstring>
+
+#include "gh_internal.h"
+
+namespace gh {
+namespace {
+
+constexpr int kMaxBlocks = 256, kMaxThreads = 1024, kMinRows = 512, kMaxWords = 3;
+constexpr uint64_t kEmpty = 0xfff7a11ce5107000ull;  // a NaN that no sum is (see exchange)
+constexpr int kStageRows = 256;  // rows whose values are staged at once
+constexpr int kPause = 2048;
+constexpr size_t kMaxLds = 150 * 1024;
+constexpr uint64_t kArrive = 200000, kLost = 100000000;  // ticks of 10 ns
+constexpr int kOut = 8;
+constexpr double kNone = 0, kDone = 1, kPaused = 2;
+
+struct ResidentArgs {
+  Box B;
+  int rb, maxit, jacobi, resume;
+  double rtol;
+  const int32_t *cp;
+  const double *val, *b;
+  const float *g14;
+  double *x, *r, *p, *z, *pub;
+  // {kNone, kDone or kPaused, iterations, converged, relative residual; a paused solve's
+  //  rz, beta, threshold, restarts}
+  double *out;
+  uint32_t *abort;
+  uint64_t *slots;  // [3][kMaxWords][kMaxBlocks]
+};
+
+__device__ __forceinline__ double get(const double *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void put(double *p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The value again, unknown to the compiler: what is computed from it is computed here and
+// does not take a register from one turn of the solve to the next.
+__device__ __forceinline__ int fresh(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// One exchange: v becomes its sums over all workgroups.  False: aborted.  A slot that is not
+// written yet holds kEmpty, so that a sum and the news that it is there are one word.  Of
+// the three sets of slots, exchange num writes num % 3, and a workgroup past it empties its
+// own slots of (num + 2) % 3: all have read those (exchange num - 1), as all have written
+// num; and the emptying has completed before this workgroup writes num + 1, so whoever gets
+// past that finds no old value in them.
+template <int NS>
+__device__ __forceinline__ bool exchange(const ResidentArgs &A, uint32_t &num,
+                                         double (&v)[NS ? NS : 1]) {
+  constexpr int kW = NS ? NS : 1;
+  __shared__ double mine[3][16], all[3][kMaxBlocks / 64];
+  __shared__ int dead;
+  const int t = fresh(threadIdx.x), lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6), nb = (int)gridDim.x;
+  ++num;
+  uint64_t *slot = A.slots + (size_t)(num % 3) * kMaxWords * kMaxBlocks;
+  uint64_t *last = A.slots + (size_t)((num + 2) % 3) * kMaxWords * kMaxBlocks;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const double w = wave_sum(v[s]);
+    if (lane == 0) mine[s][wave] = w;
+  }
+  if (t == 0) dead = 0;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what this wave published is there
+  __syncthreads();
+  if (wave == 0) {
+    const int q = lane >> 4, i = lane & 15;
+    double w = 0.0;
+    if (NS) w = row16_sum(q < NS && i < (int)blockDim.x / 64 ? mine[q < NS ? q : 0][i] : 0.0);
+    uint64_t word = 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const uint64_t u = (uint64_t)__double_as_longlong(lane_value(w, 16 * s + 15));
+      if (lane == s) word = u == kEmpty ? kEmpty - 1 : u;
+    }
+    if (lane < kW)
+      __hip_atomic_store(slot + (size_t)lane * kMaxBlocks + blockIdx.x, word, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (wave < kMaxBlocks / 64) {
+    uint64_t w[kW] = {};
+    const uint64_t t0 = wall_clock64(), limit = num == 1 ? kArrive : kLost;
+    for (int spin = 0; t < nb; ++spin) {
+      bool here = true;
+#pragma unroll
+      for (int k = 0; k < kW; ++k)
+        w[k] = __hip_atomic_load(slot + (size_t)k * kMaxBlocks + t, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int k = 0; k < kW; ++k) here = here && w[k] != kEmpty;
+      if (here) break;
+      if ((spin & 15) == 15 &&
+          (wall_clock64() - t0 > limit ||
+           __hip_atomic_load(A.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        dead = 1;
+        break;
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const double sum = wave_sum(t < nb ? __longlong_as_double((long long)w[s]) : 0.0);
+      if (lane == 0) all[s][wave] = sum;
+    }
+  }
+  __syncthreads();
+  if (wave == 0 && lane < kMaxWords)
+    __hip_atomic_store(last + (size_t)lane * kMaxBlocks + blockIdx.x, kEmpty, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  if (dead) {
+    if (t == 0)
+      __hip_atomic_store(A.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+  }
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    double sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < kMaxBlocks / 64; ++k)
+      if (64 * k < nb) sum += all[s][k];
+    v[s] = lane_value(sum, 0);
+  }
+  return true;
+}
+
+// The runs of a workgroup's rows in LDS: run d holds rows i0 + (z0 + d) m0 m1 - m0 - 1 + k,
+// k < len = rb + 2 (m0 + 1); zero outside [0, n).
+struct Window {
+  int n, m0, m01, i0, rb, len;
+  __device__ __forceinline__ int at(int t, int o, int z0) const {  // row t's neighbour o
+    return (o / 9 - 1 - z0) * len + m0 + 1 + ((o / 3) % 3 - 1) * m0 + (o % 3 - 1) + t;
+  }
+  // dst = src (copy) or src + beta dst on the runs z0 .. z0 + NZ - 1; own rows: mine
+  template <int NZ>
+  __device__ __forceinline__ void refresh(double *dst, const double *src, int z0, bool copy,
+                                          double beta, double mine) const {
+    const int t = fresh(threadIdx.x), bd = blockDim.x;
+    double v[NZ][2];
+#pragma unroll
+    for (int d = 0; d < NZ; ++d) {
+      const bool own = z0 + d == 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        // the own run: only the rows before and after the workgroup's own; lanes past the
+        // end read one address together
+        const int e = min(t + u * bd, (own ? 2 * (m0 + 1) : len) - 1);
+        const int j = i0 + (z0 + d) * m01 - m0 - 1 + (own && e > m0 ? e + rb : e);
+        v[d][u] = get(src + min(max(j, 0), n - 1));
+        if (j < 0 || j >= n) v[d][u] = 0.0;
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < NZ; ++d) {
+      const bool own = z0 + d == 0;
+      double *run = dst + d * len;
+      const int count = own ? 2 * (m0 + 1) : len;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int e = t + u * bd, k = own && e > m0 ? e + rb : e;
+        if (e < count) run[k] = copy ? v[d][u] : v[d][u] + beta * run[k];
+      }
+      for (int e = t + 2 * bd; e < count; e += bd) {
+        const int k = own && e > m0 ? e + rb : e;
+        const int j = i0 + (z0 + d) * m01 - m0 - 1 + k;
+        double w = get(src + min(max(j, 0), n - 1));
+        if (j < 0 || j >= n) w = 0.0;
+        run[k] = copy ? w : w + beta * run[k];
+      }
+      if (own) run[m0 + 1 + t] = mine;
+    }
+  }
+};
+
+template <bool FACT>
+__global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const ResidentArgs A) {
+  extern __shared__ __align__(16) double lds[];
+  __shared__ int bad;
+  const int t = threadIdx.x, n = (int)A.B.n, bd = blockDim.x;
+  Window W;
+  W.n = n;
+  W.m0 = (int)A.B.m0;
+  W.m01 = (int)(A.B.m0 * A.B.m1);
+  W.i0 = (int)blockIdx.x * A.rb;
+  W.rb = A.rb;
+  W.len = A.rb + 2 * (W.m0 + 1);
+  double *run = lds, *tmp = lds + 3 * W.len;
+  const int i = W.i0 + t, ic = min(i, n - 1);
+  const bool own = i < n;
+  // coefficients: rows are runs of nzval; a lattice row holds its in-box neighbours in
+  // offset order
+  double a[27];
+  {
+    const uint32_t vm = own ? box_valid(A.B, i) : 0;
+    const int q0 = A.cp[ic], q1 = A.cp[ic + 1];
+    const bool ok = !own || q1 - q0 == __popc(vm);
+    if (t == 0) bad = 0;
+    __syncthreads();
+    if (!ok) bad = 1;
+    for (int c0 = 0; c0 < bd; c0 += kStageRows) {
+      const int r0 = min(W.i0 + c0, n), r1 = min(r0 + kStageRows, n);
+      const int p0 = A.cp[r0], count = min(A.cp[r1] - p0, kStageRows * 27);
+      __syncthreads();
+      for (int k = t; k < count; k += bd) lds[k] = A.val[p0 + k];
+      __syncthreads();
+      if (t >= c0 && t < c0 + kStageRows) {
+        int k = min(q0 - p0, kStageRows * 27 - 27);  // in bounds for other matrices too
+        if (k < 0) k = 0;
+#pragma unroll
+        for (int o = 0; o < 27; ++o) {
+          const bool in = (vm >> o) & 1u;
+          a[o] = in ? lds[k] : 0.0;
+          k += in ? 1 : 0;
+        }
+      }
+    }
+    __syncthreads();
+    if (bad) {  // not the lattice matrix: the general kernels take it
+      if (t == 0)
+        __hip_atomic_store(A.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+  }
+  const double dinv = A.jacobi && a[13] != 0.0 ? 1.0 / a[13] : 1.0;
+  uint32_t num = 0;
+  int turn = 0;
+  double *src = nullptr;  // the last publication
+  double none[1], xi = own ? A.x[i] : 0.0, ri = 0.0, zi = 0.0, pi = 0.0;
+  auto publish = [&](double v) {
+    src = A.pub + (turn ? n : 0);
+    turn ^= 1;
+    if (own) put(src + W.i0 + fresh(t), v);
+  };
+  // z = Gᵀ G r, r published; z published and its sum exchanged.  False: aborted
+  auto apply = [&](double &rz) {
+    float g[14];
+    const int t1 = fresh(t), j1 = min(W.i0 + t1, n - 1);
+#pragma unroll
+    for (int o = 0; o < 14; ++o) g[o] = A.g14[(int64_t)o * n + j1];
+    W.refresh<2>(tmp, src, -1, true, 0.0, ri);
+    __syncthreads();
+    double y = 0.0;
+#pragma unroll
+    for (int o = 0; o < 14; ++o) y += (double)g[o] * tmp[W.at(t1, o, -1)];
+    if (!own) y = 0.0;
+    publish(y);
+    if (!exchange<0>(A, num, none)) return false;
+    const int t2 = fresh(t), j2 = min(W.i0 + t2, n - 1);
+#pragma unroll
+    for (int o = 0; o < 14; ++o) g[o] = A.g14[(int64_t)o * n + j2 - box_off(A.B, o)];
+    W.refresh<2>(tmp, src, 0, true, 0.0, y);
+    __syncthreads();
+    zi = 0.0;
+#pragma unroll
+    for (int o = 13; o >= 0; --o) zi += (double)g[o] * tmp[W.at(t2, 26 - o, 0)];
+    if (!own) zi = 0.0;
+    publish(zi);
+    double v[1] = {zi * ri};
+    const bool there = exchange<1>(A, num, v);
+    rz = v[0];
+    return there;
+  };
+  int it = 0, restarts = 0, converged = 0;
+  double relres = INFINITY, rz = 0.0, thr = 0.0, beta = 0.0, how = kDone;
+  bool start = !A.resume, first = false;
+  if (start) {
+    publish(xi);
+    if (!exchange<0>(A, num, none)) return;
+  } else {
+    it = (int)A.out[1];
+    rz = A.out[4];
+    beta = A.out[5];
+    thr = A.out[6];
+    restarts = (int)A.out[7];
+    if (own) {
+      ri = A.r[i];
+      pi = A.p[i];
+      zi = A.z[i];
+    }
+    publish(pi);
+    if (!exchange<0>(A, num, none)) return;
+    W.refresh<3>(run, src, -1, true, 0.0, pi);
+    publish(zi);
+    if (!exchange<0>(A, num, none)) return;
+  }
+  const int until = A.maxit - it > kPause ? it + kPause : A.maxit;
+  // each turn multiplies by A once: a step of the recurrence, or (start) the true residual
+  for (;;) {
+    pi = start ? xi : first ? zi : zi + beta * pi;
+    W.refresh<3>(run, src, -1, start || first, beta, pi);
+    __syncthreads();
+    double q = 0.0;
+    const int t1 = fresh(t);
+#pragma unroll
+    for (int o = 0; o < 27; ++o) q += a[o] * run[W.at(t1, o, -1)];
+    if (!own) q = 0.0;
+    if (start) {
+      const double bi = own ? A.b[W.i0 + fresh(t)] : 0.0;
+      ri = bi - q;
+      zi = dinv * ri;
+      publish(FACT ? ri : zi);
+      double v[3] = {ri * ri, bi * bi, zi * ri};
+      if (!exchange<3>(A, num, v)) return;
+      const double bnorm = sqrt(v[1]) > 0 ? sqrt(v[1]) : 1.0;
+      relres = lane_value(sqrt(v[0]) / bnorm, 0);
+      converged = relres <= A.rtol;
+      if (converged || it >= A.maxit || restarts > 3) break;
+      rz = v[2];
+      if (FACT && !apply(rz)) return;
+      ++restarts;
+      thr = lane_value((A.rtol * bnorm) * (A.rtol * bnorm), 0);
+      first = true;
+      start = false;
+    } else {
+      double pq[1] = {pi * q};
+      if (!exchange<1>(A, num, pq)) return;
+      const double alpha = lane_value(rz / pq[0], 0);
+      xi += alpha * pi;
+      ri -= alpha * q;
+      zi = dinv * ri;
+      publish(FACT ? ri : zi);
+      double v[2] = {ri * ri, zi * ri};
+      if (!exchange<2>(A, num, v)) return;
+      ++it;
+      first = false;
+      // at the tolerance, not finite or at the limit: the true residual decides
+      start = !(v[0] > thr) || !isfinite(v[0]) || it >= A.maxit;
+      if (start) {
+        publish(xi);
+        if (!exchange<0>(A, num, none)) return;
+      } else {
+        if (FACT && !apply(v[1])) return;
+        beta = lane_value(v[1] / rz, 0);
+        rz = v[1];
+      }
+    }
+    if (!start && it >= until) {
+      how = kPaused;
+      if (own) {
+        const int j = W.i0 + fresh(t);
+        A.r[j] = ri;
+        A.p[j] = pi;
+        A.z[j] = zi;
+      }
+      break;
+    }
+  }
+  if (own) A.x[W.i0 + fresh(t)] = xi;
+  if (blockIdx.x == 0 && t == 0) {
+    A.out[0] = how;
+    A.out[1] = it;
+    A.out[2] = converged;
+    A.out[3] = relres;
+    A.out[4] = rz;
+    A.out[5] = beta;
+    A.out[6] = thr;
+    A.out[7] = restarts;
+  }
+}
+
+// Before each launch: no exchange has happened, nothing is aborted.
+__global__ void resident_clear_kernel(ResidentArgs A) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < 3 * kMaxWords * kMaxBlocks) A.slots[k] = kEmpty;
+  if (k == 0) *A.abort = 0;
+  if (k == 0) A.out[0] = kNone;
+}
+
+struct Shape {
+  int rb, blocks;
+  size_t lds;
+};
+Shape shape(const Box &B, int cus, bool fact) {
+  const int64_t nb = std::min(cus, kMaxBlocks);
+  const int64_t rb = std::max<int64_t>(((B.n + nb - 1) / nb + 63) / 64 * 64, kMinRows);
+  const int64_t runs = (fact ? 5 : 3) * (rb + 2 * (B.m0 + 1)) * (int64_t)sizeof(double);
+  return {(int)std::min<int64_t>(rb, INT32_MAX), (int)((B.n + rb - 1) / rb),
+          (size_t)std::max<int64_t>(runs, kStageRows * 27 * sizeof(double))};
+}
+
+int compute_units(int device) {
+  int v = 0;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+    return 0;
+  return v;
+}
+
+// One resident solve per device at a time: two that each hold a part of the device
+// would wait for each other until both give up.
+constexpr int kMaxDevices = 64;
+std::atomic<bool> g_busy[kMaxDevices];
+struct Turn {
+  std::atomic<bool> *flag = nullptr;
+  explicit Turn(int device) {
+    if (device < 0 || device >= kMaxDevices) return;
+    bool idle = false;
+    if (g_busy[device].compare_exchange_strong(idle, true)) flag = &g_busy[device];
+  }
+  ~Turn() {
+    if (flag) flag->store(false);
+  }
+};
+
+}  // namespace
+
+bool resident_system(const Ctx &c, const Box &B, int precond) {
+  const char *off = std::getenv("GRIDAP_HIP_RESIDENT_PCG");
+  if ((off && off[0] == '0') || std::getenv("GRIDAP_HIP_STENCIL_PCG")) return false;
+  const int cus = compute_units(c.device);
+  if (cus < 1 || B.n < 1) return false;
+  const Shape S = shape(B, cus, precond == GH_PRECOND_FSAI);
+  return S.rb <= kMaxThreads && S.lds <= kMaxLds;
+}
+
+bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, double *x,
+                  const double *b, double *const (&state)[3], double *pub, unsigned char *ws,
+                  gh_solve_stats *st) {
+  static_assert(sizeof(double) * (kOut + 8) + sizeof(uint64_t) * 3 * kMaxWords * kMaxBlocks <=
+                    kResidentWs, "workspace");
+  Turn turn(c.device);
+  if (!turn.flag) return false;
+  const bool fact = precond == GH_PRECOND_FSAI;
+  const Shape S = shape(B, compute_units(c.device), fact);
+  ResidentArgs A{};
+  A.B = B;
+  A.rb = S.rb;
+  A.maxit = maxit;
+  A.jacobi = precond == GH_PRECOND_JACOBI;
+  A.rtol = rtol;
+  A.cp = c.colptr.get();
+  A.val = c.nzval.get();
+  A.b = b;
+  A.g14 = fact ? c.g14.get() : nullptr;
+  A.x = x;
+  A.r = state[0];
+  A.p = state[1];
+  A.z = state[2];
+  A.pub = pub;
+  A.out = reinterpret_cast<double *>(ws);
+  A.abort = reinterpret_cast<uint32_t *>(A.out + kOut);
+  A.slots = reinterpret_cast<uint64_t *>(A.out + kOut + 8);
+  auto kern = fact ? resident_pcg_kernel<true> : resident_pcg_kernel<false>;
+  GH_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)S.lds));
+  double h[kOut + 1];
+  do {
+    hipLaunchKernelGGL(resident_clear_kernel, dim3((3 * kMaxWords * kMaxBlocks + 255) / 256),
+                       dim3(256), 0, c.stream, A);
+    hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks), dim3((unsigned)S.rb), S.lds, c.stream, A);
+    GH_CHECK_HIP(hipGetLastError());
+    HostCopy copy(c);
+    copy.down(h, A.out, sizeof(h));
+    uint32_t aborted;
+    std::memcpy(&aborted, h + kOut, sizeof(aborted));
+    if (aborted || h[0] == kNone) return false;
+    A.resume = 1;
+  } while (h[0] == kPaused);
+  st->iterations = (int)h[1];
+  st->converged = h[2] != 0.0;
+  st->rel_residual = h[3];
+  return true;
+}
+
+}  // namespace gh

@@ -1,0 +1,135 @@
+"""The solve of a box system in one launch of resident workgroups against the launched
+stencil kernels on the same system: fewer rows than a workgroup, rows at the edges of the
+workgroups (512 and 1024 rows) and of their number (256), long and short lattice rows, the
+largest system it takes and one past it, restarts, limits, a solve over several launches
+and calls from two threads at once (needs an MI355X).
+
+Both form the same products and add a row's entries in the same order; they differ in the
+grouping of the dot products only, so the iteration count agrees to one and the solutions,
+stopped at 1e-10, to 1e-10 times the condition (below 1e4 here)."""
+import os
+import threading
+
+import numpy as np
+import pytest
+
+import gridap_hip as G
+from gridap_hip import _lib
+from gridap_hip import fsai as FS
+
+pytestmark = pytest.mark.gpu
+
+PRECONDS = (_lib.GH_PRECOND_NONE, _lib.GH_PRECOND_JACOBI, _lib.GH_PRECOND_FSAI)
+
+
+@pytest.fixture(autouse=True)
+def no_small(monkeypatch):
+    monkeypatch.setenv("GRIDAP_HIP_SMALL_PCG", "0")
+
+
+def system(part, spread=1.0):
+    # cubic cells: the condition number is set by the shortest axis
+    model = G.CartesianDiscreteModel(tuple(v for n in part for v in (0, n)), part)
+    V = G.TestFESpace(model, G.ReferenceFE(G.lagrangian, G.Float64, 1),
+                      dirichlet_tags="boundary")
+    dx = G.Measure(G.Triangulation(model), 2)
+    rng = np.random.default_rng(sum(part))
+    k = G.CellField(np.exp(rng.normal(0, spread, model.num_cells())), None)
+    op = G.AffineFEOperator(lambda u, v: G.integrate(k * G.inner(G.gradient(v), G.gradient(u)), dx),
+                            lambda v: G.integrate(1.0 * v, dx), G.TrialFESpace(V), V)
+    assert op.assem.ctx.pattern_info()["box"] == 1
+    return op, op.assem.ctx
+
+
+def launched(monkeypatch, ctx, **kw):
+    with monkeypatch.context() as m:
+        m.setenv("GRIDAP_HIP_RESIDENT_PCG", "0")
+        return ctx.pcg(**kw)
+
+
+# free rows: 1, 2, 40, 512, 528, 8 long lattice rows, 16 x 15 x 1025, 64 x 64 x 63 = 258,048
+# (1024 a workgroup), 64^3 = 262,144 (the largest), 65 x 64 x 63 = 262,080, 64 x 65 x 64 past
+PARTS = [(2, 2, 2), (3, 2, 2), (2, 6, 9), (33, 17, 2), (34, 17, 2), (514, 3, 3), (1100, 4, 5),
+         (17, 16, 1026), (65, 65, 64), (65, 65, 65), (66, 65, 64), (65, 66, 65)]
+
+
+@pytest.mark.parametrize("part", PARTS)
+def test_matches_launched_kernels(part, monkeypatch):
+    print("[gpu-case] resident PCG %s" % (part,), flush=True)
+    op, ctx = system(part)
+    A, b = op.get_matrix().to_scipy(), op.get_vector()
+    x0 = np.random.default_rng(1).standard_normal(len(b))
+    FS.LearnedFSAI.load(FS.DEFAULT_WEIGHTS).attach(ctx)
+    for precond in PRECONDS:
+        kw = dict(x0=x0, precond=precond, rtol=1e-10, maxit=5000)
+        x, st = ctx.pcg(**kw)
+        y, sy = launched(monkeypatch, ctx, **kw)
+        assert st.converged and sy.converged and abs(st.iterations - sy.iterations) <= 1
+        assert np.linalg.norm(b - A @ x) <= 1.01e-10 * np.linalg.norm(b)
+        assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+        z, _ = ctx.pcg(**kw)  # the same bits every time
+        np.testing.assert_array_equal(x, z)
+
+
+def test_limits_and_exact_starts(monkeypatch):
+    print("[gpu-case] resident PCG: limits", flush=True)
+    op, ctx = system((20, 18, 17))
+    b = op.get_vector()
+    FS.LearnedFSAI.load(FS.DEFAULT_WEIGHTS).attach(ctx)
+    for precond in PRECONDS:
+        x, _ = ctx.pcg(precond=precond, rtol=1e-10)
+        for maxit in (0, 1, 5):
+            kw = dict(precond=precond, rtol=1e-10, maxit=maxit, raise_on_noconv=False)
+            got, s1 = ctx.pcg(**kw)
+            ref, s2 = launched(monkeypatch, ctx, **kw)
+            # (FSAI that ends at its limit is followed by as many Jacobi iterations)
+            assert s1.iterations == s2.iterations and not s1.converged
+            assert s1.iterations == maxit * (2 if precond == _lib.GH_PRECOND_FSAI else 1)
+            np.testing.assert_allclose(got, ref, rtol=1e-10, atol=1e-13 * abs(ref).max())
+        y, s3 = ctx.pcg(x0=x, precond=precond, rtol=1e-8)
+        assert s3.iterations == 0 and np.array_equal(x, y)
+        zero, s4 = ctx.pcg(b=np.zeros_like(b), precond=precond, rtol=1e-8)
+        assert s4.converged and s4.iterations == 0 and not zero.any()
+        # below what FP64 reaches: the restarts run out
+        _, s5 = ctx.pcg(precond=precond, rtol=1e-30, maxit=3000, raise_on_noconv=False)
+        assert not s5.converged
+    nz, _ = ctx.values_get()
+    nz[3] = np.nan
+    ctx.values_set(nz)
+    _, s6 = ctx.pcg(rtol=1e-8, maxit=50, raise_on_noconv=False)
+    assert not s6.converged
+
+
+def test_solve_over_several_launches(monkeypatch):
+    """Coefficients over many decades, no preconditioner: more iterations than one launch
+    runs (2048).  In floating point such counts move by a percent or two with the rounding
+    of the dot products (5% allowed)."""
+    print("[gpu-case] resident PCG: several launches", flush=True)
+    op, ctx = system((40, 40, 2), spread=4.0)
+    A, b = op.get_matrix().to_scipy(), op.get_vector()
+    kw = dict(rtol=1e-8, maxit=60000, precond=_lib.GH_PRECOND_NONE)
+    x, st = ctx.pcg(**kw)
+    _, sy = launched(monkeypatch, ctx, **kw)
+    assert st.converged and sy.converged
+    assert st.iterations > 2048 and abs(st.iterations - sy.iterations) <= 0.05 * sy.iterations
+    assert np.linalg.norm(b - A @ x) <= 1.01e-8 * np.linalg.norm(b)
+
+
+def test_two_threads():
+    """Two contexts solve at once: one holds the device's turn, the other takes the
+    launched kernels; both are right."""
+    print("[gpu-case] resident PCG: two threads", flush=True)
+    systems = [system((33, 30, 31)), system((40, 28, 26))]
+    refs = [ctx.pcg(rtol=1e-10)[0] for _, ctx in systems]
+    err = [None, None]
+
+    def work(k):
+        for _ in range(4):
+            x, st = systems[k][1].pcg(rtol=1e-10)
+            e = np.linalg.norm(x - refs[k]) / np.linalg.norm(refs[k])
+            err[k] = max(err[k] or 0.0, e if st.converged else np.inf)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in (0, 1)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert max(err) <= 1e-6
