@@ -1126,8 +1126,8 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
   const Box B{c.nfree, c.box_m[0], c.box_m[1], c.box_m[2]};
   if (c.box && resident_system(c, B, precond) &&
       (precond != GH_PRECOND_FSAI || (c.fsai_built && c.g14.get())) && timed([&] {
-        return pcg_resident(c, B, precond, rtol, maxit, V.x, V.b, {V.r, V.p, V.z}, V.p2,
-                            c.s_small.get(), st);
+        return pcg_resident(c, B, precond, rtol, maxit, V.x, V.b, {V.r, V.p, V.z},
+                            {V.p2, V.r2, V.y}, c.s_small.get(), st);
       }))
     return;
   pcg_run(c, V, precond, rtol, maxit, true, true, st);

@@ -10,19 +10,27 @@
 // that z alone is exchanged: p = z + β p is formed for the neighbours' rows as well.
 //
 // Workgroups meet in exchanges: each stores its partial sums in its own slots, and every
-// workgroup polls all slots and adds them in the same order: a barrier and the dot products in one, and every workgroup takes the
-// same decisions.  Two a Jacobi iteration (p·q; r·z and r·r, with z published), four with
-// FSAI (r, y = G r and z = Gᵀ y published).  Published data and slots are relaxed
-// agent-scope atomics, which the L2s of the eight XCDs keep coherent; a workgroup's stores
-// have completed (s_waitcnt) before its slot is written.  Publications alternate between
-// two buffers: when a workgroup writes one, all have passed the exchange after its last
-// reading.
+// workgroup polls all slots and adds them in the same order: a barrier and the dot products
+// in one, and every workgroup takes the same decisions.  Two an iteration: p·q, then r·z
+// with r·r.  Published data and slots are relaxed agent-scope atomics, which the L2s of
+// the eight XCDs keep coherent.
 //
-// Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.6, 31³
-// 12.1 and 7.1; FSAI 24.9 and 16.6, 18.1 and 11.2.  What bounds it: the exchanges, 4.2 µs
-// each with 245 workgroups and 2.3 with 14 (a store and a load through the fabric, and
-// the slots' lines polled by all); the neighbours' rows take 1 µs.  Hence the largest
-// workgroups that fit (512 rows at least: 31³ with 256 8.3, 512 7.1, 1024 7.3).
+// Published vectors (z; with FSAI also r and y = G r on the way to z = Gᵀ y) need no
+// barrier of their own: what is not published yet holds kEmpty, a NaN that no published
+// value is, and a reader polls until it has a value.  z alternates between two buffers.
+// With E1, E2 the exchanges of an iteration and z(k) the z published before E2(k):
+//  - past E2(k) every workgroup has read z(k-1), r(k) and y(k) (they enter what it sent to
+//    E1(k) and E2(k)), so each empties its own rows of them then;
+//  - the emptying has completed (s_waitcnt) before the workgroup sends to E1(k+1);
+//  - r, y and z(k+1) are published and read past E1(k+1): no reader finds an old value.
+// On a (re)start, where there is no E1 between, the vectors are published with a wait
+// and read past the exchange instead.
+//
+// Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.1, 31³
+// 11.9 and 6.8; FSAI 25.3 and 19.3, 17.5 and 12.4.  (Barriers for the published vectors
+// too: 10.7, 7.6, 22.6, 16.0.)  What bounds it: the trips through the fabric, 3 to 4 µs an
+// exchange or published vector with 245 workgroups, 2 with 14.  Hence the largest
+// workgroups that fit, 512 rows at least (31³ with barriers: 256 rows 8.3, 512 7.1, 1024 7.3).
 //
 // Every wait ends: a workgroup that waits longer than kArrive for the first exchange (some
 // workgroups are not on the device: other work holds it) or kLost for a later one sets the
@@ -39,8 +47,8 @@
 namespace gh {
 namespace {
 
-constexpr int kMaxBlocks = 256, kMaxThreads = 1024, kMinRows = 512, kMaxWords = 3;
-constexpr uint64_t kEmpty = 0xfff7a11ce5107000ull;  // a NaN that no sum is (see exchange)
+constexpr int kMaxBlocks = 256, kMaxThreads = 1024, kMinRows = 512, kMaxWords = 3, kSets = 4;
+constexpr uint64_t kEmpty = 0xfff7a11ce5107000ull;  // a NaN (see exchange)
 constexpr int kStageRows = 256;  // rows whose values are staged at once
 constexpr int kPause = 2048;
 constexpr size_t kMaxLds = 150 * 1024;
@@ -55,19 +63,24 @@ struct ResidentArgs {
   const int32_t *cp;
   const double *val, *b;
   const float *g14;
-  double *x, *r, *p, *z, *pub;
+  double *x, *r, *p, *z;
+  uint64_t *zpub, *rpub, *ypub;  // published z (two buffers), r and y
   // {kNone, kDone or kPaused, iterations, converged, relative residual; a paused solve's
   //  rz, beta, threshold, restarts}
   double *out;
   uint32_t *abort;
-  uint64_t *slots;  // [3][kMaxWords][kMaxBlocks]
+  uint64_t *slots;  // [kSets][kMaxWords][kMaxBlocks]
 };
 
-__device__ __forceinline__ double get(const double *p) {
+// Words that cross workgroups.
+__device__ __forceinline__ uint64_t get(const uint64_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void put(double *p, double v) {
+__device__ __forceinline__ void store(uint64_t *p, uint64_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void put(uint64_t *p, uint64_t v) {  // a value: never kEmpty
+  store(p, v == kEmpty ? v - 1 : v);
 }
 
 // The value again, unknown to the compiler: what is computed from it is computed here and
@@ -77,30 +90,53 @@ __device__ __forceinline__ int fresh(int v) {
   return v;
 }
 
-// One exchange: v becomes its sums over all workgroups.  False: aborted.  A slot that is not
-// written yet holds kEmpty, so that a sum and the news that it is there are one word.  Of
-// the three sets of slots, exchange num writes num % 3, and a workgroup past it empties its
-// own slots of (num + 2) % 3: all have read those (exchange num - 1), as all have written
-// num; and the emptying has completed before this workgroup writes num + 1, so whoever gets
-// past that finds no old value in them.
-template <int NS>
-__device__ __forceinline__ bool exchange(const ResidentArgs &A, uint32_t &num,
-                                         double (&v)[NS ? NS : 1]) {
+// State of the waits: exchanges so far, and whether one of the workgroup's was given up.
+struct Waits {
+  uint32_t num;
+  int *dead;  // LDS
+};
+// For a thread that polls: false when it is time to give up.
+__device__ __forceinline__ bool keep_on(const ResidentArgs &A, const Waits &E, int spin,
+                                        uint64_t t0, uint64_t limit) {
+  if ((spin & 15) != 15) return true;
+  if (wall_clock64() - t0 <= limit &&
+      __hip_atomic_load(A.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    return true;
+  *E.dead = 1;
+  return false;
+}
+// After a barrier: true when the workgroup gives up (and tells the others).
+__device__ __forceinline__ bool gave_up(const ResidentArgs &A, const Waits &E) {
+  if (!*E.dead) return false;
+  if (threadIdx.x == 0)
+    __hip_atomic_store(A.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// One exchange: v becomes its sums over all workgroups.  False: aborted.  FLUSH: this
+// workgroup's stores have completed before its sums are there.  during() runs between
+// sending and waiting.  A slot that is not written yet holds kEmpty, so that a sum and the
+// news that it is there are one word.  Of the four sets of slots, exchange num writes
+// num % 4, and a workgroup past it empties its own slots of (num + 3) % 4: all have read
+// those (exchange num - 1), as all have written num; and of two exchanges in turn one
+// flushes, so the emptying has completed before this workgroup sends to num + 2, and
+// whoever gets past that finds no old value in them.
+template <int NS, bool FLUSH, class During>
+__device__ __forceinline__ bool exchange(const ResidentArgs &A, Waits &E,
+                                         double (&v)[NS ? NS : 1], During during) {
   constexpr int kW = NS ? NS : 1;
   __shared__ double mine[3][16], all[3][kMaxBlocks / 64];
-  __shared__ int dead;
   const int t = fresh(threadIdx.x), lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6), nb = (int)gridDim.x;
-  ++num;
-  uint64_t *slot = A.slots + (size_t)(num % 3) * kMaxWords * kMaxBlocks;
-  uint64_t *last = A.slots + (size_t)((num + 2) % 3) * kMaxWords * kMaxBlocks;
+  const uint32_t num = ++E.num;
+  uint64_t *slot = A.slots + (size_t)(num % kSets) * kMaxWords * kMaxBlocks;
+  uint64_t *last = A.slots + (size_t)((num + kSets - 1) % kSets) * kMaxWords * kMaxBlocks;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const double w = wave_sum(v[s]);
     if (lane == 0) mine[s][wave] = w;
   }
-  if (t == 0) dead = 0;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what this wave published is there
+  if (FLUSH) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (wave == 0) {
     const int q = lane >> 4, i = lane & 15;
@@ -110,30 +146,21 @@ __device__ __forceinline__ bool exchange(const ResidentArgs &A, uint32_t &num,
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const uint64_t u = (uint64_t)__double_as_longlong(lane_value(w, 16 * s + 15));
-      if (lane == s) word = u == kEmpty ? kEmpty - 1 : u;
+      if (lane == s) word = u;
     }
-    if (lane < kW)
-      __hip_atomic_store(slot + (size_t)lane * kMaxBlocks + blockIdx.x, word, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+    if (lane < kW) put(slot + (size_t)lane * kMaxBlocks + blockIdx.x, word);
   }
+  during();
   if (wave < kMaxBlocks / 64) {
     uint64_t w[kW] = {};
     const uint64_t t0 = wall_clock64(), limit = num == 1 ? kArrive : kLost;
     for (int spin = 0; t < nb; ++spin) {
       bool here = true;
 #pragma unroll
-      for (int k = 0; k < kW; ++k)
-        w[k] = __hip_atomic_load(slot + (size_t)k * kMaxBlocks + t, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
+      for (int k = 0; k < kW; ++k) w[k] = get(slot + (size_t)k * kMaxBlocks + t);
 #pragma unroll
       for (int k = 0; k < kW; ++k) here = here && w[k] != kEmpty;
-      if (here) break;
-      if ((spin & 15) == 15 &&
-          (wall_clock64() - t0 > limit ||
-           __hip_atomic_load(A.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-        dead = 1;
-        break;
-      }
+      if (here || !keep_on(A, E, spin, t0, limit)) break;
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -143,13 +170,8 @@ __device__ __forceinline__ bool exchange(const ResidentArgs &A, uint32_t &num,
   }
   __syncthreads();
   if (wave == 0 && lane < kMaxWords)
-    __hip_atomic_store(last + (size_t)lane * kMaxBlocks + blockIdx.x, kEmpty, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  if (dead) {
-    if (t == 0)
-      __hip_atomic_store(A.abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return false;
-  }
+    store(last + (size_t)lane * kMaxBlocks + blockIdx.x, kEmpty);
+  if (gave_up(A, E)) return false;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     double sum = 0.0;
@@ -160,6 +182,11 @@ __device__ __forceinline__ bool exchange(const ResidentArgs &A, uint32_t &num,
   }
   return true;
 }
+template <int NS>
+__device__ __forceinline__ bool exchange(const ResidentArgs &A, Waits &E,
+                                         double (&v)[NS ? NS : 1]) {
+  return exchange<NS, true>(A, E, v, [] {});
+}
 
 // The runs of a workgroup's rows in LDS: run d holds rows i0 + (z0 + d) m0 m1 - m0 - 1 + k,
 // k < len = rb + 2 (m0 + 1); zero outside [0, n).
@@ -168,43 +195,69 @@ struct Window {
   __device__ __forceinline__ int at(int t, int o, int z0) const {  // row t's neighbour o
     return (o / 9 - 1 - z0) * len + m0 + 1 + ((o / 3) % 3 - 1) * m0 + (o % 3 - 1) + t;
   }
-  // dst = src (copy) or src + beta dst on the runs z0 .. z0 + NZ - 1; own rows: mine
-  template <int NZ>
-  __device__ __forceinline__ void refresh(double *dst, const double *src, int z0, bool copy,
-                                          double beta, double mine) const {
-    const int t = fresh(threadIdx.x), bd = blockDim.x;
-    double v[NZ][2];
+  // entry e of what run d reads (the own run: only the rows before and after the
+  // workgroup's own): how many, position in the run, row
+  __device__ __forceinline__ int count(int dz) const { return dz ? len : 2 * (m0 + 1); }
+  __device__ __forceinline__ int pos(int dz, int e) const { return dz || e <= m0 ? e : e + rb; }
+  __device__ __forceinline__ int row(int dz, int e) const {
+    return i0 + dz * m01 - m0 - 1 + pos(dz, e);
+  }
+};
+
+// A published vector into the runs z0 .. z0 + NZ - 1: issue() starts the loads, finish()
+// polls what was not there and stores dst = value (copy) or value + beta dst; own rows: mine.
+template <int NZ>
+struct Halo {
+  uint64_t v[NZ][2];
+  __device__ __forceinline__ void issue(const Window &W, const uint64_t *src, int z0) {
+    const int t = fresh(threadIdx.x);
 #pragma unroll
-    for (int d = 0; d < NZ; ++d) {
-      const bool own = z0 + d == 0;
+    for (int d = 0; d < NZ; ++d)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        // the own run: only the rows before and after the workgroup's own; lanes past the
-        // end read one address together
-        const int e = min(t + u * bd, (own ? 2 * (m0 + 1) : len) - 1);
-        const int j = i0 + (z0 + d) * m01 - m0 - 1 + (own && e > m0 ? e + rb : e);
-        v[d][u] = get(src + min(max(j, 0), n - 1));
-        if (j < 0 || j >= n) v[d][u] = 0.0;
+      for (int u = 0; u < (z0 + d == 0 ? 1 : 2); ++u) {  // lanes past the end read one address
+        const int j = W.row(z0 + d, min(t + u * (int)blockDim.x, W.count(z0 + d) - 1));
+        v[d][u] = get(src + min(max(j, 0), W.n - 1));
+      }
+  }
+  __device__ __forceinline__ bool missing(const Window &W, int z0) const {
+    bool m = false;
+#pragma unroll
+    for (int d = 0; d < NZ; ++d)
+#pragma unroll
+      for (int u = 0; u < (z0 + d == 0 ? 1 : 2); ++u) m = m || v[d][u] == kEmpty;
+    return m;
+  }
+  __device__ __forceinline__ void finish(const Window &W, const ResidentArgs &A, const Waits &E,
+                                         const uint64_t *src, int z0, double *dst, bool copy,
+                                         double beta, double mine) {
+    if (missing(W, z0)) {
+      const uint64_t t0 = wall_clock64();
+      for (int spin = 0; missing(W, z0) && keep_on(A, E, spin, t0, kLost); ++spin) {
+        __builtin_amdgcn_s_sleep(2);
+        issue(W, src, z0);  // all again: one round trip however many are missing
       }
     }
+    const int t = fresh(threadIdx.x), bd = blockDim.x;
 #pragma unroll
     for (int d = 0; d < NZ; ++d) {
-      const bool own = z0 + d == 0;
-      double *run = dst + d * len;
-      const int count = own ? 2 * (m0 + 1) : len;
+      double *run = dst + d * W.len;
+      auto one = [&](int e, uint64_t w) {
+        const int j = W.row(z0 + d, e), k = W.pos(z0 + d, e);
+        const double x = j >= 0 && j < W.n ? __longlong_as_double((long long)w) : 0.0;
+        run[k] = copy ? x : x + beta * run[k];
+      };
+      const int held = z0 + d == 0 ? 1 : 2;
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int e = t + u * bd, k = own && e > m0 ? e + rb : e;
-        if (e < count) run[k] = copy ? v[d][u] : v[d][u] + beta * run[k];
+      for (int u = 0; u < held; ++u)
+        if (t + u * bd < W.count(z0 + d)) one(t + u * bd, v[d][u]);
+      for (int e = t + held * bd; e < W.count(z0 + d); e += bd) {  // long lattice rows
+        const uint64_t *p = src + min(max(W.row(z0 + d, e), 0), W.n - 1);
+        const uint64_t t0 = wall_clock64();
+        uint64_t w = get(p);
+        for (int spin = 0; w == kEmpty && keep_on(A, E, spin, t0, kLost); ++spin) w = get(p);
+        one(e, w);
       }
-      for (int e = t + 2 * bd; e < count; e += bd) {
-        const int k = own && e > m0 ? e + rb : e;
-        const int j = i0 + (z0 + d) * m01 - m0 - 1 + k;
-        double w = get(src + min(max(j, 0), n - 1));
-        if (j < 0 || j >= n) w = 0.0;
-        run[k] = copy ? w : w + beta * run[k];
-      }
-      if (own) run[m0 + 1 + t] = mine;
+      if (z0 + d == 0) run[W.m0 + 1 + t] = mine;
     }
   }
 };
@@ -212,7 +265,7 @@ struct Window {
 template <bool FACT>
 __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const ResidentArgs A) {
   extern __shared__ __align__(16) double lds[];
-  __shared__ int bad;
+  __shared__ int bad, dead;
   const int t = threadIdx.x, n = (int)A.B.n, bd = blockDim.x;
   Window W;
   W.n = n;
@@ -221,7 +274,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
   W.i0 = (int)blockIdx.x * A.rb;
   W.rb = A.rb;
   W.len = A.rb + 2 * (W.m0 + 1);
-  double *run = lds, *tmp = lds + 3 * W.len;
+  double *run = lds, *rrun = lds + 3 * W.len, *yrun = lds + 5 * W.len;
   const int i = W.i0 + t, ic = min(i, n - 1);
   const bool own = i < n;
   // coefficients: rows are runs of nzval; a lattice row holds its in-box neighbours in
@@ -259,50 +312,60 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     }
   }
   const double dinv = A.jacobi && a[13] != 0.0 ? 1.0 / a[13] : 1.0;
-  uint32_t num = 0;
-  int turn = 0;
-  double *src = nullptr;  // the last publication
+  if (t == 0) dead = 0;
+  Waits E{0, &dead};
+  int turn = 1;  // the buffer of the last z
   double none[1], xi = own ? A.x[i] : 0.0, ri = 0.0, zi = 0.0, pi = 0.0;
-  auto publish = [&](double v) {
-    src = A.pub + (turn ? n : 0);
-    turn ^= 1;
-    if (own) put(src + W.i0 + fresh(t), v);
+  Halo<3> H;
+  auto publish = [&](uint64_t *buf, double v) {
+    if (own) put(buf + W.i0 + fresh(t), (uint64_t)__double_as_longlong(v));
   };
-  // z = Gᵀ G r, r published; z published and its sum exchanged.  False: aborted
-  auto apply = [&](double &rz) {
+  auto zbuf = [&](int k) { return A.zpub + (k & 1 ? n : 0); };
+  // r published: z = Gᵀ G r
+  auto apply = [&] {
     float g[14];
+    Halo<2> P;
+    P.issue(W, A.rpub, -1);
     const int t1 = fresh(t), j1 = min(W.i0 + t1, n - 1);
 #pragma unroll
     for (int o = 0; o < 14; ++o) g[o] = A.g14[(int64_t)o * n + j1];
-    W.refresh<2>(tmp, src, -1, true, 0.0, ri);
+    P.finish(W, A, E, A.rpub, -1, rrun, true, 0.0, ri);
     __syncthreads();
+    if (gave_up(A, E)) return false;
     double y = 0.0;
 #pragma unroll
-    for (int o = 0; o < 14; ++o) y += (double)g[o] * tmp[W.at(t1, o, -1)];
+    for (int o = 0; o < 14; ++o) y += (double)g[o] * rrun[W.at(t1, o, -1)];
     if (!own) y = 0.0;
-    publish(y);
-    if (!exchange<0>(A, num, none)) return false;
+    publish(A.ypub, y);
+    P.issue(W, A.ypub, 0);
     const int t2 = fresh(t), j2 = min(W.i0 + t2, n - 1);
 #pragma unroll
     for (int o = 0; o < 14; ++o) g[o] = A.g14[(int64_t)o * n + j2 - box_off(A.B, o)];
-    W.refresh<2>(tmp, src, 0, true, 0.0, y);
+    P.finish(W, A, E, A.ypub, 0, yrun, true, 0.0, y);
     __syncthreads();
+    if (gave_up(A, E)) return false;
     zi = 0.0;
 #pragma unroll
-    for (int o = 13; o >= 0; --o) zi += (double)g[o] * tmp[W.at(t2, 26 - o, 0)];
+    for (int o = 13; o >= 0; --o) zi += (double)g[o] * yrun[W.at(t2, 26 - o, 0)];
     if (!own) zi = 0.0;
-    publish(zi);
-    double v[1] = {zi * ri};
-    const bool there = exchange<1>(A, num, v);
-    rz = v[0];
-    return there;
+    return true;
+  };
+  // past the exchange that follows the publication of z: the buffers of the next turn
+  auto empty = [&](bool other) {
+    if (!own) return;
+    const int j = W.i0 + fresh(t);
+    if (other) store(zbuf(turn + 1) + j, kEmpty);
+    if (FACT) {
+      store(A.rpub + j, kEmpty);
+      store(A.ypub + j, kEmpty);
+    }
   };
   int it = 0, restarts = 0, converged = 0;
   double relres = INFINITY, rz = 0.0, thr = 0.0, beta = 0.0, how = kDone;
   bool start = !A.resume, first = false;
   if (start) {
-    publish(xi);
-    if (!exchange<0>(A, num, none)) return;
+    publish(zbuf(++turn), xi);
+    if (!exchange<0>(A, E, none)) return;
   } else {
     it = (int)A.out[1];
     rz = A.out[4];
@@ -314,18 +377,22 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       pi = A.p[i];
       zi = A.z[i];
     }
-    publish(pi);
-    if (!exchange<0>(A, num, none)) return;
-    W.refresh<3>(run, src, -1, true, 0.0, pi);
-    publish(zi);
-    if (!exchange<0>(A, num, none)) return;
+    publish(zbuf(++turn), pi);
+    if (!exchange<0>(A, E, none)) return;
+    H.issue(W, zbuf(turn), -1);
+    H.finish(W, A, E, zbuf(turn), -1, run, true, 0.0, pi);
+    publish(zbuf(++turn), zi);
+    if (!exchange<0>(A, E, none)) return;
+    empty(true);
   }
+  H.issue(W, zbuf(turn), -1);
   const int until = A.maxit - it > kPause ? it + kPause : A.maxit;
   // each turn multiplies by A once: a step of the recurrence, or (start) the true residual
   for (;;) {
     pi = start ? xi : first ? zi : zi + beta * pi;
-    W.refresh<3>(run, src, -1, start || first, beta, pi);
+    H.finish(W, A, E, zbuf(turn), -1, run, start || first, beta, pi);
     __syncthreads();
+    if (gave_up(A, E)) return;
     double q = 0.0;
     const int t1 = fresh(t);
 #pragma unroll
@@ -335,40 +402,52 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       const double bi = own ? A.b[W.i0 + fresh(t)] : 0.0;
       ri = bi - q;
       zi = dinv * ri;
-      publish(FACT ? ri : zi);
+      publish(FACT ? A.rpub : zbuf(++turn), FACT ? ri : zi);
       double v[3] = {ri * ri, bi * bi, zi * ri};
-      if (!exchange<3>(A, num, v)) return;
+      if (!exchange<3>(A, E, v)) return;
       const double bnorm = sqrt(v[1]) > 0 ? sqrt(v[1]) : 1.0;
       relres = lane_value(sqrt(v[0]) / bnorm, 0);
       converged = relres <= A.rtol;
       if (converged || it >= A.maxit || restarts > 3) break;
       rz = v[2];
-      if (FACT && !apply(rz)) return;
+      if (FACT) {
+        if (!apply()) return;
+        publish(zbuf(++turn), zi);
+        double w[1] = {zi * ri};
+        if (!exchange<1>(A, E, w)) return;
+        rz = w[0];
+      }
+      H.issue(W, zbuf(turn), -1);
+      empty(true);
       ++restarts;
       thr = lane_value((A.rtol * bnorm) * (A.rtol * bnorm), 0);
       first = true;
       start = false;
     } else {
       double pq[1] = {pi * q};
-      if (!exchange<1>(A, num, pq)) return;
+      if (!exchange<1>(A, E, pq)) return;
       const double alpha = lane_value(rz / pq[0], 0);
       xi += alpha * pi;
       ri -= alpha * q;
       zi = dinv * ri;
-      publish(FACT ? ri : zi);
+      if (FACT) {
+        publish(A.rpub, ri);
+        if (!apply()) return;
+      }
+      publish(zbuf(++turn), zi);
       double v[2] = {ri * ri, zi * ri};
-      if (!exchange<2>(A, num, v)) return;
+      if (!exchange<2, false>(A, E, v, [&] { H.issue(W, zbuf(turn), -1); })) return;
+      beta = lane_value(v[1] / rz, 0);
+      rz = v[1];
       ++it;
       first = false;
       // at the tolerance, not finite or at the limit: the true residual decides
       start = !(v[0] > thr) || !isfinite(v[0]) || it >= A.maxit;
+      empty(!start);
       if (start) {
-        publish(xi);
-        if (!exchange<0>(A, num, none)) return;
-      } else {
-        if (FACT && !apply(v[1])) return;
-        beta = lane_value(v[1] / rz, 0);
-        rz = v[1];
+        publish(zbuf(++turn), xi);
+        if (!exchange<0>(A, E, none)) return;
+        H.issue(W, zbuf(turn), -1);
       }
     }
     if (!start && it >= until) {
@@ -395,10 +474,14 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
   }
 }
 
-// Before each launch: no exchange has happened, nothing is aborted.
+// Before each launch: no exchange has happened, nothing is published or aborted.
 __global__ void resident_clear_kernel(ResidentArgs A) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < 3 * kMaxWords * kMaxBlocks) A.slots[k] = kEmpty;
+  if (k < kSets * kMaxWords * kMaxBlocks) A.slots[k] = kEmpty;
+  if (k < (int)A.B.n) {
+    A.zpub[k] = A.zpub[k + A.B.n] = kEmpty;
+    if (A.rpub) A.rpub[k] = A.ypub[k] = kEmpty;
+  }
   if (k == 0) *A.abort = 0;
   if (k == 0) A.out[0] = kNone;
 }
@@ -410,7 +493,7 @@ struct Shape {
 Shape shape(const Box &B, int cus, bool fact) {
   const int64_t nb = std::min(cus, kMaxBlocks);
   const int64_t rb = std::max<int64_t>(((B.n + nb - 1) / nb + 63) / 64 * 64, kMinRows);
-  const int64_t runs = (fact ? 5 : 3) * (rb + 2 * (B.m0 + 1)) * (int64_t)sizeof(double);
+  const int64_t runs = (fact ? 7 : 3) * (rb + 2 * (B.m0 + 1)) * (int64_t)sizeof(double);
   return {(int)std::min<int64_t>(rb, INT32_MAX), (int)((B.n + rb - 1) / rb),
           (size_t)std::max<int64_t>(runs, kStageRows * 27 * sizeof(double))};
 }
@@ -450,9 +533,9 @@ bool resident_system(const Ctx &c, const Box &B, int precond) {
 }
 
 bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, double *x,
-                  const double *b, double *const (&state)[3], double *pub, unsigned char *ws,
-                  gh_solve_stats *st) {
-  static_assert(sizeof(double) * (kOut + 8) + sizeof(uint64_t) * 3 * kMaxWords * kMaxBlocks <=
+                  const double *b, double *const (&state)[3], double *const (&pub)[3],
+                  unsigned char *ws, gh_solve_stats *st) {
+  static_assert(sizeof(double) * (kOut + 8) + sizeof(uint64_t) * kSets * kMaxWords * kMaxBlocks <=
                     kResidentWs, "workspace");
   Turn turn(c.device);
   if (!turn.flag) return false;
@@ -472,17 +555,20 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
   A.r = state[0];
   A.p = state[1];
   A.z = state[2];
-  A.pub = pub;
+  A.zpub = reinterpret_cast<uint64_t *>(pub[0]);
+  A.rpub = fact ? reinterpret_cast<uint64_t *>(pub[1]) : nullptr;
+  A.ypub = fact ? reinterpret_cast<uint64_t *>(pub[2]) : nullptr;
   A.out = reinterpret_cast<double *>(ws);
   A.abort = reinterpret_cast<uint32_t *>(A.out + kOut);
   A.slots = reinterpret_cast<uint64_t *>(A.out + kOut + 8);
   auto kern = fact ? resident_pcg_kernel<true> : resident_pcg_kernel<false>;
   GH_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)S.lds));
+  const int64_t clear = std::max<int64_t>(B.n, kSets * kMaxWords * kMaxBlocks);
   double h[kOut + 1];
   do {
-    hipLaunchKernelGGL(resident_clear_kernel, dim3((3 * kMaxWords * kMaxBlocks + 255) / 256),
-                       dim3(256), 0, c.stream, A);
+    hipLaunchKernelGGL(resident_clear_kernel, dim3((unsigned)((clear + 255) / 256)), dim3(256), 0,
+                       c.stream, A);
     hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks), dim3((unsigned)S.rb), S.lds, c.stream, A);
     GH_CHECK_HIP(hipGetLastError());
     HostCopy copy(c);
