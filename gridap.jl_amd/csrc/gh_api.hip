@@ -492,6 +492,8 @@ int gh_symbolic(gh_ctx *ctx, int64_t *nnz_out) {
                    c.h_cell_dofs.size() == c.cell_dofs.n,
                GH_ERR_STATE, "the FE space does not match the mesh: upload it again");
     invalidate_pattern(c);
+    c.adjptr.release();
+    c.adj.release();
     if (c.have_trial) {
       gh::rect_symbolic(c);
       if (nnz_out) *nnz_out = c.nnz;

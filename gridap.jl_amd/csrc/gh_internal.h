@@ -454,7 +454,9 @@ void rect_assemble(Ctx &c, int form, int precision);  // its values and lifting 
 // one composite block's current nzval moved to its positions in c.comp_nz, enqueued on
 // the block's stream
 void compose_move(Ctx &c, int block);
-void elemlist_symbolic(Ctx &c);         // dof -> cell adjacency, Dirichlet masks
+void adjacency_build(Ctx &c);           // dof -> cell adjacency
+int adjacency_bits(const Ctx &c);       // its local index bits
+void elemlist_symbolic(Ctx &c);         // adjacency (if not built), Dirichlet masks, lists
 void elemlist_sum(Ctx &c, bool f32);     // nzval from the element entries
 void assemble_simplex(Ctx &c, int precision);
 // boundary.hip

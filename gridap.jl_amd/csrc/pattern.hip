@@ -3,8 +3,9 @@
 // Gridap (src/Algebra/SparseMatrixCSC.jl:72-283) counts, allocates, inserts each
 // (i,j) touched by a cell into column j by binary search and compacts: the result
 // is, per column, the sorted unique rows of every (i>0, j>0) pair of every cell,
-// explicit zeros kept.  Here every cell emits its pairs as packed (col,row) keys,
-// one radix sort orders them, and a unique-flag scan writes rowval/colptr.  The
+// explicit zeros kept.  Here the cells of a column give its candidates, sorted in LDS
+// (spaces that keep contribution lists), or every cell emits its pairs as packed (col,row)
+// keys, one radix sort orders them, and a unique-flag scan writes rowval/colptr.  The
 // order is total, so the pattern is bit-identical whatever the launch order.
 #include <hipcub/hipcub.hpp>
 
@@ -98,6 +99,135 @@ __global__ void scatter_rows(int64_t n, const uint64_t *__restrict__ keys,
   int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n || !flags[k]) return;
   rowval[pos[k]] = (int32_t)(keys[k] & rowmask);
+}
+
+// ---- pattern and contributions column by column, from the dof -> cell adjacency ----
+// A column's candidates are its cells' dofs: nloc per adjacent cell, a few hundred at most on
+// usual meshes, sorted by (row, emit index) in LDS by one wave.  The candidates of all
+// columns sorted together as (column, row) keys with their indices took, for scalar Q2 of
+// 14³ cells (2 M pairs), 0.2 ms of sorting and 2.0 ms of allocating and freeing the keys;
+// here they are never stored: symbolic phase 2.5 -> 0.41 ms.  Columns with more than
+// kMaxCandidates keep the global sort.
+constexpr int kMaxCandidates = 2048, kColWaves = 4;
+
+// Free dofs of each cell.
+__global__ void cell_free_counts(int64_t ncells, int nloc, const int32_t *__restrict__ cell_dofs,
+                                 int32_t *__restrict__ nfree) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= ncells) return;
+  int m = 0;
+  for (int a = 0; a < nloc; ++a) m += cell_dofs[c * nloc + a] > 0;
+  nfree[c] = m;
+}
+
+// Contributions of each column (0 past the last); the most adjacent cells of a column.
+__global__ void column_contributions(int ncols, const int32_t *__restrict__ adjptr,
+                                     const int32_t *__restrict__ adj, int lbits,
+                                     const int32_t *__restrict__ cell_free,
+                                     int32_t *__restrict__ count, int32_t *__restrict__ most) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  int len = 0;
+  if (j < ncols) {
+    const int a0 = adjptr[j], a1 = adjptr[j + 1];
+    int m = 0;
+    for (int a = a0; a < a1; ++a) m += cell_free[adj[a] >> lbits];
+    count[j] = m;
+    len = a1 - a0;
+  } else if (j == ncols) {
+    count[j] = 0;
+  }
+  for (int o = 32; o > 0; o >>= 1) len = max(len, __shfl_xor(len, o));
+  if ((threadIdx.x & 63) == 0) atomicMax(most, len);
+}
+
+// One wave per column: its candidates sorted by (row, emit index); perm takes the emit
+// indices, count the number of rows (flagged when there is none; 0 past the last column).
+__global__ __launch_bounds__(64 * kColWaves) void column_sort(
+    int ncols, int nloc, int lbits, int cap, const int32_t *__restrict__ cell_dofs,
+    const int32_t *__restrict__ adjptr, const int32_t *__restrict__ adj,
+    const int32_t *__restrict__ qptr, int32_t *__restrict__ perm, int32_t *__restrict__ count,
+    int32_t *__restrict__ bad) {
+  extern __shared__ __align__(16) uint64_t cand[];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int j = blockIdx.x * kColWaves + w;
+  if (j >= ncols) {
+    if (j == ncols && lane == 0) count[j] = 0;
+    return;
+  }
+  uint64_t *key = cand + (size_t)w * cap;
+  const int a0 = adjptr[j], m = (adjptr[j + 1] - a0) * nloc;
+  const int q0 = qptr[j], valid = qptr[j + 1] - q0;
+  int n = 64;
+  while (n < m) n *= 2;
+  for (int k = lane; k < n; k += 64) {
+    uint64_t v = ~uint64_t(0);  // Dirichlet rows and the padding sort last
+    if (k < m) {
+      const int row = cell_dofs[(adj[a0 + k / nloc] >> lbits) * nloc + k % nloc];
+      if (row > 0) v = ((uint64_t)(row - 1) << 32) | (uint32_t)k;
+    }
+    key[k] = v;
+  }
+  wave_sync();
+  for (int size = 2; size <= n; size *= 2)
+    for (int step = size / 2; step > 0; step /= 2) {
+      for (int k = lane; k < n / 2; k += 64) {
+        const int x = 2 * k - (k & (step - 1)), y = x + step;
+        const uint64_t a = key[x], b = key[y];
+        if ((a > b) == ((x & size) == 0)) {
+          key[x] = b;
+          key[y] = a;
+        }
+      }
+      wave_sync();
+    }
+  int rows = 0;
+  for (int k0 = 0; k0 < valid; k0 += 64) {
+    const int k = k0 + lane;
+    bool first = false;
+    if (k < valid) {
+      const uint64_t v = key[k];
+      const int pos = (int)(uint32_t)v, e = adj[a0 + pos / nloc];
+      perm[q0 + k] =
+          ((e >> lbits) * nloc + (e & ((1 << lbits) - 1))) * nloc + pos % nloc;
+      first = k == 0 || (key[k - 1] >> 32) != (v >> 32);
+    }
+    rows += __popcll(__ballot(first));
+  }
+  if (lane == 0) {
+    count[j] = rows;
+    if (rows == 0) atomicOr(bad, 1);
+  }
+}
+
+// One wave per column: its rows and the first contribution of each.
+__global__ __launch_bounds__(64 * kColWaves) void column_rows(
+    int ncols, int nloc, int64_t nnz, const int32_t *__restrict__ cell_dofs,
+    const int32_t *__restrict__ qptr, const int32_t *__restrict__ perm,
+    const int32_t *__restrict__ colptr, int32_t *__restrict__ rowval,
+    int32_t *__restrict__ cstart) {
+  const int lane = threadIdx.x & 63, j = blockIdx.x * kColWaves + (threadIdx.x >> 6);
+  if (j >= ncols) return;
+  if (j == 0 && lane == 0) cstart[nnz] = qptr[ncols];
+  const int q0 = qptr[j], valid = qptr[j + 1] - q0;
+  int at = colptr[j], last = -1;
+  for (int k0 = 0; k0 < valid; k0 += 64) {
+    const int k = k0 + lane;
+    int row = -1;
+    if (k < valid) {
+      const int t = perm[q0 + k], cell = t / (nloc * nloc);
+      row = cell_dofs[cell * nloc + t % nloc] - 1;
+    }
+    int before = __shfl_up(row, 1);
+    if (lane == 0) before = last;
+    const uint64_t first = __ballot(row >= 0 && row != before);
+    if (row >= 0 && row != before) {
+      const int p = at + __popcll(first & ((uint64_t(1) << lane) - 1));
+      rowval[p] = row;
+      cstart[p] = q0 + k;
+    }
+    at += __popcll(first);
+    last = __shfl(row, 63);
+  }
 }
 
 // ---- lattice eligibility (Cartesian mesh, scalar Q1) ----
@@ -322,6 +452,55 @@ void exclusive_sum_ws(const T *in, T *out, int64_t n, hipStream_t s, DBuf<unsign
 
 }  // namespace
 
+// false (nothing set): a column has too many candidates
+static bool symbolic_columns(Ctx &c) {
+  hipStream_t s = c.stream;
+  const int N = (int)c.nfree, lbits = adjacency_bits(c);
+  const int64_t L = N + 1;
+  // cell_free, contributions, their starts, rows per column; the flags
+  DBuf<int32_t> ws;
+  ws.resize(c.ncells + 3 * L + 2);
+  int32_t *cell_free = ws.get(), *count = cell_free + c.ncells, *qptr = count + L;
+  int32_t *rows = qptr + L, *most = rows + L, *bad = most + 1;
+  GH_CHECK_HIP(hipMemsetAsync(most, 0, 2 * sizeof(int32_t), s));
+  hipLaunchKernelGGL(cell_free_counts, dim3(grid_for(c.ncells)), dim3(kBlock), 0, s, c.ncells,
+                     c.nloc, c.cell_dofs.get(), cell_free);
+  hipLaunchKernelGGL(column_contributions, dim3(grid_for(L)), dim3(kBlock), 0, s, N,
+                     c.adjptr.get(), c.adj.get(), lbits, cell_free, count, most);
+  GH_CHECK_HIP(hipGetLastError());
+  exclusive_sum_ws(count, qptr, L, s, c.ws_cub);
+  int32_t h[2] = {0, 0};
+  HostCopy copy(c);
+  copy.down(&h[0], qptr + N, sizeof(int32_t));
+  copy.down(&h[1], most, sizeof(int32_t));
+  int cap = 64;
+  while (cap < kMaxCandidates && cap < (int64_t)h[1] * c.nloc) cap *= 2;
+  if (cap < (int64_t)h[1] * c.nloc) return false;
+  c.perm.resize(std::max(h[0], 1));
+  c.colptr.resize(L);
+  const unsigned grid = (unsigned)((L + kColWaves - 1) / kColWaves);
+  hipLaunchKernelGGL(column_sort, dim3(grid), dim3(64 * kColWaves),
+                     sizeof(uint64_t) * cap * kColWaves, s, N, c.nloc, lbits, cap,
+                     c.cell_dofs.get(), c.adjptr.get(), c.adj.get(), qptr, c.perm.get(), rows, bad);
+  GH_CHECK_HIP(hipGetLastError());
+  exclusive_sum_ws(rows, c.colptr.get(), L, s, c.ws_cub);
+  copy.down(&h[0], c.colptr.get() + N, sizeof(int32_t));
+  copy.down(&h[1], bad, sizeof(int32_t));
+  GH_REQUIRE(h[1] == 0, GH_ERR_UNSUPPORTED, "a free dof with no matrix entry");
+  c.nnz = h[0];
+  c.rowval.resize(std::max<int64_t>(c.nnz, 1));
+  c.cstart.resize(c.nnz + 1);
+  hipLaunchKernelGGL(column_rows, dim3(grid), dim3(64 * kColWaves), 0, s, N, c.nloc, c.nnz,
+                     c.cell_dofs.get(), qptr, c.perm.get(), c.colptr.get(), c.rowval.get(),
+                     c.cstart.get());
+  GH_CHECK_HIP(hipGetLastError());
+  c.nzval.resize(std::max<int64_t>(c.nnz, 1));
+  c.b.resize(std::max<int64_t>(c.nfree, 1));
+  GH_CHECK_HIP(hipStreamSynchronize(s));  // ws is freed
+  c.have_pattern = true;
+  return true;
+}
+
 void symbolic_general(Ctx &c, bool contributions) {
   hipStream_t s = c.stream;
   const int64_t per = (int64_t)c.nloc * c.nloc;
@@ -330,6 +509,10 @@ void symbolic_general(Ctx &c, bool contributions) {
              "cell pair count exceeds 2^31 in one symbolic pass");
   const int rb = bits_for(std::max<int64_t>(c.nfree, 1));
   GH_REQUIRE(2 * rb <= 64, GH_ERR_UNSUPPORTED, "dof count too large for packed keys");
+  if (contributions && total > 0 && c.nfree > 0) {
+    adjacency_build(c);
+    if (symbolic_columns(c)) return;
+  }
   const uint64_t invalid = (uint64_t)c.nfree << rb;
 
   DBuf<uint64_t> keys, sorted;

@@ -732,42 +732,47 @@ void compact_contributions(Ctx &c, int lbits) {
   c.elem.release();
 }
 
-void elemlist_symbolic(Ctx &c) {
-  c.elemlist = false;
-  c.adjptr.release();
-  c.adj.release();
-  c.dmask.release();
-  c.elem.release();
-  if (!(simplex_eligible(c) || hexq2_eligible(c) || hexgen_eligible(c)) || c.nfree == 0) return;
+int adjacency_bits(const Ctx &c) { return c.nloc <= 16 ? 4 : 7; }
+
+// adjptr, adj: per free dof its (cell << bits | local) in ascending order.
+void adjacency_build(Ctx &c) {
   hipStream_t s = c.stream;
   const int64_t total = c.ncells * c.nloc;
-  const int lbits = c.nloc <= 16 ? 4 : 7;
+  const int lbits = adjacency_bits(c);
   GH_REQUIRE(total < (int64_t(1) << 31) && c.ncells < (int64_t(1) << (31 - lbits)),
              GH_ERR_UNSUPPORTED, "mesh too large for the element-list adjacency");
   int rb = 1;
   while ((int64_t(1) << rb) <= c.nfree) ++rb;
   const uint64_t invalid = (uint64_t)c.nfree << 32;
-  DBuf<uint64_t> keys, sorted;
-  keys.resize(total);
-  sorted.resize(total);
+  // the keys are made in (cell, local) order and the sort is stable: the dof bits suffice
+  size_t bytes = 0;
+  GH_CHECK_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, bytes, (const uint64_t *)nullptr,
+                                                 (uint64_t *)nullptr, (int)total, 32, 32 + rb, s));
+  DBuf<uint64_t> ws;  // the sort's storage, keys, sorted
+  const size_t head = (bytes + 255) / 256 * 32;
+  ws.resize(head + 2 * total);
+  uint64_t *keys = ws.get() + head, *sorted = keys + total;
   hipLaunchKernelGGL(dof_cell_keys, dim3(grid_for(total)), dim3(kBlock), 0, s, c.ncells, c.nloc,
-                     lbits, c.cell_dofs.get(), invalid, keys.get());
+                     lbits, c.cell_dofs.get(), invalid, keys);
   GH_CHECK_HIP(hipGetLastError());
-  {
-    size_t bytes = 0;
-    GH_CHECK_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, bytes, keys.get(), sorted.get(),
-                                                   (int)total, 0, 32 + rb, s));
-    DBuf<unsigned char> tmp;
-    tmp.resize(std::max<size_t>(bytes, 1));
-    GH_CHECK_HIP(hipcub::DeviceRadixSort::SortKeys(tmp.get(), bytes, keys.get(), sorted.get(),
-                                                   (int)total, 0, 32 + rb, s));
-    GH_CHECK_HIP(hipStreamSynchronize(s));
-  }
-  keys.release();
+  GH_CHECK_HIP(hipcub::DeviceRadixSort::SortKeys((void *)ws.get(), bytes,
+                                                 (const uint64_t *)keys, sorted, (int)total, 32,
+                                                 32 + rb, s));
   c.adjptr.resize(c.nfree + 1);
   c.adj.resize(total);
   hipLaunchKernelGGL(adjacency_fill, dim3(grid_for(total)), dim3(kBlock), 0, s, total, c.nfree,
-                     sorted.get(), c.adjptr.get(), c.adj.get());
+                     sorted, c.adjptr.get(), c.adj.get());
+  GH_CHECK_HIP(hipGetLastError());
+  GH_CHECK_HIP(hipStreamSynchronize(s));  // ws is freed
+}
+
+void elemlist_symbolic(Ctx &c) {
+  c.elemlist = false;
+  c.dmask.release();
+  c.elem.release();
+  if (!(simplex_eligible(c) || hexq2_eligible(c) || hexgen_eligible(c)) || c.nfree == 0) return;
+  hipStream_t s = c.stream;
+  if (!c.adjptr.get()) adjacency_build(c);  // else by symbolic_general, from this pattern
   c.dmask.resize(c.ncells);
   hipLaunchKernelGGL(dirichlet_mask_kernel, dim3(grid_for(c.ncells)), dim3(kBlock), 0, s,
                      c.ncells, c.nloc, c.cell_dofs.get(), c.dmask.get());
@@ -775,7 +780,7 @@ void elemlist_symbolic(Ctx &c) {
   GH_CHECK_HIP(hipStreamSynchronize(s));
   c.fdet.resize(c.ncells);
   c.elemlist = true;
-  compact_contributions(c, lbits);
+  compact_contributions(c, adjacency_bits(c));
 }
 
 template <class T>
