@@ -406,7 +406,8 @@ struct Ctx {
 // that ends without it waits before its staging is reused.
 class HostCopy {
  public:
-  explicit HostCopy(Ctx &c);
+  // direct: the runtime's own copies, nothing allocated (pinned memory or events)
+  explicit HostCopy(Ctx &c, bool direct = false);
   ~HostCopy();
   HostCopy(const HostCopy &) = delete;
   HostCopy &operator=(const HostCopy &) = delete;
@@ -415,6 +416,8 @@ class HostCopy {
   // 0-based 32-bit ids on the device to 1-based 64-bit ids on the host
   void down_ids(int64_t *host, const int32_t *dev, size_t count);
   void finish();
+  // a word of pinned memory that the device may write; null when direct
+  uint64_t *word() const;
   template <class T>
   void up(DBuf<T> &dev, const T *host, size_t count) {
     up(dev.get(), host, sizeof(T) * count);
@@ -483,8 +486,9 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
 constexpr int kSmallMaxN = 4096;
 constexpr int kSmallStream = 1 << 17;  // streamed entries (10 bytes each)
 constexpr size_t kSmallWs = (size_t)kSmallStream * 10 + 8 * (16 + 2 * kSmallMaxN);
-bool pcg_small(Ctx &c, int precond, double rtol, int maxit, double *x, const double *b,
-               unsigned char *ws, gh_solve_stats *st);
+class HostCopy;
+bool pcg_small(Ctx &c, HostCopy &copy, int precond, double rtol, int maxit, double *x,
+               const double *b, unsigned char *ws, gh_solve_stats *st);
 // solve_resident.hip: the whole solve of a box system in one launch of workgroups that stay
 // on their compute units.  state: r, p, z of a solve that takes several launches; pub: 2n
 // words, and n and n with FSAI; ws kResidentWs bytes.  False: not taken (st untouched), x a valid initial guess.

@@ -24,14 +24,16 @@ namespace {
 
 constexpr size_t kChunk = size_t(1) << 20;
 constexpr int kSlots = 4;
-constexpr size_t kMaxIdle = 8;
+constexpr size_t kMaxIdle = 8, kBytes = kSlots * kChunk + 64;  // the slots, a word
 
 std::mutex g_mu;
-std::vector<char *> g_idle;  // kSlots x kChunk bytes each
+std::vector<char *> g_idle;  // kBytes each
 
 }  // namespace
 
-HostCopy::HostCopy(Ctx &c) : s_(c.stream), ev_(c.copy_events()) {
+HostCopy::HostCopy(Ctx &c, bool direct) : s_(c.stream) {
+  if (direct) return;
+  ev_ = c.copy_events();
   {
     std::lock_guard<std::mutex> lock(g_mu);
     if (!g_idle.empty()) {
@@ -40,12 +42,13 @@ HostCopy::HostCopy(Ctx &c) : s_(c.stream), ev_(c.copy_events()) {
     }
   }
   if (!buf_)
-    GH_CHECK_HIP(hipHostMalloc((void **)&buf_, kSlots * kChunk,
-                               hipHostMallocDefault | hipHostMallocPortable));
+    GH_CHECK_HIP(hipHostMalloc((void **)&buf_, kBytes,
+                               hipHostMallocCoherent | hipHostMallocPortable));
 }
 
 HostCopy::~HostCopy() {
   if (busy_) (void)hipStreamSynchronize(s_);  // an error path: copies may be in flight
+  if (!buf_) return;
   try {
     std::lock_guard<std::mutex> lock(g_mu);
     if (g_idle.size() < kMaxIdle) {
@@ -62,7 +65,16 @@ void HostCopy::wait_slot(int k) {
   used_[k] = false;
 }
 
+uint64_t *HostCopy::word() const {
+  return buf_ ? reinterpret_cast<uint64_t *>(buf_ + kSlots * kChunk) : nullptr;
+}
+
 void HostCopy::up(void *dev, const void *host, size_t bytes) {
+  if (!buf_) {
+    busy_ = true;
+    if (bytes) GH_CHECK_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s_));
+    return;
+  }
   for (size_t o = 0; o < bytes; o += kChunk) {
     const size_t n = std::min(kChunk, bytes - o);
     const int k = next_;
@@ -104,6 +116,11 @@ void HostCopy::down_chunks(const void *dev, size_t bytes, size_t unit,
 }
 
 void HostCopy::down(void *host, const void *dev, size_t bytes) {
+  if (!buf_) {
+    if (bytes) GH_CHECK_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s_));
+    GH_CHECK_HIP(hipStreamSynchronize(s_));
+    return;
+  }
   down_chunks(dev, bytes, 1, [&](const char *src, size_t at, size_t n) {
     std::memcpy((char *)host + at, src, n);
   });

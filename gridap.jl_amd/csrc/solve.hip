@@ -34,14 +34,14 @@ namespace gh {
 namespace {
 
 constexpr int kBlock = 512;
-constexpr int kMaxParts = 8192;  // partial slots per reduced quantity (max blocks per grid)
+constexpr int kMaxParts = 1024;  // partial slots per reduced quantity (max blocks per grid)
 constexpr int kApplyLanes = 4;   // lanes per row in the FSAI applications
 
 // scalar slots
 constexpr int kRz = 0;  // [0..1]: r·z, double-buffered by iteration parity
 // convergence decided on the device: kStop = 0 (running), 1 (r·r met the threshold),
 // 2 (r·r not finite); kStopIt = the iteration at whose start it was decided
-constexpr int kStop = 5, kStopIt = 6;
+constexpr int kStop = 5, kStopIt = 6, kBad = 7;
 
 // One partial per block: part[blockIdx.x] = Σ_block v, for up to four quantities with one
 // barrier (wave sums inside the vector unit, the wave sums by the first wave).
@@ -129,13 +129,20 @@ constexpr int kStartLds = 2 * (kBlock / 64) + 1;
 // previous update against thr = (rtol ‖b‖)²; true when the solve stops here (block 0
 // records why and at which iteration).  Every block has summed the same partials in the
 // same order, so every block takes the same decision.
-__device__ __forceinline__ bool iteration_stops(double *scal, double rr, int first, double thr,
-                                                int it) {
-  if (first) return false;
-  const bool stop = !(rr > thr) || !isfinite(rr);
-  if (stop && blockIdx.x == 0 && threadIdx.x == 0) {
-    scal[kStop] = isfinite(rr) ? 1.0 : 2.0;
-    scal[kStopIt] = (double)it;
+// news (a word of pinned host memory, or null): the iteration that has begun, and
+// kStopped when it is the one that stops.
+constexpr uint64_t kStopped = uint64_t(1) << 32;
+__device__ __forceinline__ bool iteration_stops(double *scal, uint64_t *news, double rr, int first,
+                                                double thr, int it) {
+  const bool stop = !first && (!(rr > thr) || !isfinite(rr));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (stop) {
+      scal[kStop] = isfinite(rr) ? 1.0 : 2.0;
+      scal[kStopIt] = (double)it;
+    }
+    if (news)
+      __hip_atomic_store(news, (stop ? kStopped : 0) | (uint32_t)it, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
   return stop;
 }
@@ -287,7 +294,8 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_kernel(
     const double *__restrict__ val, const double2 *__restrict__ zp, double2 *__restrict__ zpnew,
     double *__restrict__ q, double *scal, int par, int first,
     const double *__restrict__ part_rz, const double *__restrict__ part_rr, int np_rz, double thr,
-    int it, double *__restrict__ part_pq) {
+    int it, uint64_t *news,
+    double *__restrict__ part_pq) {
   __shared__ double sh[kStartLds];
   StartIn S = start_loads(scal, part_rz, first ? nullptr : part_rr, np_rz);
   const double rz_old = scal[kRz + (par ^ 1)];
@@ -312,7 +320,7 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_kernel(
   if (t < ntiles) open(t);
   if (start_sums(S, sh)) return;
   const double rz = S.a;
-  if (iteration_stops(scal, S.b, first, thr, it)) return;
+  if (iteration_stops(scal, news, S.b, first, thr, it)) return;
   const double beta = first ? 0.0 : rz / rz_old;
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[kRz + par] = rz;
   double dot = 0.0;
@@ -680,7 +688,7 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_box_kernel(
     const double *__restrict__ pold, double *__restrict__ pnew, double *__restrict__ q,
     double *scal, int par, int first, const double *__restrict__ part_rz,
     const double *__restrict__ part_rr, int np_rz, double thr, int it,
-    double *__restrict__ part_pq) {
+    uint64_t *news, double *__restrict__ part_pq) {
   extern __shared__ __align__(16) double run[];
   __shared__ double sh[kStartLds];
   using R = Runs<WIDE, -1, 3>;
@@ -704,7 +712,7 @@ __global__ __launch_bounds__(kBlock) void spmv_dir_box_kernel(
   if (T.t < T.end) loads(T.t);
   if (start_sums(S, sh)) return;
   const double rz = S.a;
-  if (iteration_stops(scal, S.b, first, thr, it)) return;
+  if (iteration_stops(scal, news, S.b, first, thr, it)) return;
   const double beta = first ? 0.0 : rz / rz_old;
   if (blockIdx.x == 0 && threadIdx.x == 0) scal[kRz + par] = rz;
   double dot = 0.0;
@@ -893,7 +901,8 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
     e1 = c.timing_events()[1];
     GH_CHECK_HIP(hipEventRecord(e0, s));
   }
-  HostCopy copy(c);
+  HostCopy copy(c, !timed);
+  uint64_t *news = copy.word();
   double *dinv = nullptr;
   const int factored = precond == GH_PRECOND_FSAI;
   // box lattice: stencil kernels (A as 14 offset arrays, G as 14), one thread per row
@@ -905,16 +914,14 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   const Box B{n, c.box_m[0], c.box_m[1], c.box_m[2]};
   if (box) {
     c.a27.resize((size_t)14 * nn);
-    DBuf<int> bad;
-    bad.resize(1);
-    GH_CHECK_HIP(hipMemsetAsync(bad.get(), 0, sizeof(int), s));
+    int *bad = reinterpret_cast<int *>(V.scal + kBad);
+    GH_CHECK_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
     hipLaunchKernelGGL(stencil_values_kernel, dim3((unsigned)((n + kConvRows - 1) / kConvRows)),
                        dim3(kConvRows), 0, s, B, c.colptr.get(), c.nzval.get(), c.a27.get(),
-                       bad.get());
+                       bad);
     GH_CHECK_HIP(hipGetLastError());
     int hbad = 0;
-    GH_CHECK_HIP(hipMemcpyAsync(&hbad, bad.get(), sizeof(int), hipMemcpyDeviceToHost, s));
-    GH_CHECK_HIP(hipStreamSynchronize(s));
+    copy.down(&hbad, bad, sizeof(int));
     box = hbad == 0;
   }
   if (precond == GH_PRECOND_JACOBI) {
@@ -950,7 +957,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
     auto kern = wide ? spmv_dir_box_kernel<true> : spmv_dir_box_kernel<false>;
     hipLaunchKernelGGL(kern, dim3(g_box), dim3(kBlock), 3 * run_bytes, s, B, ntiles, c.a27.get(),
                        V.z, pold, pnew, V.q, scal, par, first, part_rz, part_rr, np_rz, thr, itk,
-                       part_pq);
+                       news, part_pq);
   };
   auto lower_box = [&](bool start, int par, double *rold, double *rnew, double *pnew) {
     auto kern = wide ? (start ? update_lower_box_kernel<true, true>
@@ -968,7 +975,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   };
   // partial counts of each quantity, by producer
   const int np_rz = factored ? (int)g_apply : (int)g_vec;
-  double hrr[kPcgGrid], hbb[kPcgGrid];  // g_vec <= kPcgGrid partials
+  double hsum[kMaxParts + kPcgGrid];  // r·r and b·b: neighbours, g_vec <= kPcgGrid of each
 
   double bnorm = 1.0, relres = INFINITY;
   int it = 0, restarts = 0;
@@ -990,69 +997,89 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
                          c.gue.get(), c.gui.get(), V.y, rbuf[0], zpbuf[0], scal, part_rz);
     }
     GH_CHECK_HIP(hipGetLastError());
-    copy.down(hrr, part_rr, sizeof(double) * g_vec);
-    copy.down(hbb, part_bb, sizeof(double) * g_vec);
-    const double bb = host_sum(hbb, (int)g_vec);
+    copy.down(hsum, part_rr, sizeof(double) * (kMaxParts + g_vec));
+    const double bb = host_sum(hsum + kMaxParts, (int)g_vec);
     bnorm = std::sqrt(bb) > 0 ? std::sqrt(bb) : 1.0;
-    relres = std::sqrt(host_sum(hrr, (int)g_vec)) / bnorm;
+    relres = std::sqrt(host_sum(hsum, (int)g_vec)) / bnorm;
     if (relres <= rtol) {
       converged = true;
       break;
     }
     if (it >= maxit || restarts > 3) break;
     ++restarts;
-    // iterations are enqueued in chunks; each spmv_dir decides on the device whether
-    // the previous update met the tolerance, and once it has, every later kernel of
-    // the chunk returns at once.  The host reads the decision after each chunk.
-    const int chunk = 16;
+    // each spmv_dir decides on the device whether the previous update met the tolerance,
+    // and once it has, every later kernel returns at once
     const double thr = (rtol * bnorm) * (rtol * bnorm);
     int k = 0;  // iteration since this start: selects the buffers and scalar slots
-    bool stopped = false;
-    while (it < maxit && !stopped) {
-      for (int m = 0; m < chunk && it + m < maxit; ++m, ++k) {
-        const int par = k & 1;
-        const int itk = it + m;
-        double *pold = pbuf[par], *pnew = pbuf[par ^ 1];
-        double2 *zpold = zpbuf[par], *zpnew = zpbuf[par ^ 1];
-        if (box)
-          spmv_dir_box(pold, pnew, par, k == 0 ? 1 : 0, np_rz, thr, itk);
-        else
-          row_shape(c.nnz, n, [&](auto L, auto U) {
-            const int nt = (int)((n + kBlock / L() - 1) / (kBlock / L()));
-            hipLaunchKernelGGL((spmv_dir_kernel<L(), U()>), dim3(g_spmv), dim3(kBlock), 0, s,
-                               (int)n, nt, c.colptr.get(), c.rowval.get(), c.nzval.get(), zpold,
-                               zpnew, V.q, scal, par, k == 0 ? 1 : 0, part_rz, part_rr, np_rz,
-                               thr, itk, part_pq);
-          });
-        if (factored && box) {
-          double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
-          lower_box(false, par, rold, rnew, pnew);
-          upper_box(rnew);
-        } else if (factored) {
-          double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
-          hipLaunchKernelGGL(update_lower_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, par,
-                             c.gle.get(), c.gli.get(), V.x, rold, rnew, zpnew, V.q,
-                             V.y, scal, part_pq, (int)g_spmv, part_rr);
-          hipLaunchKernelGGL(upper_rz_kernel<false>, dim3(g_apply), dim3(kBlock), 0, s, n,
-                             c.gue.get(), c.gui.get(), V.y, rnew, zpnew, scal, part_rz);
-        } else if (!box) {
-          hipLaunchKernelGGL(update_zp_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, par, dinv,
-                             V.x, rbuf[0], zpnew, V.q, scal, part_pq, (int)g_spmv, part_rz,
-                             part_rr);
-        } else {
-          hipLaunchKernelGGL(update_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, par, dinv,
-                             V.x, rbuf[0], V.z, pnew, V.q, scal, part_pq,
-                             (int)g_spmv, part_rz, part_rr);
+    auto iteration = [&](int itk) {
+      const int par = k & 1;
+      double *pold = pbuf[par], *pnew = pbuf[par ^ 1];
+      double2 *zpold = zpbuf[par], *zpnew = zpbuf[par ^ 1];
+      if (box)
+        spmv_dir_box(pold, pnew, par, k == 0 ? 1 : 0, np_rz, thr, itk);
+      else
+        row_shape(c.nnz, n, [&](auto L, auto U) {
+          const int nt = (int)((n + kBlock / L() - 1) / (kBlock / L()));
+          hipLaunchKernelGGL((spmv_dir_kernel<L(), U()>), dim3(g_spmv), dim3(kBlock), 0, s,
+                             (int)n, nt, c.colptr.get(), c.rowval.get(), c.nzval.get(), zpold,
+                             zpnew, V.q, scal, par, k == 0 ? 1 : 0, part_rz, part_rr, np_rz,
+                             thr, itk, news, part_pq);
+        });
+      if (factored && box) {
+        double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
+        lower_box(false, par, rold, rnew, pnew);
+        upper_box(rnew);
+      } else if (factored) {
+        double *rold = rbuf[par], *rnew = rbuf[par ^ 1];
+        hipLaunchKernelGGL(update_lower_kernel, dim3(g_apply), dim3(kBlock), 0, s, n, par,
+                           c.gle.get(), c.gli.get(), V.x, rold, rnew, zpnew, V.q,
+                           V.y, scal, part_pq, (int)g_spmv, part_rr);
+        hipLaunchKernelGGL(upper_rz_kernel<false>, dim3(g_apply), dim3(kBlock), 0, s, n,
+                           c.gue.get(), c.gui.get(), V.y, rnew, zpnew, scal, part_rz);
+      } else if (!box) {
+        hipLaunchKernelGGL(update_zp_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, par, dinv,
+                           V.x, rbuf[0], zpnew, V.q, scal, part_pq, (int)g_spmv, part_rz,
+                           part_rr);
+      } else {
+        hipLaunchKernelGGL(update_kernel, dim3(g_vec), dim3(kBlock), 0, s, n, par, dinv,
+                           V.x, rbuf[0], V.z, pnew, V.q, scal, part_pq,
+                           (int)g_spmv, part_rz, part_rr);
+      }
+      ++k;
+    };
+    // The host enqueues at most kAhead iterations past the one that the device says it has
+    // begun, and none once it has stopped: the device never waits for the host (a read-back
+    // every 16 iterations left it idle for 18 µs each time), and little is enqueued in
+    // vain.  Without the word, chunks of 16 and a read-back.
+    constexpr int kAhead = 3, kChunk = 16;
+    constexpr uint64_t kNoNews = ~uint64_t(0);
+    bool stopped = false, ended = false;
+    if (news) __atomic_store_n(news, kNoNews, __ATOMIC_RELAXED);  // the stream is idle
+    for (int m = 0; it < maxit && !stopped; ++m) {
+      iteration(it++);
+      GH_CHECK_HIP(hipGetLastError());
+      if (news) {
+        for (unsigned spin = 1; !ended; ++spin) {
+          const uint64_t v = __atomic_load_n(news, __ATOMIC_RELAXED);
+          const int begun = v == kNoNews ? it - m - 2 : (int)(uint32_t)v;
+          stopped = v != kNoNews && (v & kStopped);
+          if (stopped) it = begun;  // iterations completed before the stop
+          if (stopped || it - 1 - begun <= kAhead) break;
+          __builtin_ia32_pause();
+          if (spin % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(s);
+            if (e == hipErrorNotReady) (void)hipGetLastError();
+            else GH_CHECK_HIP(e);
+            ended = e == hipSuccess;  // nothing more will come: read back below
+          }
         }
       }
-      GH_CHECK_HIP(hipGetLastError());
-      double st2[2] = {0.0, 0.0};
-      copy.down(st2, scal + kStop, sizeof(st2));
-      if (st2[0] != 0.0) {
-        it = (int)st2[1];  // iterations completed before the stop
-        stopped = true;
-      } else {
-        it = std::min(it + chunk, maxit);
+      if (!stopped && (it == maxit || ended || (!news && (m + 1) % kChunk == 0))) {
+        double st2[2] = {0.0, 0.0};
+        copy.down(st2, scal + kStop, sizeof(st2));
+        stopped = st2[0] != 0.0;
+        if (stopped) it = (int)st2[1];
+        ended = false;
       }
     }
     // the true residual of the next start decides convergence (and, if the stopped
@@ -1105,7 +1132,9 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
   };
   c.s_small.resize(std::max(kSmallWs, kResidentWs));
   if (small_system(c, precond) && timed([&] {
-        return pcg_small(c, precond, rtol, maxit, c.s_x.get(), c.s_b.get(), c.s_small.get(), st);
+        HostCopy copy(c);
+        return pcg_small(c, copy, precond, rtol, maxit, c.s_x.get(), c.s_b.get(),
+                         c.s_small.get(), st);
       }))
     return;
   const size_t nn = (size_t)std::max<int64_t>(c.nfree, 1);
@@ -1182,7 +1211,7 @@ void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, i
                   nullptr, base + 4 * L, part, part + 4 * (size_t)kMaxParts,
                   (double2 *)(base + 5 * L), (double2 *)(base + 7 * L)};
   const auto t0 = std::chrono::steady_clock::now();
-  HostCopy copy(c);
+  HostCopy copy(c, true);
   copy.up(V.x, x, sizeof(double) * n);
   if (b)
     copy.up(V.b, b, sizeof(double) * n);
@@ -1192,7 +1221,7 @@ void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, i
   // the one-workgroup solve's workspace: the two {z, p}, which it does not need
   static_assert(kSmallWs <= 4 * kNoAllocVec * sizeof(double), "workspace");
   if (!(small_system(c, precond) &&
-        pcg_small(c, precond, rtol, maxit, V.x, V.b, (unsigned char *)V.zp, st)))
+        pcg_small(c, copy, precond, rtol, maxit, V.x, V.b, (unsigned char *)V.zp, st)))
     pcg_run(c, V, precond, rtol, maxit, false, false, st);
   copy.down(x, V.x, sizeof(double) * n);
   copy.finish();

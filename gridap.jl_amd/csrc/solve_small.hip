@@ -303,8 +303,8 @@ void launch(const SmallArgs &A, hipStream_t s) {
 }  // namespace
 
 // At most kSmallMaxN rows; the bound on the padded slices is checked by the kernel.
-bool pcg_small(Ctx &c, int precond, double rtol, int maxit, double *x, const double *b,
-               unsigned char *ws, gh_solve_stats *st) {
+bool pcg_small(Ctx &c, HostCopy &copy, int precond, double rtol, int maxit, double *x,
+               const double *b, unsigned char *ws, gh_solve_stats *st) {
   const int64_t n = c.nfree;
   double *at = reinterpret_cast<double *>(ws);
   SmallArgs A{};
@@ -329,7 +329,6 @@ bool pcg_small(Ctx &c, int precond, double rtol, int maxit, double *x, const dou
     else if (n <= 2 * kT) launch<2, 32>(A, c.stream);
     else if (n <= 4 * kT) launch<4, 18>(A, c.stream);
     else launch<8, 9>(A, c.stream);
-    HostCopy copy(c);
     copy.down(h, A.out, sizeof(h));
     A.resume = 1;
   } while (h[3] == kPaused);
