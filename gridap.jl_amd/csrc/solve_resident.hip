@@ -1,5 +1,5 @@
 // PCG on a box lattice in one launch: the workgroups stay on their compute units for the
-// whole solve and keep their rows' matrix in registers.
+// whole solve and keep their rows' matrix in registers (and some in LDS).
 //
 // The two kernels of an iteration (solve.hip) read the stencil again every time, 28 MB at
 // 64³, and pay two launches.  Here a workgroup owns rb consecutive rows, one per thread, with
@@ -28,7 +28,8 @@
 //
 // Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.1, 31³
 // 11.9 and 6.8; FSAI 25.3 and 19.3, 17.5 and 12.4.  (Barriers for the published vectors
-// too: 10.7, 7.6, 22.6, 16.0.)  What bounds it: the trips through the fabric, 3 to 4 µs an
+// too: 10.7, 7.6, 22.6, 16.0.)  Rows past one a thread, in LDS: 65³ 19.6 and 16.2, 70³ 20.6
+// and 17.2.  What bounds it: the trips through the fabric, 3 to 4 µs an
 // exchange or published vector with 245 workgroups, 2 with 14.  Hence the largest
 // workgroups that fit, 512 rows at least (31³ with barriers: 256 rows 8.3, 512 7.1, 1024 7.3).
 //
@@ -49,7 +50,7 @@ namespace {
 
 constexpr int kMaxBlocks = 256, kMaxThreads = 1024, kMinRows = 512, kMaxWords = 3, kSets = 4;
 constexpr uint64_t kEmpty = 0xfff7a11ce5107000ull;  // a NaN (see exchange)
-constexpr int kStageRows = 256;  // rows whose values are staged at once
+constexpr int kStageRows = 128;  // rows whose values are staged at once
 constexpr int kPause = 2048;
 constexpr size_t kMaxLds = 150 * 1024;
 constexpr uint64_t kArrive = 200000, kLost = 100000000;  // ticks of 10 ns
@@ -262,7 +263,7 @@ struct Halo {
   }
 };
 
-template <bool FACT>
+template <bool FACT, bool EXTRA>
 __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const ResidentArgs A) {
   extern __shared__ __align__(16) double lds[];
   __shared__ int bad, dead;
@@ -275,8 +276,13 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
   W.rb = A.rb;
   W.len = A.rb + 2 * (W.m0 + 1);
   double *run = lds, *rrun = lds + 3 * W.len, *yrun = lds + 5 * W.len;
+  // EXTRA: rows past one per thread, their state and coefficients in LDS
+  const int ext = EXTRA ? A.rb - bd : 0;
+  double *xs = lds + max(3 * W.len, kStageRows * 27), *rs = xs + ext, *zs = rs + ext;
+  double *ps = zs + ext, *ds = ps + ext, *as = ds + ext;
+  const bool has2 = EXTRA && t < ext;
   const int i = W.i0 + t, ic = min(i, n - 1);
-  const bool own = i < n;
+  const bool own = i < n, own2 = has2 && i + bd < n;
   // coefficients: rows are runs of nzval; a lattice row holds its in-box neighbours in
   // offset order
   double a[27];
@@ -287,7 +293,14 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     if (t == 0) bad = 0;
     __syncthreads();
     if (!ok) bad = 1;
-    for (int c0 = 0; c0 < bd; c0 += kStageRows) {
+    uint32_t vm2 = 0;
+    int q2 = 0;
+    if (EXTRA && own2) {
+      vm2 = box_valid(A.B, i + bd);
+      q2 = A.cp[i + bd];
+      if (A.cp[i + bd + 1] - q2 != __popc(vm2)) bad = 1;
+    }
+    for (int c0 = 0; c0 < A.rb; c0 += kStageRows) {
       const int r0 = min(W.i0 + c0, n), r1 = min(r0 + kStageRows, n);
       const int p0 = A.cp[r0], count = min(A.cp[r1] - p0, kStageRows * 27);
       __syncthreads();
@@ -303,6 +316,18 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
           k += in ? 1 : 0;
         }
       }
+      if (has2 && t + bd >= c0 && t + bd < c0 + kStageRows) {
+        int k = max(min(q2 - p0, kStageRows * 27 - 27), 0);
+        for (int o = 0; o < 27; ++o) {
+          const bool in = (vm2 >> o) & 1u;
+          as[o * ext + t] = in ? lds[k] : 0.0;
+          k += in ? 1 : 0;
+        }
+        const double d = as[13 * ext + t];
+        ds[t] = A.jacobi && d != 0.0 ? 1.0 / d : 1.0;
+        xs[t] = own2 ? A.x[i + bd] : 0.0;
+        rs[t] = zs[t] = ps[t] = 0.0;
+      }
     }
     __syncthreads();
     if (bad) {  // not the lattice matrix: the general kernels take it
@@ -317,8 +342,10 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
   int turn = 1;  // the buffer of the last z
   double none[1], xi = own ? A.x[i] : 0.0, ri = 0.0, zi = 0.0, pi = 0.0;
   Halo<3> H;
-  auto publish = [&](uint64_t *buf, double v) {
-    if (own) put(buf + W.i0 + fresh(t), (uint64_t)__double_as_longlong(v));
+  auto publish = [&](uint64_t *buf, double v, const double *v2) {
+    const int j = W.i0 + fresh(t);
+    if (own) put(buf + j, (uint64_t)__double_as_longlong(v));
+    if (own2) put(buf + j + bd, (uint64_t)__double_as_longlong(v2[j - W.i0]));
   };
   auto zbuf = [&](int k) { return A.zpub + (k & 1 ? n : 0); };
   // r published: z = Gᵀ G r
@@ -336,7 +363,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
 #pragma unroll
     for (int o = 0; o < 14; ++o) y += (double)g[o] * rrun[W.at(t1, o, -1)];
     if (!own) y = 0.0;
-    publish(A.ypub, y);
+    publish(A.ypub, y, nullptr);
     P.issue(W, A.ypub, 0);
     const int t2 = fresh(t), j2 = min(W.i0 + t2, n - 1);
 #pragma unroll
@@ -355,6 +382,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     if (!own) return;
     const int j = W.i0 + fresh(t);
     if (other) store(zbuf(turn + 1) + j, kEmpty);
+    if (other && own2) store(zbuf(turn + 1) + j + bd, kEmpty);
     if (FACT) {
       store(A.rpub + j, kEmpty);
       store(A.ypub + j, kEmpty);
@@ -364,7 +392,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
   double relres = INFINITY, rz = 0.0, thr = 0.0, beta = 0.0, how = kDone;
   bool start = !A.resume, first = false;
   if (start) {
-    publish(zbuf(++turn), xi);
+    publish(zbuf(++turn), xi, xs);
     if (!exchange<0>(A, E, none)) return;
   } else {
     it = (int)A.out[1];
@@ -377,11 +405,16 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       pi = A.p[i];
       zi = A.z[i];
     }
-    publish(zbuf(++turn), pi);
+    if (own2) {
+      rs[t] = A.r[i + bd];
+      ps[t] = A.p[i + bd];
+      zs[t] = A.z[i + bd];
+    }
+    publish(zbuf(++turn), pi, ps);
     if (!exchange<0>(A, E, none)) return;
     H.issue(W, zbuf(turn), -1);
     H.finish(W, A, E, zbuf(turn), -1, run, true, 0.0, pi);
-    publish(zbuf(++turn), zi);
+    publish(zbuf(++turn), zi, zs);
     if (!exchange<0>(A, E, none)) return;
     empty(true);
   }
@@ -391,6 +424,11 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
   for (;;) {
     pi = start ? xi : first ? zi : zi + beta * pi;
     H.finish(W, A, E, zbuf(turn), -1, run, start || first, beta, pi);
+    if (has2) {
+      const int e = fresh(t);
+      ps[e] = start ? xs[e] : first ? zs[e] : zs[e] + beta * ps[e];
+      run[W.at(e + bd, 13, -1)] = ps[e];
+    }
     __syncthreads();
     if (gave_up(A, E)) return;
     double q = 0.0;
@@ -398,12 +436,27 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
 #pragma unroll
     for (int o = 0; o < 27; ++o) q += a[o] * run[W.at(t1, o, -1)];
     if (!own) q = 0.0;
+    double q2 = 0.0;
+    if (own2) {
+      const int e = fresh(t);
+#pragma unroll 9
+      for (int o = 0; o < 27; ++o) q2 += as[o * ext + e] * run[W.at(e + bd, o, -1)];
+    }
     if (start) {
       const double bi = own ? A.b[W.i0 + fresh(t)] : 0.0;
       ri = bi - q;
       zi = dinv * ri;
-      publish(FACT ? A.rpub : zbuf(++turn), FACT ? ri : zi);
       double v[3] = {ri * ri, bi * bi, zi * ri};
+      if (own2) {
+        const int e = fresh(t);
+        const double b2 = A.b[W.i0 + e + bd], r2 = b2 - q2, z2 = ds[e] * r2;
+        rs[e] = r2;
+        zs[e] = z2;
+        v[0] += r2 * r2;
+        v[1] += b2 * b2;
+        v[2] += z2 * r2;
+      }
+      publish(FACT ? A.rpub : zbuf(++turn), FACT ? ri : zi, zs);
       if (!exchange<3>(A, E, v)) return;
       const double bnorm = sqrt(v[1]) > 0 ? sqrt(v[1]) : 1.0;
       relres = lane_value(sqrt(v[0]) / bnorm, 0);
@@ -412,7 +465,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       rz = v[2];
       if (FACT) {
         if (!apply()) return;
-        publish(zbuf(++turn), zi);
+        publish(zbuf(++turn), zi, nullptr);
         double w[1] = {zi * ri};
         if (!exchange<1>(A, E, w)) return;
         rz = w[0];
@@ -425,17 +478,27 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       start = false;
     } else {
       double pq[1] = {pi * q};
+      if (own2) pq[0] += ps[fresh(t)] * q2;
       if (!exchange<1>(A, E, pq)) return;
       const double alpha = lane_value(rz / pq[0], 0);
       xi += alpha * pi;
       ri -= alpha * q;
       zi = dinv * ri;
       if (FACT) {
-        publish(A.rpub, ri);
+        publish(A.rpub, ri, nullptr);
         if (!apply()) return;
       }
-      publish(zbuf(++turn), zi);
       double v[2] = {ri * ri, zi * ri};
+      if (own2) {
+        const int e = fresh(t);
+        xs[e] += alpha * ps[e];
+        const double r2 = rs[e] - alpha * q2, z2 = ds[e] * r2;
+        rs[e] = r2;
+        zs[e] = z2;
+        v[0] += r2 * r2;
+        v[1] += z2 * r2;
+      }
+      publish(zbuf(++turn), zi, zs);
       if (!exchange<2, false>(A, E, v, [&] { H.issue(W, zbuf(turn), -1); })) return;
       beta = lane_value(v[1] / rz, 0);
       rz = v[1];
@@ -445,7 +508,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       start = !(v[0] > thr) || !isfinite(v[0]) || it >= A.maxit;
       empty(!start);
       if (start) {
-        publish(zbuf(++turn), xi);
+        publish(zbuf(++turn), xi, xs);
         if (!exchange<0>(A, E, none)) return;
         H.issue(W, zbuf(turn), -1);
       }
@@ -458,10 +521,17 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
         A.p[j] = pi;
         A.z[j] = zi;
       }
+      if (own2) {
+        const int e = fresh(t), j = W.i0 + e + bd;
+        A.r[j] = rs[e];
+        A.p[j] = ps[e];
+        A.z[j] = zs[e];
+      }
       break;
     }
   }
   if (own) A.x[W.i0 + fresh(t)] = xi;
+  if (own2) A.x[W.i0 + bd + fresh(t)] = xs[t];
   if (blockIdx.x == 0 && t == 0) {
     A.out[0] = how;
     A.out[1] = it;
@@ -486,16 +556,19 @@ __global__ void resident_clear_kernel(ResidentArgs A) {
   if (k == 0) A.out[0] = kNone;
 }
 
+// rb rows per workgroup, one per thread up to 1024; without FSAI the rows past that are
+// kept in LDS (5 vectors and 27 coefficients each) while it lasts.
 struct Shape {
-  int rb, blocks;
+  int rb, threads, blocks;
   size_t lds;
 };
 Shape shape(const Box &B, int cus, bool fact) {
   const int64_t nb = std::min(cus, kMaxBlocks);
   const int64_t rb = std::max<int64_t>(((B.n + nb - 1) / nb + 63) / 64 * 64, kMinRows);
-  const int64_t runs = (fact ? 7 : 3) * (rb + 2 * (B.m0 + 1)) * (int64_t)sizeof(double);
-  return {(int)std::min<int64_t>(rb, INT32_MAX), (int)((B.n + rb - 1) / rb),
-          (size_t)std::max<int64_t>(runs, kStageRows * 27 * sizeof(double))};
+  const int64_t threads = std::min<int64_t>(rb, kMaxThreads);
+  const int64_t runs = std::max<int64_t>((fact ? 7 : 3) * (rb + 2 * (B.m0 + 1)), kStageRows * 27);
+  return {(int)std::min<int64_t>(rb, INT32_MAX), (int)threads, (int)((B.n + rb - 1) / rb),
+          sizeof(double) * (size_t)(runs + 32 * (rb - threads))};
 }
 
 int compute_units(int device) {
@@ -529,7 +602,7 @@ bool resident_system(const Ctx &c, const Box &B, int precond) {
   const int cus = compute_units(c.device);
   if (cus < 1 || B.n < 1) return false;
   const Shape S = shape(B, cus, precond == GH_PRECOND_FSAI);
-  return S.rb <= kMaxThreads && S.lds <= kMaxLds;
+  return (S.rb == S.threads || precond != GH_PRECOND_FSAI) && S.lds <= kMaxLds;
 }
 
 bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, double *x,
@@ -561,7 +634,9 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
   A.out = reinterpret_cast<double *>(ws);
   A.abort = reinterpret_cast<uint32_t *>(A.out + kOut);
   A.slots = reinterpret_cast<uint64_t *>(A.out + kOut + 8);
-  auto kern = fact ? resident_pcg_kernel<true> : resident_pcg_kernel<false>;
+  auto kern = fact ? resident_pcg_kernel<true, false>
+              : S.rb > S.threads ? resident_pcg_kernel<false, true>
+                                 : resident_pcg_kernel<false, false>;
   GH_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)S.lds));
   const int64_t clear = std::max<int64_t>(B.n, kSets * kMaxWords * kMaxBlocks);
@@ -569,7 +644,8 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
   do {
     hipLaunchKernelGGL(resident_clear_kernel, dim3((unsigned)((clear + 255) / 256)), dim3(256), 0,
                        c.stream, A);
-    hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks), dim3((unsigned)S.rb), S.lds, c.stream, A);
+    hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks), dim3((unsigned)S.threads), S.lds, c.stream,
+                       A);
     GH_CHECK_HIP(hipGetLastError());
     HostCopy copy(c);
     copy.down(h, A.out, sizeof(h));

@@ -1,12 +1,15 @@
 """The solve of a box system in one launch of resident workgroups against the launched
 stencil kernels on the same system: fewer rows than a workgroup, rows at the edges of the
 workgroups (512 and 1024 rows) and of their number (256), long and short lattice rows, the
-largest system it takes and one past it, restarts, limits, a solve over several launches
+largest systems it takes and ones past them, restarts, limits, a solve over several launches
 and calls from two threads at once (needs an MI355X).
 
 Both form the same products and add a row's entries in the same order; they differ in the
-grouping of the dot products only, so the iteration count agrees to one and the solutions,
-stopped at 1e-10, to 1e-10 times the condition (below 1e4 here)."""
+grouping of the dot products only: after 20 iterations the iterates agree to rounding
+(20 iterations x condition 1e4 x 2 eps = 1e-10), and the
+solutions, stopped at 1e-10, to 1e-10 times the condition (below 1e4 here).  Rounding acts
+on CG like a small spread of the eigenvalues (Greenbaum 1989), whose effect on the count
+grows with the count: one iteration, or 1% in solves of hundreds."""
 import os
 import threading
 
@@ -48,9 +51,11 @@ def launched(monkeypatch, ctx, **kw):
 
 
 # free rows: 1, 2, 40, 512, 528, 8 long lattice rows, 16 x 15 x 1025, 64 x 64 x 63 = 258,048
-# (1024 a workgroup), 64^3 = 262,144 (the largest), 65 x 64 x 63 = 262,080, 64 x 65 x 64 past
+# (1024 a workgroup), 64^3 = 262,144, 65 x 64 x 63 = 262,080, 64 x 65 x 64 past one row a
+# thread (FSAI's largest), 71 x 70 x 69 and 72 x 70 x 72 around the most that LDS holds
 PARTS = [(2, 2, 2), (3, 2, 2), (2, 6, 9), (33, 17, 2), (34, 17, 2), (514, 3, 3), (1100, 4, 5),
-         (17, 16, 1026), (65, 65, 64), (65, 65, 65), (66, 65, 64), (65, 66, 65)]
+         (17, 16, 1026), (65, 65, 64), (65, 65, 65), (66, 65, 64), (65, 66, 65),
+         (72, 71, 70), (73, 71, 73)]
 
 
 @pytest.mark.parametrize("part", PARTS)
@@ -64,9 +69,14 @@ def test_matches_launched_kernels(part, monkeypatch):
         kw = dict(x0=x0, precond=precond, rtol=1e-10, maxit=5000)
         x, st = ctx.pcg(**kw)
         y, sy = launched(monkeypatch, ctx, **kw)
-        assert st.converged and sy.converged and abs(st.iterations - sy.iterations) <= 1
+        assert st.converged and sy.converged
+        assert abs(st.iterations - sy.iterations) <= max(1, 0.01 * sy.iterations)
         assert np.linalg.norm(b - A @ x) <= 1.01e-10 * np.linalg.norm(b)
         assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+        if precond != _lib.GH_PRECOND_FSAI:  # (FSAI at its limit goes on with Jacobi)
+            few = dict(kw, maxit=20, raise_on_noconv=False)
+            u, v = ctx.pcg(**few)[0], launched(monkeypatch, ctx, **few)[0]
+            assert np.linalg.norm(u - v) <= 1e-10 * np.linalg.norm(v)
         z, _ = ctx.pcg(**kw)  # the same bits every time
         np.testing.assert_array_equal(x, z)
 
