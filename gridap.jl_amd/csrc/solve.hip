@@ -15,8 +15,9 @@
 // G and Gᵀ are read from the solver's 16-slot row copy (weights with D^-1/2
 // folded in, column indices), written with the factor.  When the free dofs form a
 // full box of Q1 lattice nodes, the same iteration runs on stencil kernels with no
-// column indices: A as 27 offset arrays, G as 14, Gᵀ read from G's arrays at the
-// mirrored offsets.
+// column indices: A as 14 offset arrays (lower half, the upper mirrored), G as 14, Gᵀ read
+// from G's arrays at the mirrored offsets.  Small systems (solve_small.hip) and boxes that
+// fit the device's registers (solve_resident.hip) are solved in one launch instead.
 // Reductions are deterministic and need no grid-wide synchronisation: a kernel
 // writes one partial per block, and every block of the consuming kernel sums all
 // of them in index order at its start (the same value everywhere); block 0 of
@@ -146,6 +147,8 @@ __device__ __forceinline__ bool iteration_stops(double *scal, uint64_t *news, do
   }
   return stop;
 }
+
+constexpr unsigned kStencilGrid = 512;  // two workgroups on each of 256 compute units
 
 inline unsigned grid_rows(int64_t rows, int rows_per_block) {
   return (unsigned)std::min<int64_t>(
@@ -596,7 +599,8 @@ __global__ void diag_inv_box_kernel(int64_t n, const double *__restrict__ a27,
 // the 14 arrays.  All 27 coefficient loads of a row are independent and issued together,
 // ahead of the reduction that gives β.  A row used to load coefficient and vector inside
 // the branch of each neighbour, 27 round trips one after the other: spmv_dir 22.5 µs at
-// 64³ and 181 µs at 128³ (latency), now 11.1 and 70 µs (bandwidth: 294 MB, 4.2 TB/s);
+// 64³ and 181 µs at 128³ (latency), now 10.2 and 70 µs (bandwidth: 294 MB, 4.2 TB/s; with
+// the mirrored entries that miss L2 490 MB, 7 TB/s);
 // update_lower 10.6 -> 7.8 µs, upper_rz 6.5 -> 4.8 µs at 64³.
 // Each XCD sweeps a contiguous slab of the tiles in order, so the mirrored coefficients
 // of the next plane are in its L2 when the plane itself reads them.
@@ -945,7 +949,9 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   // the vector kernels: two entries per thread, one with the interleaved z and p
   const unsigned g_vec = grid_rows(box ? (n + 1) / 2 : n, kBlock);
   const unsigned g_box = grid_rows(n, kBlock);            // one tile per block and turn
-  unsigned g_spmv = g_box;
+  // the stencil product: the two workgroups a compute unit holds, so that every slab is
+  // swept once in order (1024 of them, half waiting: 100³ 45.8 µs an iteration, now 43.9)
+  unsigned g_spmv = std::min(g_box, kStencilGrid);
   if (!box) row_shape(c.nnz, n, [&](auto L, auto) { g_spmv = grid_rows(n, kBlock / L()); });
   const unsigned g_apply = box ? g_box : grid_rows(n, kBlock / kApplyLanes);
   // the stencil kernels' form: one run per dz, or per (dz, dy) for long rows
@@ -955,7 +961,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   auto spmv_dir_box = [&](double *pold, double *pnew, int par, int first, int np_rz, double thr,
                           int itk) {
     auto kern = wide ? spmv_dir_box_kernel<true> : spmv_dir_box_kernel<false>;
-    hipLaunchKernelGGL(kern, dim3(g_box), dim3(kBlock), 3 * run_bytes, s, B, ntiles, c.a27.get(),
+    hipLaunchKernelGGL(kern, dim3(g_spmv), dim3(kBlock), 3 * run_bytes, s, B, ntiles, c.a27.get(),
                        V.z, pold, pnew, V.q, scal, par, first, part_rz, part_rr, np_rz, thr, itk,
                        news, part_pq);
   };
@@ -965,7 +971,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
                      : (start ? update_lower_box_kernel<false, true>
                               : update_lower_box_kernel<false, false>);
     hipLaunchKernelGGL(kern, dim3(g_box), dim3(kBlock), 2 * run_bytes, s, B, ntiles, par,
-                       c.g14.get(), V.x, rold, rnew, pnew, V.q, V.y, scal, part_pq, (int)g_box,
+                       c.g14.get(), V.x, rold, rnew, pnew, V.q, V.y, scal, part_pq, (int)g_spmv,
                        part_rr);
   };
   auto upper_box = [&](double *r) {
@@ -1101,18 +1107,19 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
 
 }  // namespace
 
-// Systems that the one-workgroup solve takes: at most 4096 rows, 49,152 entries and 64
-// entries a row on average.  Past the entries one compute unit streams too much of the
-// matrix (µs an iteration, one workgroup and general kernels: 3-D Q1 39,304 entries 7.5 and
-// 16.2, 50,653 14.6 and 16.3, 64,000 15.6 and 15.2); with longer rows a thread's serial
-// share is too long (3-D Q2 of 41 a row 9.8 and 14.2; vector Q2 of 110 a row and 38,124
-// entries 11.5 and 10.0).  GRIDAP_HIP_SMALL_PCG=0 switches it off, and so does choosing
-// between the other forms (GRIDAP_HIP_STENCIL_PCG).
-constexpr int64_t kSmallMaxNnz = 49152, kSmallMaxRow = 64;
+// Systems that the one-workgroup solve takes: at most 4096 rows, 40,960 entries and 64
+// entries a row on average, boxes 1536 rows.  Past the entries one compute unit streams too
+// much of the matrix (µs an iteration: 3-D Q1 39,304 entries 7.5, 50,653 14.6, 64,000 15.6,
+// where the general kernels take 10 to 12); with longer rows a thread's serial share is too
+// long (one workgroup and general kernels: 3-D Q2 of 41 a row 9.8 and 12.2; vector Q2 of
+// 110 a row and 38,124 entries 11.5 and 10.0); larger boxes fit the resident solve (1000
+// rows 182 and 252 µs a solve, 1728 297 and 284).  GRIDAP_HIP_SMALL_PCG=0 switches it off, and
+// so does choosing between the other forms (GRIDAP_HIP_STENCIL_PCG).
+constexpr int64_t kSmallMaxNnz = 40960, kSmallMaxRow = 64, kSmallMaxBox = 1536;
 bool small_system(const Ctx &c, int precond) {
   const char *off = std::getenv("GRIDAP_HIP_SMALL_PCG");
   return (precond == GH_PRECOND_NONE || precond == GH_PRECOND_JACOBI) && c.nfree > 0 &&
-         c.nfree <= kSmallMaxN && c.nnz <= kSmallMaxNnz &&
+         c.nfree <= (c.box ? kSmallMaxBox : kSmallMaxN) && c.nnz <= kSmallMaxNnz &&
          c.nnz <= kSmallMaxRow * c.nfree && !(off && off[0] == '0') &&
          !std::getenv("GRIDAP_HIP_STENCIL_PCG");
 }

@@ -27,11 +27,11 @@
 // and read past the exchange instead.
 //
 // Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.1, 31³
-// 11.9 and 6.8; FSAI 25.3 and 19.3, 17.5 and 12.4.  (Barriers for the published vectors
-// too: 10.7, 7.6, 22.6, 16.0.)  Rows past one a thread, in LDS: 65³ 19.6 and 16.2, 70³ 20.6
-// and 17.2.  What bounds it: the trips through the fabric, 3 to 4 µs an
-// exchange or published vector with 245 workgroups, 2 with 14.  Hence the largest
-// workgroups that fit, 512 rows at least (31³ with barriers: 256 rows 8.3, 512 7.1, 1024 7.3).
+// 11.9 and 6.8; FSAI 25.3 and 19.3, 17.5 and 12.4; rows past one a thread, in LDS: 65³ 19.6
+// and 16.2, 70³ 20.6 and 17.2.  (Barriers for the published vectors too: 10.7, 7.6, 22.6,
+// 16.0.)  What bounds it: the trips through the fabric, 3 to 4 µs an exchange or published
+// vector with 245 workgroups, 2 with 14.  Hence the largest workgroups that fit, 512 rows
+// at least (31³ with barriers: 256 rows 8.3, 512 7.1, 1024 7.3).
 //
 // Every wait ends: a workgroup that waits longer than kArrive for the first exchange (some
 // workgroups are not on the device: other work holds it) or kLost for a later one sets the
