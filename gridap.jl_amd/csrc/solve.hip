@@ -148,7 +148,10 @@ __device__ __forceinline__ bool iteration_stops(double *scal, uint64_t *news, do
   return stop;
 }
 
-constexpr unsigned kStencilGrid = 512;  // two workgroups on each of 256 compute units
+// Workgroups of the stencil product: two on each of 256 compute units, or one.  µs an
+// iteration with 1024, 512 and 256: 84³ -, 26.9 and 29.5; 100³ 44.6, 42.4 and -; 160² x 50
+// -, 55.8 and 56.7; 110³ -, 53.9 and 52.8; 140² x 80 -, 70.9 and 64.2; 128³ 98.0, 95.2 and 93.3.
+constexpr unsigned kStencilGrid = 512;
 
 inline unsigned grid_rows(int64_t rows, int rows_per_block) {
   return (unsigned)std::min<int64_t>(
@@ -949,15 +952,17 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   // the vector kernels: two entries per thread, one with the interleaved z and p
   const unsigned g_vec = grid_rows(box ? (n + 1) / 2 : n, kBlock);
   const unsigned g_box = grid_rows(n, kBlock);            // one tile per block and turn
-  // the stencil product: the two workgroups a compute unit holds, so that every slab is
-  // swept once in order (1024 of them, half waiting: 100³ 45.8 µs an iteration, now 43.9)
-  unsigned g_spmv = std::min(g_box, kStencilGrid);
+  // the stencil product: the two workgroups a compute unit holds, so that every slab is swept
+  // once in order; one where the matrix and the vectors (176 bytes a row) no longer stay in
+  // the 256 MB cache, so that less of a plane's mirrored coefficients leaves L2 before the
+  // plane needs them (kStencilGrid)
+  unsigned g_spmv = std::min(g_box, n * 176 > 224000000 ? kStencilGrid / 2 : kStencilGrid);
   if (!box) row_shape(c.nnz, n, [&](auto L, auto) { g_spmv = grid_rows(n, kBlock / L()); });
   const unsigned g_apply = box ? g_box : grid_rows(n, kBlock / kApplyLanes);
   // the stencil kernels' form: one run per dz, or per (dz, dy) for long rows
   const bool wide = B.m0 > kBlock;
-  const size_t run_bytes =
-      sizeof(double) * (wide ? 3 * Runs<true, 0, 1>::run_len(B.m0) : Runs<false, 0, 1>::run_len(B.m0));
+  const size_t run_bytes = sizeof(double) * (wide ? 3 * Runs<true, 0, 1>::run_len(B.m0)
+                                                  : Runs<false, 0, 1>::run_len(B.m0));
   auto spmv_dir_box = [&](double *pold, double *pnew, int par, int first, int np_rz, double thr,
                           int itk) {
     auto kern = wide ? spmv_dir_box_kernel<true> : spmv_dir_box_kernel<false>;
