@@ -817,6 +817,7 @@ int gh_pcg(gh_ctx *ctx, int precond, const double *b, double *x, double rtol, in
                GH_ERR_UNSUPPORTED, "unknown preconditioner");
     GH_REQUIRE(rtol > 0 && maxit >= 0, GH_ERR_ARG, "bad tolerance or iteration cap");
     size_t n = c.nfree;
+    c.solve_form = GH_SOLVE_NONE;
     c.s_x.resize(std::max<size_t>(n, 1));
     c.s_b.resize(std::max<size_t>(n, 1));
     gh::HostCopy copy(c);
@@ -858,10 +859,18 @@ int gh_pcg_noalloc(gh_ctx *ctx, int precond, const double *b, double *x, double 
     GH_REQUIRE(x, GH_ERR_ARG, "NULL solution vector");
     GH_REQUIRE(rtol > 0 && maxit >= 0, GH_ERR_ARG, "bad tolerance or iteration cap");
     gh_solve_stats local{};
+    c.solve_form = GH_SOLVE_NONE;
     gh::pcg_noalloc(c, precond, b, x, rtol, maxit, &local);
     if (stats) *stats = local;
     if (!local.converged)
       throw gh::Error(GH_ERR_NOCONV, "PCG did not reach the requested tolerance");
+  });
+}
+
+int gh_solve_form_get(gh_ctx *ctx, int32_t *form) {
+  return guarded(ctx, [&](gh::Ctx &c) {
+    GH_REQUIRE(form, GH_ERR_ARG, "NULL form");
+    *form = c.solve_form;
   });
 }
 

@@ -369,6 +369,7 @@ struct Ctx {
   DBuf<double> s_r, s_z, s_p, s_q, s_x, s_dinv, s_b, s_part, s_scal, s_y;
   DBuf<double> s_r2, s_p2;          // second buffers of r (factored M) and p
   DBuf<unsigned char> s_small;      // workspace of the one-launch solves
+  int32_t solve_form = 0;           // GH_SOLVE_* of the last solve
   // box lattice: the free dofs are all nodes of a box of box_m[0] x box_m[1] x box_m[2]
   // lattice nodes, numbered in node order (Q1, every boundary node outside the box
   // Dirichlet), so A is a 27-point stencil in dof space and PCG runs the stencil

@@ -1104,6 +1104,7 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
   } else {
     GH_CHECK_HIP(hipStreamSynchronize(s));
   }
+  c.solve_form = box ? GH_SOLVE_STENCIL : GH_SOLVE_ROWS;
   st->iterations = it;
   st->converged = converged ? 1 : 0;
   st->rel_residual = relres;

@@ -654,6 +654,7 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
     if (aborted || h[0] == kNone) return false;
     A.resume = 1;
   } while (h[0] == kPaused);
+  c.solve_form = GH_SOLVE_RESIDENT;
   st->iterations = (int)h[1];
   st->converged = h[2] != 0.0;
   st->rel_residual = h[3];

@@ -333,6 +333,7 @@ bool pcg_small(Ctx &c, HostCopy &copy, int precond, double rtol, int maxit, doub
     A.resume = 1;
   } while (h[3] == kPaused);
   if (h[3] == kDeclined) return false;
+  c.solve_form = GH_SOLVE_WORKGROUP;
   st->iterations = (int)h[0];
   st->converged = h[1] != 0.0;
   st->rel_residual = h[2];

@@ -38,6 +38,11 @@ GH_KERNEL_CELL = 2
 GH_KERNEL_COLUMN_SUM = 3
 GH_KERNEL_LIST_SUM = 4
 GH_KERNEL_Q2_LATTICE = 5
+GH_SOLVE_NONE = 0
+GH_SOLVE_ROWS = 1
+GH_SOLVE_STENCIL = 2
+GH_SOLVE_WORKGROUP = 3
+GH_SOLVE_RESIDENT = 4
 GH_PRECOND_NONE = 0
 GH_PRECOND_JACOBI = 1
 GH_PRECOND_FSAI = 2
@@ -94,6 +99,7 @@ SIGNATURES = {
     "gh_spmv": (_i32, [_vp, _vp, _vp]),
     "gh_pcg": (_i32, [_vp, _i32, _vp, _vp, _dbl, _i32, C.POINTER(SolveStats)]),
     "gh_pcg_noalloc": (_i32, [_vp, _i32, _vp, _vp, _dbl, _i32, C.POINTER(SolveStats)]),
+    "gh_solve_form_get": (_i32, [_vp, C.POINTER(_i32)]),
     "gh_mlp_nparams": (_i32, [_pi64]),
     "gh_mlp_init": (_i32, [_vp, C.c_uint64]),
     "gh_mlp_set": (_i32, [_vp, _vp, _i64]),
@@ -426,6 +432,12 @@ class Context:
         if code != GH_OK and (code != GH_ERR_NOCONV or raise_on_noconv):
             self.check(code)
         return x, st
+
+    def solve_form(self):
+        """Which form (GH_SOLVE_*) ended the last solve."""
+        form = C.c_int32()
+        self.check(lib().gh_solve_form_get(self.h, C.byref(form)))
+        return form.value
 
     # learned FSAI ------------------------------------------------------------
     @staticmethod

@@ -89,6 +89,13 @@ extern "C" {
 #define GH_PRECOND_FSAI 2 /* learned factorized sparse approximate inverse, M = GᵀG;
                              Jacobi-PCG is rerun from x0 if it fails to converge  */
 
+/* Forms of the solve (gh_solve_form_get). */
+#define GH_SOLVE_NONE 0      /* no solve yet, or the last one failed with an error     */
+#define GH_SOLVE_ROWS 1      /* CSR kernels, launched for every iteration              */
+#define GH_SOLVE_STENCIL 2   /* stencil kernels of a box lattice, launched likewise    */
+#define GH_SOLVE_WORKGROUP 3 /* small systems: one workgroup                           */
+#define GH_SOLVE_RESIDENT 4  /* box lattices: workgroups that stay on the device       */
+
 typedef struct gh_ctx gh_ctx;
 
 typedef struct gh_solve_stats {
@@ -323,6 +330,9 @@ int gh_pcg(gh_ctx *ctx, int precond, const double *b, double *x, double rtol, in
 #define GH_NOALLOC_MAX_N 262144
 int gh_pcg_noalloc(gh_ctx *ctx, int precond, const double *b, double *x, double rtol,
                    int maxit, gh_solve_stats *stats);
+/* Which form (GH_SOLVE_*) ended this context's last solve (diagnostic; no counterpart in
+ * Gridap). */
+int gh_solve_form_get(gh_ctx *ctx, int32_t *form);
 
 /* ---- learned FSAI preconditioner (3-D Cartesian mesh, scalar Q1) ----
  * No counterpart in Gridap (it ships LU only, src/Algebra/LinearSolvers.jl:249-303).

@@ -260,8 +260,10 @@ def test_stencil_pcg_matches_general_pcg(case, monkeypatch):
     for precond in (_lib.GH_PRECOND_JACOBI, _lib.GH_PRECOND_FSAI):
         monkeypatch.setenv("GRIDAP_HIP_STENCIL_PCG", "1")
         xs, ss = ctx.pcg(precond=precond, rtol=1e-10)
+        assert ctx.solve_form() == _lib.GH_SOLVE_STENCIL
         monkeypatch.setenv("GRIDAP_HIP_STENCIL_PCG", "0")
         xg, sg = ctx.pcg(precond=precond, rtol=1e-10)
+        assert ctx.solve_form() == _lib.GH_SOLVE_ROWS
         assert ss.converged == 1 and sg.converged == 1
         assert ss.precond_used == precond and sg.precond_used == precond
         assert abs(ss.iterations - sg.iterations) <= 1

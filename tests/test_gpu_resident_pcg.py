@@ -47,15 +47,34 @@ def system(part, spread=1.0):
 def launched(monkeypatch, ctx, **kw):
     with monkeypatch.context() as m:
         m.setenv("GRIDAP_HIP_RESIDENT_PCG", "0")
-        return ctx.pcg(**kw)
+        r = ctx.pcg(**kw)
+    assert ctx.solve_form() == _lib.GH_SOLVE_STENCIL
+    return r
+
+
+def resident(ctx, **kw):
+    r = ctx.pcg(**kw)
+    assert ctx.solve_form() == _lib.GH_SOLVE_RESIDENT
+    return r
+
+
+def fits(part, precond):
+    """Rows a workgroup (256 compute units): at most 1024 with FSAI, else what LDS holds of
+    the vector's three runs and 32 values of each row past 1024."""
+    m0, n = part[0] - 1, int(np.prod([p - 1 for p in part]))
+    rows = max(-(-(-(-n // 256)) // 64) * 64, 512)
+    if precond == _lib.GH_PRECOND_FSAI:
+        return rows <= 1024 and 7 * (rows + 2 * m0 + 2) <= 150 * 128
+    return max(3 * (rows + 2 * m0 + 2), 3456) + 32 * max(rows - 1024, 0) <= 150 * 128
 
 
 # free rows: 1, 2, 40, 512, 528, 8 long lattice rows, 16 x 15 x 1025, 64 x 64 x 63 = 258,048
 # (1024 a workgroup), 64^3 = 262,144, 65 x 64 x 63 = 262,080, 64 x 65 x 64 past one row a
-# thread (FSAI's largest), 71 x 70 x 69 and 72 x 70 x 72 around the most that LDS holds
+# thread (FSAI's largest), 71 x 70 x 69 and 72 x 70 x 72 up to the most that LDS holds, and
+# 74 x 72 x 72 past it
 PARTS = [(2, 2, 2), (3, 2, 2), (2, 6, 9), (33, 17, 2), (34, 17, 2), (514, 3, 3), (1100, 4, 5),
          (17, 16, 1026), (65, 65, 64), (65, 65, 65), (66, 65, 64), (65, 66, 65),
-         (72, 71, 70), (73, 71, 73)]
+         (72, 71, 70), (73, 71, 73), (75, 73, 73)]
 
 
 @pytest.mark.parametrize("part", PARTS)
@@ -68,6 +87,8 @@ def test_matches_launched_kernels(part, monkeypatch):
     for precond in PRECONDS:
         kw = dict(x0=x0, precond=precond, rtol=1e-10, maxit=5000)
         x, st = ctx.pcg(**kw)
+        assert ctx.solve_form() == (_lib.GH_SOLVE_RESIDENT if fits(part, precond)
+                                    else _lib.GH_SOLVE_STENCIL)
         y, sy = launched(monkeypatch, ctx, **kw)
         assert st.converged and sy.converged
         assert abs(st.iterations - sy.iterations) <= max(1, 0.01 * sy.iterations)
@@ -87,26 +108,26 @@ def test_limits_and_exact_starts(monkeypatch):
     b = op.get_vector()
     FS.LearnedFSAI.load(FS.DEFAULT_WEIGHTS).attach(ctx)
     for precond in PRECONDS:
-        x, _ = ctx.pcg(precond=precond, rtol=1e-10)
+        x, _ = resident(ctx, precond=precond, rtol=1e-10)
         for maxit in (0, 1, 5):
             kw = dict(precond=precond, rtol=1e-10, maxit=maxit, raise_on_noconv=False)
-            got, s1 = ctx.pcg(**kw)
+            got, s1 = resident(ctx, **kw)
             ref, s2 = launched(monkeypatch, ctx, **kw)
             # (FSAI that ends at its limit is followed by as many Jacobi iterations)
             assert s1.iterations == s2.iterations and not s1.converged
             assert s1.iterations == maxit * (2 if precond == _lib.GH_PRECOND_FSAI else 1)
             np.testing.assert_allclose(got, ref, rtol=1e-10, atol=1e-13 * abs(ref).max())
-        y, s3 = ctx.pcg(x0=x, precond=precond, rtol=1e-8)
+        y, s3 = resident(ctx, x0=x, precond=precond, rtol=1e-8)
         assert s3.iterations == 0 and np.array_equal(x, y)
-        zero, s4 = ctx.pcg(b=np.zeros_like(b), precond=precond, rtol=1e-8)
+        zero, s4 = resident(ctx, b=np.zeros_like(b), precond=precond, rtol=1e-8)
         assert s4.converged and s4.iterations == 0 and not zero.any()
         # below what FP64 reaches: the restarts run out
-        _, s5 = ctx.pcg(precond=precond, rtol=1e-30, maxit=3000, raise_on_noconv=False)
+        _, s5 = resident(ctx, precond=precond, rtol=1e-30, maxit=3000, raise_on_noconv=False)
         assert not s5.converged
     nz, _ = ctx.values_get()
     nz[3] = np.nan
     ctx.values_set(nz)
-    _, s6 = ctx.pcg(rtol=1e-8, maxit=50, raise_on_noconv=False)
+    _, s6 = resident(ctx, rtol=1e-8, maxit=50, raise_on_noconv=False)
     assert not s6.converged
 
 
@@ -118,7 +139,7 @@ def test_solve_over_several_launches(monkeypatch):
     op, ctx = system((40, 40, 2), spread=4.0)
     A, b = op.get_matrix().to_scipy(), op.get_vector()
     kw = dict(rtol=1e-8, maxit=60000, precond=_lib.GH_PRECOND_NONE)
-    x, st = ctx.pcg(**kw)
+    x, st = resident(ctx, **kw)
     _, sy = launched(monkeypatch, ctx, **kw)
     assert st.converged and sy.converged
     assert st.iterations > 2048 and abs(st.iterations - sy.iterations) <= 0.05 * sy.iterations
@@ -126,16 +147,17 @@ def test_solve_over_several_launches(monkeypatch):
 
 
 def test_two_threads():
-    """Two contexts solve at once: one holds the device's turn, the other takes the
-    launched kernels; both are right."""
+    """Two contexts solve at once: whichever finds the device's turn taken runs the launched
+    kernels; both are right."""
     print("[gpu-case] resident PCG: two threads", flush=True)
     systems = [system((33, 30, 31)), system((40, 28, 26))]
-    refs = [ctx.pcg(rtol=1e-10)[0] for _, ctx in systems]
-    err = [None, None]
+    refs = [resident(ctx, rtol=1e-10)[0] for _, ctx in systems]
+    err, forms = [None, None], set()
 
     def work(k):
         for _ in range(4):
             x, st = systems[k][1].pcg(rtol=1e-10)
+            forms.add(systems[k][1].solve_form())
             e = np.linalg.norm(x - refs[k]) / np.linalg.norm(refs[k])
             err[k] = max(err[k] or 0.0, e if st.converged else np.inf)
 
@@ -143,3 +165,5 @@ def test_two_threads():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert max(err) <= 1e-6
+    assert _lib.GH_SOLVE_RESIDENT in forms  # the first to find the turn free
+    assert forms <= {_lib.GH_SOLVE_RESIDENT, _lib.GH_SOLVE_STENCIL}

@@ -33,6 +33,19 @@ class env:
                 os.environ[k] = v
 
 
+def small(ctx, **kw):
+    r = ctx.pcg(**kw)
+    assert ctx.solve_form() == _lib.GH_SOLVE_WORKGROUP
+    return r
+
+
+def general(ctx, **kw):
+    with env(GRIDAP_HIP_SMALL_PCG="0", GRIDAP_HIP_RESIDENT_PCG="0"):
+        r = ctx.pcg(**kw)
+    assert ctx.solve_form() in (_lib.GH_SOLVE_ROWS, _lib.GH_SOLVE_STENCIL)
+    return r
+
+
 def system(D, part, order=1, ncomp=1, tags="boundary", seed=0, spread=0.5):
     model = G.CartesianDiscreteModel((0, 1) * D, part)
     T = G.VectorValue[D, G.Float64] if ncomp > 1 else G.Float64
@@ -66,15 +79,18 @@ def test_matches_general_kernels(case):
     n = S.shape[0]
     rng = np.random.default_rng(n)
     b, x0 = rng.standard_normal(n), rng.standard_normal(n)
+    fits = (n <= (1536 if ctx.pattern_info()["box"] else 4096) and S.nnz <= 40960 and
+            S.nnz <= 64 * n)
     for precond in (_lib.GH_PRECOND_JACOBI, _lib.GH_PRECOND_NONE):
         x, st = ctx.pcg(b=b, x0=x0, precond=precond, rtol=1e-10)
-        with env(GRIDAP_HIP_SMALL_PCG="0"):
-            y, sy = ctx.pcg(b=b, x0=x0, precond=precond, rtol=1e-10)
+        assert (ctx.solve_form() == _lib.GH_SOLVE_WORKGROUP) == fits
+        y, sy = general(ctx, b=b, x0=x0, precond=precond, rtol=1e-10)
         assert st.converged and sy.converged and abs(st.iterations - sy.iterations) <= 1
         assert np.linalg.norm(b - S @ x) <= 1.01e-10 * np.linalg.norm(b)
         assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
         z, sz = ctx.pcg_noalloc(b=b, x0=x0, precond=precond, rtol=1e-10)
-        if S.nnz <= 40960 and S.nnz <= 64 * n:  # the same kernel, on other buffers
+        assert ctx.solve_form() == (_lib.GH_SOLVE_WORKGROUP if fits else _lib.GH_SOLVE_ROWS)
+        if fits:  # the same kernel, on other buffers
             np.testing.assert_array_equal(x, z)
         assert np.linalg.norm(x - z) <= 1e-6 * np.linalg.norm(x)
         assert abs(sz.iterations - st.iterations) <= 1
@@ -89,28 +105,26 @@ def test_limits_and_exact_starts():
     A, ctx, _ = system(2, (20, 17))
     S = A.to_scipy()
     b = np.random.default_rng(4).standard_normal(S.shape[0])
-    x, st = ctx.pcg(b=b, rtol=1e-10)
+    x, st = small(ctx, b=b, rtol=1e-10)
     for maxit in (0, 1, 7):
-        got, s1 = ctx.pcg(b=b, rtol=1e-10, maxit=maxit, raise_on_noconv=False)
-        with env(GRIDAP_HIP_SMALL_PCG="0"):
-            ref, s2 = ctx.pcg(b=b, rtol=1e-10, maxit=maxit, raise_on_noconv=False)
+        got, s1 = small(ctx, b=b, rtol=1e-10, maxit=maxit, raise_on_noconv=False)
+        ref, s2 = general(ctx, b=b, rtol=1e-10, maxit=maxit, raise_on_noconv=False)
         assert s1.iterations == s2.iterations == maxit and not s1.converged
         np.testing.assert_allclose(got, ref, rtol=1e-10, atol=1e-14)
         assert abs(s1.rel_residual - s2.rel_residual) <= 1e-10 * s2.rel_residual
-    y, s3 = ctx.pcg(b=b, x0=x, rtol=1e-8)
+    y, s3 = small(ctx, b=b, x0=x, rtol=1e-8)
     assert s3.iterations == 0 and np.array_equal(x, y)
-    zero, s4 = ctx.pcg(b=np.zeros_like(b), rtol=1e-8)
+    zero, s4 = small(ctx, b=np.zeros_like(b), rtol=1e-8)
     assert s4.converged and s4.iterations == 0 and not zero.any()
     # a tolerance below what FP64 reaches: restarts run out, as in the general form
-    _, s5 = ctx.pcg(b=b, rtol=1e-30, maxit=5000, raise_on_noconv=False)
-    with env(GRIDAP_HIP_SMALL_PCG="0"):
-        _, s6 = ctx.pcg(b=b, rtol=1e-30, maxit=5000, raise_on_noconv=False)
+    _, s5 = small(ctx, b=b, rtol=1e-30, maxit=5000, raise_on_noconv=False)
+    _, s6 = general(ctx, b=b, rtol=1e-30, maxit=5000, raise_on_noconv=False)
     assert not s5.converged and not s6.converged
     # a matrix that is not finite ends like there
     nz, _ = ctx.values_get()
     nz[3] = np.nan
     ctx.values_set(nz)
-    _, s7 = ctx.pcg(b=b, rtol=1e-8, maxit=50, raise_on_noconv=False)
+    _, s7 = small(ctx, b=b, rtol=1e-8, maxit=50, raise_on_noconv=False)
     assert not s7.converged
 
 
@@ -122,9 +136,8 @@ def test_solve_over_several_launches():
     A, ctx, _ = system(2, (40, 40), spread=4.0)
     S = A.to_scipy()
     b = np.random.default_rng(4).standard_normal(S.shape[0])
-    x, st = ctx.pcg(b=b, rtol=1e-8, maxit=60000, precond=_lib.GH_PRECOND_NONE)
-    with env(GRIDAP_HIP_SMALL_PCG="0"):
-        _, sy = ctx.pcg(b=b, rtol=1e-8, maxit=60000, precond=_lib.GH_PRECOND_NONE)
+    x, st = small(ctx, b=b, rtol=1e-8, maxit=60000, precond=_lib.GH_PRECOND_NONE)
+    _, sy = general(ctx, b=b, rtol=1e-8, maxit=60000, precond=_lib.GH_PRECOND_NONE)
     assert st.converged and sy.converged
     assert st.iterations > 8192 and abs(st.iterations - sy.iterations) <= 0.05 * sy.iterations
     assert np.linalg.norm(b - S @ x) <= 1.01e-8 * np.linalg.norm(b)
@@ -159,10 +172,10 @@ def test_uneven_rows_are_declined():
     ctx.reffe_tabulation(q.weights, shp, grad)
     ctx.symbolic()
     ctx.assemble()
-    assert ctx.nfree <= 4096
+    assert ctx.nfree <= 4096 and ctx.nnz <= 40960
     x, st = ctx.pcg(rtol=1e-10)
-    with env(GRIDAP_HIP_SMALL_PCG="0"):
-        y, sy = ctx.pcg(rtol=1e-10)
+    assert ctx.solve_form() == _lib.GH_SOLVE_ROWS  # declined by the kernel, not by the rule
+    y, sy = general(ctx, rtol=1e-10)
     assert st.converged and abs(st.iterations - sy.iterations) <= 1
     np.testing.assert_allclose(x, y, rtol=1e-7, atol=1e-12)
     ctx.close()

@@ -43,7 +43,8 @@ CASES = [
 
 
 @pytest.mark.parametrize("case", CASES)
-def test_row_kernels(case):
+def test_row_kernels(case, monkeypatch):
+    monkeypatch.setenv("GRIDAP_HIP_STENCIL_PCG", "0")  # the CSR kernels, whatever the size
     print("[gpu-case] CSR rows %s" % (case,), flush=True)
     _, A, assem = _operator(*case)
     S = A.to_scipy()
@@ -54,6 +55,7 @@ def test_row_kernels(case):
     b = rng.standard_normal(S.shape[0])
     for precond in (_lib.GH_PRECOND_NONE, _lib.GH_PRECOND_JACOBI):
         u, st = assem.ctx.pcg(b=b, precond=precond, rtol=1e-10)
+        assert assem.ctx.solve_form() == _lib.GH_SOLVE_ROWS
         assert np.linalg.norm(b - S @ u) <= 1.01e-10 * np.linalg.norm(b), st.rel_residual
 
 

@@ -53,7 +53,9 @@ def test_stencil_and_csr_forms_agree(part):
     FS.LearnedFSAI.load(FS.DEFAULT_WEIGHTS).attach(ctx)
     for precond in (_lib.GH_PRECOND_NONE, _lib.GH_PRECOND_JACOBI, _lib.GH_PRECOND_FSAI):
         x, st = solve(ctx, precond, "1")
+        assert ctx.solve_form() == _lib.GH_SOLVE_STENCIL
         y, sy = solve(ctx, precond, "0")
+        assert ctx.solve_form() == _lib.GH_SOLVE_ROWS
         assert abs(st.iterations - sy.iterations) <= 1
         assert np.linalg.norm(b - A @ x) <= 1e-10 * np.linalg.norm(b)
         assert np.linalg.norm(x - y) <= 1e-7 * np.linalg.norm(y)
