@@ -59,7 +59,7 @@ constexpr double kNone = 0, kDone = 1, kPaused = 2;
 
 struct ResidentArgs {
   Box B;
-  int rb, maxit, jacobi, resume;
+  int rb, maxit, jacobi, resume, pause;  // pause: most iterations of this launch
   double rtol;
   const int32_t *cp;
   const double *val, *b;
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     empty(true);
   }
   H.issue(W, zbuf(turn), -1);
-  const int until = A.maxit - it > kPause ? it + kPause : A.maxit;
+  const int until = A.maxit - it > A.pause ? it + A.pause : A.maxit;
   // each turn multiplies by A once: a step of the recurrence, or (start) the true residual
   for (;;) {
     pi = start ? xi : first ? zi : zi + beta * pi;
@@ -515,16 +515,17 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     }
     if (!start && it >= until) {
       how = kPaused;
+      if (first) beta = 0.0;  // right after a restart the next p is z: pi still holds x
       if (own) {
         const int j = W.i0 + fresh(t);
         A.r[j] = ri;
-        A.p[j] = pi;
+        A.p[j] = first ? 0.0 : pi;
         A.z[j] = zi;
       }
       if (own2) {
         const int e = fresh(t), j = W.i0 + e + bd;
         A.r[j] = rs[e];
-        A.p[j] = ps[e];
+        A.p[j] = first ? 0.0 : ps[e];
         A.z[j] = zs[e];
       }
       break;
@@ -619,6 +620,9 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
   A.rb = S.rb;
   A.maxit = maxit;
   A.jacobi = precond == GH_PRECOND_JACOBI;
+  A.pause = kPause;
+  if (const char *env = std::getenv("GRIDAP_HIP_RESIDENT_PAUSE"))
+    A.pause = std::min(std::max(std::atoi(env), 1), kPause);
   A.rtol = rtol;
   A.cp = c.colptr.get();
   A.val = c.nzval.get();

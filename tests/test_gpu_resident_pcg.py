@@ -146,6 +146,28 @@ def test_solve_over_several_launches(monkeypatch):
     assert np.linalg.norm(b - A @ x) <= 1.01e-8 * np.linalg.norm(b)
 
 
+# one row a thread and rows past it in LDS
+@pytest.mark.parametrize("part", [(20, 18, 17), (66, 65, 66)])
+def test_pauses_leave_no_trace(part, monkeypatch):
+    """A launch that ends after every iteration, or every third, gives the bits of an
+    undivided solve, also where it ends right after a restart: the tolerance is one that
+    only the recurrence's r reaches, so that every solve restarts until it may no more."""
+    print("[gpu-case] resident PCG: pauses %s" % (part,), flush=True)
+    _, ctx = system(part)
+    FS.LearnedFSAI.load(FS.DEFAULT_WEIGHTS).attach(ctx)
+    for precond in PRECONDS:
+        if not fits(part, precond):
+            continue
+        kw = dict(precond=precond, rtol=1e-30, maxit=1200, raise_on_noconv=False)
+        x, st = resident(ctx, **kw)
+        for pause in ("1", "3"):
+            with monkeypatch.context() as m:
+                m.setenv("GRIDAP_HIP_RESIDENT_PAUSE", pause)
+                y, sy = resident(ctx, **kw)
+            assert (st.iterations, st.rel_residual) == (sy.iterations, sy.rel_residual)
+            np.testing.assert_array_equal(x, y)
+
+
 def test_two_threads():
     """Two contexts solve at once: whichever finds the device's turn taken runs the launched
     kernels; both are right."""
