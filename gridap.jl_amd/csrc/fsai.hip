@@ -305,13 +305,15 @@ __global__ __launch_bounds__(kFwdWaves * 64) void mlp_fwd_mfma(const float *__re
 // lane's 16 operands are contiguous, in LDS and in the BF16 weights (read from L1).
 // The backward kernel recomputes the activations from the features: it reads 64 B
 // of features and 160 B of output gradient per cell and keeps the rest in LDS, and each
-// workgroup writes one partial of every gradient.  Bound by the matrix cores at large
+// workgroup writes one partial of every gradient; an FP32 sum covers at most 256 cells
+// however large the mesh (kRunTiles).  Bound by the matrix cores at large
 // C (560 instructions of 32 cycles per tile and wave), by the number of tiles below
 // 256 tiles.  One lane per unit and 256 cells in turn left 128 waves for the whole chip:
 // 32³ cells 1,480 µs for forward, backward, gradients and their sums; now 20 + 58 + 9 µs.
 constexpr int kTrainCells = 64;
 constexpr int kTrainLd = kMlpHidden + 4;   // row stride of activations: conflict-free b128
 constexpr int kTrainGrid = 256;            // most workgroups of the backward (partials)
+constexpr int kRunTiles = 4;               // most tiles that one FP32 gradient sum covers
 
 struct TrainLds {
   float h[3][kTrainCells][kTrainLd];   // activations, then (backward) pre-activation gradients
@@ -449,7 +451,13 @@ struct TrainWeights {
   uint16_t w2t[kMlpHidden][kWtLd], w3t[kMlpHidden][kWtLd], w4t[kMlpHidden][kWt4Ld];
 };
 
-// Partial gradients of every weight: one kMlpParams run per workgroup.
+// Partial gradients of every weight: one kMlpParams run per workgroup.  LONG, for workgroups
+// of more than kRunTiles tiles: every kRunTiles tiles the FP32 sums go to FP64 ones, in
+// registers (74 of the 512 of one wave on a SIMD) and, W2's, in LDS (a thread's own; all in
+// registers spill).  Step at 64³ and 96³: FP32 throughout 0.768 and 2.452 ms with gradient
+// errors of 4e-8 and 6e-8 of the FP64 evaluation, LONG 0.782 and 2.502 ms and 3e-8 at both; a
+// partial for every run 0.800 and 2.568 ms, a workgroup for every run 0.815 and 2.664.
+template <bool LONG>
 __global__ __launch_bounds__(256) void mlp_train_bwd(const float *__restrict__ feat,
                                                      const uint16_t *__restrict__ wq,
                                                      const float *__restrict__ dy, int C,
@@ -474,6 +482,40 @@ __global__ __launch_bounds__(256) void mlp_train_bwd(const float *__restrict__ f
     if (t < 3) aw4[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   }
   float ab2 = 0.0f, ab3 = 0.0f, ab4[3] = {0.0f, 0.0f, 0.0f};
+  // LONG: the same in FP64 over the runs so far (entry e of W2's at sw2[256 e])
+  double sw1[4] = {}, sw3[4][4] = {}, sw4[3][4] = {}, sb2 = 0.0, sb3 = 0.0, sb4[3] = {};
+  double *sw2 = reinterpret_cast<double *>(lds_raw + sizeof(TrainLds) + sizeof(TrainWeights)) +
+                threadIdx.x;
+  if (LONG)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sw2[256 * e] = 0.0;
+  auto end_run = [&] {
+    auto move = [](float a, double &s) { s += (double)a; };
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      move(aw1[j], sw1[j]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        move(aw2[t][j], sw2[256 * (4 * t + j)]);
+        move(aw3[t][j], sw3[t][j]);
+        if (t < 3) move(aw4[t][j], sw4[t][j]);
+      }
+    }
+    move(ab2, sb2);
+    move(ab3, sb3);
+    aw1 = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    ab2 = ab3 = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      aw2[t] = aw3[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+      if (t < 3) {
+        aw4[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        move(ab4[t], sb4[t]);
+        ab4[t] = 0.0f;
+      }
+    }
+  };
+  int tiles = 0;
   float gd[3][16];
   // contraction step s of a weight gradient: the cell of lane group g (rows four apart,
   // so the groups of a half-wave read different banks)
@@ -571,16 +613,35 @@ __global__ __launch_bounds__(256) void mlp_train_bwd(const float *__restrict__ f
       const int c = cell_of(s);
       aw1 = mfma4(S.h[0][c][16 * wave + l16], S.ft[c][l16], aw1);
     }
+    if (LONG && ++tiles % kRunTiles == 0) end_run();
   }
   // bias sums over the lane groups
-  auto groups = [](float v) {
+  auto groups = [](auto v) {
     v += __shfl_xor(v, 16);
     return v + __shfl_xor(v, 32);
   };
-  ab2 = groups(ab2);
-  ab3 = groups(ab3);
+  if constexpr (LONG) {
+    end_run();
 #pragma unroll
-  for (int t = 0; t < 3; ++t) ab4[t] = groups(ab4[t]);
+    for (int j = 0; j < 4; ++j) {
+      aw1[j] = (float)sw1[j];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        aw2[t][j] = (float)sw2[256 * (4 * t + j)];
+        aw3[t][j] = (float)sw3[t][j];
+        if (t < 3) aw4[t][j] = (float)sw4[t][j];
+      }
+    }
+    ab2 = (float)groups(sb2);
+    ab3 = (float)groups(sb3);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) ab4[t] = (float)groups(sb4[t]);
+  } else {
+    ab2 = groups(ab2);
+    ab3 = groups(ab3);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) ab4[t] = groups(ab4[t]);
+  }
   float *pp = part + (size_t)blockIdx.x * kMlpParams;
   if (g == 0) {
     pp[kMlpB2 + 16 * wave + l16] = ab2;
@@ -1196,8 +1257,13 @@ double fsai_train_step(Ctx &c, int nprobes, uint64_t seed, float lr) {
                      c.gl.get(), c.dy.get());
   GH_CHECK_HIP(hipGetLastError());
   // back-propagation (weights are the BF16 values the forward pass used), Adam
-  hipLaunchKernelGGL(mlp_train_bwd, dim3(nb), dim3(256), sizeof(TrainLds) + sizeof(TrainWeights),
-                     s, c.feat.get(), c.params_bf16.get(), c.dy.get(), C, c.wpart.get());
+  const bool many = C > kTrainGrid * kRunTiles * kTrainCells;
+  auto bwd = many ? mlp_train_bwd<true> : mlp_train_bwd<false>;
+  const size_t bwd_lds = sizeof(TrainLds) + sizeof(TrainWeights) + (many ? 16 * 256 * 8 : 0);
+  GH_CHECK_HIP(hipFuncSetAttribute((const void *)bwd, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)bwd_lds));
+  hipLaunchKernelGGL(bwd, dim3(nb), dim3(256), bwd_lds, s, c.feat.get(), c.params_bf16.get(),
+                     c.dy.get(), C, c.wpart.get());
   float b1t = 0.0f, b2t = 0.0f;
   if (lr > 0.0f) {
     ++c.adam_t;

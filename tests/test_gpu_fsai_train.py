@@ -1,10 +1,10 @@
 """The training step of the learned FSAI at the edges of its tiles and batches, against
 an FP64 PyTorch evaluation of the same step (needs an MI355X).
 
-The device keeps activations, their gradients and the weight sums in FP32 (FP64 where
-the partials of the workgroups meet); weights are the same BF16 values on both sides.  A
-contraction has at most 64 terms and a weight sum at most 64 per tile, so a gradient
-carries a few 1e-7 relative; the network is three layers deep and the pattern gradient
+The device keeps activations, their gradients and the weight sums in FP32 (FP64 from 256
+cells on: between a workgroup's runs of four tiles, and where the partials of the workgroups
+meet); weights are the same BF16 values on both sides.  A contraction has at most 64 terms
+and a weight sum in FP32 at most 256, so a gradient carries a few 1e-7 relative; the network is three layers deep and the pattern gradient
 is rounded to FP32 once: 2e-5 (relative L2 per layer) bounds it, and 1e-6 the loss, whose
 factor entries are rounded to FP32.
 """
@@ -73,6 +73,32 @@ def reference(ctx, part, kappa, params, seed, m):
     return out.detach().numpy(), float(loss.detach()), g.numpy()
 
 
+# W1, b1, W2, b2, W3, b3, W4, b4 in the flat parameters
+LAYERS = ((0, 640), (640, 704), (704, 4800), (4800, 4864), (4864, 8960), (8960, 9024),
+          (9024, 11328), (11328, 11364))
+
+
+@pytest.mark.parametrize("part,bounds", [
+    # what kernels with FP32 sums of 256 cells for every partial had on this very input
+    ((64, 64, 64), (3.6e-8, 2.9e-8, 3.3e-8, 3.1e-8, 3.5e-8, 2.9e-8, 4.1e-8, 4.2e-8)),
+    # one FP32 rounding of every gradient (with sums of 3456 cells W2 had 6.7e-8)
+    ((96, 96, 96), (2.0 ** -24,) * 8)])
+def test_many_tiles_a_workgroup(part, bounds):
+    """16 and 54 tiles a workgroup of the backward: the error of the gradients does not grow
+    with the mesh."""
+    print("[gpu-case] fsai training step %s, many tiles" % (part,), flush=True)
+    kappa = np.exp(np.random.default_rng(2).normal(size=int(np.prod(part))))
+    ctx = make_context(part, kappa)
+    params = random_params(2, scale4=0.05)
+    ctx.mlp_set(params)
+    ctx.fsai_train_step(2, 4321, 0.0)
+    got = ctx.fsai_get()["grad"]
+    _, _, g = reference(ctx, part, kappa, params, 4321, 2)
+    for (lo, hi), bound in zip(LAYERS, bounds):
+        assert np.linalg.norm(got[lo:hi] - g[lo:hi]) <= bound * np.linalg.norm(g[lo:hi]), lo
+    ctx.close()
+
+
 @pytest.mark.parametrize("part,probes", CASES)
 def test_step_matches_fp64(part, probes):
     print("[gpu-case] fsai training step %s, %d probes" % (part, probes), flush=True)
@@ -87,8 +113,7 @@ def test_step_matches_fp64(part, probes):
     out, ref, g = reference(ctx, part, kappa, params, 4321, probes)
     assert np.abs(got["yout"][:, :36] - out).max() <= 1e-5 * np.abs(out).max()
     assert abs(loss - ref) <= 1e-6 * ref
-    for lo, hi in ((0, 640), (640, 704), (704, 4800), (4800, 4864), (4864, 8960), (8960, 9024),
-                   (9024, 11328), (11328, 11364)):
+    for lo, hi in LAYERS:
         err = np.linalg.norm(got["grad"][lo:hi] - g[lo:hi]) / np.linalg.norm(g[lo:hi])
         assert err <= 2e-5, (lo, err)
     # lr = 0 leaves the solver's factor of these weights; a step leaves none
