@@ -59,6 +59,25 @@ def test_row_kernels(case, monkeypatch):
         assert np.linalg.norm(b - S @ u) <= 1.01e-10 * np.linalg.norm(b), st.rel_residual
 
 
+@pytest.mark.parametrize("case", CASES)
+def test_infinite_entries(case):
+    """One ±Inf in x: the rows that hold its column are infinite (NaN where the stored value
+    is 0), whatever their length is to the turn of their lanes."""
+    print("[gpu-case] CSR rows, infinite entry %s" % (case,), flush=True)
+    _, A, assem = _operator(*case)
+    S = A.to_scipy().tocsr()
+    rng = np.random.default_rng(5)
+    for j in sorted({0, S.shape[0] - 1, *rng.integers(S.shape[0], size=6)}):
+        x = rng.standard_normal(S.shape[0])
+        x[j] = rng.choice([np.inf, -np.inf])
+        y, ref = assem.ctx.spmv(x), S @ x
+        fin = np.isfinite(ref)
+        assert not fin.all()
+        np.testing.assert_array_equal(y[~fin], ref[~fin])
+        x[j] = 0.0
+        assert np.all(np.abs((y - ref)[fin]) <= 1e-13 * (abs(S) @ np.abs(x))[fin])
+
+
 def test_one_long_row_among_short_ones():
     """A vertex shared by 300 tetrahedra: its row holds every column, the others seven."""
     print("[gpu-case] CSR rows, fan mesh", flush=True)
