@@ -11,10 +11,12 @@
 // workspace from which the wave streams them every iteration (10 bytes an entry,
 // coalesced).  Bound by the LDS reads of p and the three barriers while the matrix fits the
 // registers, else by what one compute unit draws from L2.  Microseconds an iteration, start-up
-// included, here and in the general kernels: 2-D Q1 1024 rows 3.2 and 10.2, 4096 rows 4.6
+// included, here and in the general kernels: 2-D Q1 1024 rows 3.2 and 10.2, 4096 rows 4.4
 // and 9.4; 3-D Q1 729 rows 5.7 and 15.7, 1728 rows 7.5 and 16.2; scalar Q2 729 rows 9.8
 // and 14.2.  (1024 threads and sums through LDS permutes took 6.8 for the first: twice the
-// waves at each barrier, half the registers.)
+// waves at each barrier, half the registers.)  No form spills registers: gh_pcg_noalloc runs
+// them, and the runtime would back scratch with device memory.  (Nine entries with eight rows
+// a thread, 20 registers spilled: 4.3 µs at 2070 rows for 3.8 now, 4.25 at 4096 for 4.4.)
 // Both dot products sum in a fixed order: the result is the same every time.
 // One launch runs at most kPause iterations: past them the state goes to the workspace and
 // the next launch takes it up, so that a solve that never ends on its own does not hold the
@@ -328,7 +330,7 @@ bool pcg_small(Ctx &c, HostCopy &copy, int precond, double rtol, int maxit, doub
     if (n <= kT) launch<1, 60>(A, c.stream);
     else if (n <= 2 * kT) launch<2, 32>(A, c.stream);
     else if (n <= 4 * kT) launch<4, 18>(A, c.stream);
-    else launch<8, 9>(A, c.stream);
+    else launch<8, 8>(A, c.stream);
     copy.down(h, A.out, sizeof(h));
     A.resume = 1;
   } while (h[3] == kPaused);
