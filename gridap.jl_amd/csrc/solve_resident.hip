@@ -59,7 +59,7 @@ constexpr double kNone = 0, kDone = 1, kPaused = 2;
 
 struct ResidentArgs {
   Box B;
-  int rb, maxit, jacobi, resume, pause;  // pause: most iterations of this launch
+  int rb, maxit, jacobi, resume;
   double rtol;
   const int32_t *cp;
   const double *val, *b;
@@ -69,7 +69,7 @@ struct ResidentArgs {
   // {kNone, kDone or kPaused, iterations, converged, relative residual; a paused solve's
   //  rz, beta, threshold, restarts}
   double *out;
-  uint32_t *abort;
+  uint32_t *abort;  // the abort word, then the most iterations of this launch
   uint64_t *slots;  // [kSets][kMaxWords][kMaxBlocks]
 };
 
@@ -419,7 +419,9 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     empty(true);
   }
   H.issue(W, zbuf(turn), -1);
-  const int until = A.maxit - it > A.pause ? it + A.pause : A.maxit;
+  // (from memory: as an argument of the kernel it costs registers, 2% of every iteration)
+  const int pause = __builtin_amdgcn_readfirstlane((int)A.abort[1]);
+  const int until = A.maxit - it > pause ? it + pause : A.maxit;
   // each turn multiplies by A once: a step of the recurrence, or (start) the true residual
   for (;;) {
     pi = start ? xi : first ? zi : zi + beta * pi;
@@ -476,6 +478,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
       thr = lane_value((A.rtol * bnorm) * (A.rtol * bnorm), 0);
       first = true;
       start = false;
+      beta = 0.0;  // for a pause right here: the next p is z, p itself still holds x
     } else {
       double pq[1] = {pi * q};
       if (own2) pq[0] += ps[fresh(t)] * q2;
@@ -515,17 +518,16 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
     }
     if (!start && it >= until) {
       how = kPaused;
-      if (first) beta = 0.0;  // right after a restart the next p is z: pi still holds x
       if (own) {
         const int j = W.i0 + fresh(t);
         A.r[j] = ri;
-        A.p[j] = first ? 0.0 : pi;
+        A.p[j] = pi;
         A.z[j] = zi;
       }
       if (own2) {
         const int e = fresh(t), j = W.i0 + e + bd;
         A.r[j] = rs[e];
-        A.p[j] = first ? 0.0 : ps[e];
+        A.p[j] = ps[e];
         A.z[j] = zs[e];
       }
       break;
@@ -546,15 +548,18 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
 }
 
 // Before each launch: no exchange has happened, nothing is published or aborted.
-__global__ void resident_clear_kernel(ResidentArgs A) {
+__global__ void resident_clear_kernel(ResidentArgs A, int pause) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < kSets * kMaxWords * kMaxBlocks) A.slots[k] = kEmpty;
   if (k < (int)A.B.n) {
     A.zpub[k] = A.zpub[k + A.B.n] = kEmpty;
     if (A.rpub) A.rpub[k] = A.ypub[k] = kEmpty;
   }
-  if (k == 0) *A.abort = 0;
-  if (k == 0) A.out[0] = kNone;
+  if (k == 0) {
+    A.abort[0] = 0;
+    A.abort[1] = (uint32_t)pause;
+    A.out[0] = kNone;
+  }
 }
 
 // rb rows per workgroup, one per thread up to 1024; without FSAI the rows past that are
@@ -620,9 +625,9 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
   A.rb = S.rb;
   A.maxit = maxit;
   A.jacobi = precond == GH_PRECOND_JACOBI;
-  A.pause = kPause;
+  int pause = kPause;
   if (const char *env = std::getenv("GRIDAP_HIP_RESIDENT_PAUSE"))
-    A.pause = std::min(std::max(std::atoi(env), 1), kPause);
+    pause = std::min(std::max(std::atoi(env), 1), kPause);
   A.rtol = rtol;
   A.cp = c.colptr.get();
   A.val = c.nzval.get();
@@ -647,7 +652,7 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
   double h[kOut + 1];
   do {
     hipLaunchKernelGGL(resident_clear_kernel, dim3((unsigned)((clear + 255) / 256)), dim3(256), 0,
-                       c.stream, A);
+                       c.stream, A, pause);
     hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks), dim3((unsigned)S.threads), S.lds, c.stream,
                        A);
     GH_CHECK_HIP(hipGetLastError());
