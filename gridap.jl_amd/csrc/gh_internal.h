@@ -492,12 +492,13 @@ bool pcg_small(Ctx &c, HostCopy &copy, int precond, double rtol, int maxit, doub
                const double *b, unsigned char *ws, gh_solve_stats *st);
 // solve_resident.hip: the whole solve of a box system in one launch of workgroups that stay
 // on their compute units.  state: r, p, z of a solve that takes several launches; pub: 2n
-// words, and n and n with FSAI; ws kResidentWs bytes.  False: not taken (st untouched), x a valid initial guess.
+// words, and n and n with FSAI; ws kResidentWs bytes.  False: not taken or given up (st untouched);
+// x is then the iterate after *done iterations.
 constexpr size_t kResidentWs = 32768;
 bool resident_system(const Ctx &c, const Box &B, int precond);
 bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, double *x,
                   const double *b, double *const (&state)[3], double *const (&pub)[3],
-                  unsigned char *ws, gh_solve_stats *st);
+                  unsigned char *ws, gh_solve_stats *st, int *done);
 // the allocation-free solve: vectors in the library's fixed device array
 void scratch_init(int device);
 void pcg_noalloc(Ctx &c, int precond, const double *b, double *x, double rtol, int maxit,

@@ -1143,17 +1143,21 @@ bool small_system(const Ctx &c, int precond) {
 }
 
 void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st) {
-  // a solve in one launch, timed like the general one; false: not taken
+  // a solve in one launch, timed like the general one; false: not taken.  The time of one
+  // that gave up counts too, and so do its iterations (done).
+  double spent = 0.0;
+  int done = 0;
   auto timed = [&](auto &&solve) {
     float ms = 0.f;
     hipEvent_t *ev = c.timing_events();
     GH_CHECK_HIP(hipEventRecord(ev[0], c.stream));
-    if (!solve()) return false;
+    const bool taken = solve();
     GH_CHECK_HIP(hipEventRecord(ev[1], c.stream));
     GH_CHECK_HIP(hipEventSynchronize(ev[1]));
     GH_CHECK_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
-    st->device_ms = ms;
-    return true;
+    spent += ms;
+    st->device_ms = spent;
+    return taken;
   };
   c.s_small.resize(std::max(kSmallWs, kResidentWs));
   if (small_system(c, precond) && timed([&] {
@@ -1181,10 +1185,12 @@ void pcg_device(Ctx &c, int precond, double rtol, int maxit, gh_solve_stats *st)
   if (c.box && resident_system(c, B, precond) &&
       (precond != GH_PRECOND_FSAI || (c.fsai_built && c.g14.get())) && timed([&] {
         return pcg_resident(c, B, precond, rtol, maxit, V.x, V.b, {V.r, V.p, V.z},
-                            {V.p2, V.r2, V.y}, c.s_small.get(), st);
+                            {V.p2, V.r2, V.y}, c.s_small.get(), st, &done);
       }))
     return;
-  pcg_run(c, V, precond, rtol, maxit, true, true, st);
+  pcg_run(c, V, precond, rtol, maxit - done, true, true, st);
+  st->iterations += done;
+  st->device_ms += spent;
 }
 
 // ---- the solve that allocates nothing (gh_pcg_noalloc) ------------------------------

@@ -548,7 +548,7 @@ __global__ __launch_bounds__(kMaxThreads) void resident_pcg_kernel(const Residen
 }
 
 // Before each launch: no exchange has happened, nothing is published or aborted.
-__global__ void resident_clear_kernel(ResidentArgs A, int pause) {
+__global__ void resident_clear_kernel(ResidentArgs A, int pause, bool abort) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < kSets * kMaxWords * kMaxBlocks) A.slots[k] = kEmpty;
   if (k < (int)A.B.n) {
@@ -556,7 +556,7 @@ __global__ void resident_clear_kernel(ResidentArgs A, int pause) {
     if (A.rpub) A.rpub[k] = A.ypub[k] = kEmpty;
   }
   if (k == 0) {
-    A.abort[0] = 0;
+    A.abort[0] = abort;
     A.abort[1] = (uint32_t)pause;
     A.out[0] = kNone;
   }
@@ -613,7 +613,8 @@ bool resident_system(const Ctx &c, const Box &B, int precond) {
 
 bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, double *x,
                   const double *b, double *const (&state)[3], double *const (&pub)[3],
-                  unsigned char *ws, gh_solve_stats *st) {
+                  unsigned char *ws, gh_solve_stats *st, int *done) {
+  *done = 0;
   static_assert(sizeof(double) * (kOut + 8) + sizeof(uint64_t) * kSets * kMaxWords * kMaxBlocks <=
                     kResidentWs, "workspace");
   Turn turn(c.device);
@@ -648,21 +649,27 @@ bool pcg_resident(Ctx &c, const Box &B, int precond, double rtol, int maxit, dou
                                  : resident_pcg_kernel<false, false>;
   GH_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)S.lds));
+  // for tests: in the launch of this number the last workgroup's rows never come, and whoever
+  // waits finds the abort word set
+  const char *env = std::getenv("GRIDAP_HIP_RESIDENT_GIVE_UP");
+  const int lose = env && S.blocks > 1 ? std::atoi(env) : -1;
   const int64_t clear = std::max<int64_t>(B.n, kSets * kMaxWords * kMaxBlocks);
   double h[kOut + 1];
-  do {
+  for (int launch = 0;; ++launch) {
     hipLaunchKernelGGL(resident_clear_kernel, dim3((unsigned)((clear + 255) / 256)), dim3(256), 0,
-                       c.stream, A, pause);
-    hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks), dim3((unsigned)S.threads), S.lds, c.stream,
-                       A);
+                       c.stream, A, pause, launch == lose);
+    hipLaunchKernelGGL(kern, dim3((unsigned)S.blocks - (launch == lose)),
+                       dim3((unsigned)S.threads), S.lds, c.stream, A);
     GH_CHECK_HIP(hipGetLastError());
     HostCopy copy(c);
     copy.down(h, A.out, sizeof(h));
     uint32_t aborted;
     std::memcpy(&aborted, h + kOut, sizeof(aborted));
     if (aborted || h[0] == kNone) return false;
+    if (h[0] != kPaused) break;
+    *done = (int)h[1];
     A.resume = 1;
-  } while (h[0] == kPaused);
+  }
   c.solve_form = GH_SOLVE_RESIDENT;
   st->iterations = (int)h[1];
   st->converged = h[2] != 0.0;

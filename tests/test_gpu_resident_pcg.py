@@ -168,6 +168,33 @@ def test_pauses_leave_no_trace(part, monkeypatch):
             np.testing.assert_array_equal(x, y)
 
 
+def test_given_up_solves_are_counted(monkeypatch):
+    """A solve whose first, second or fourth launch gives up goes on with the launched kernels
+    from the iterate it had: iterations, limit and time cover both."""
+    print("[gpu-case] resident PCG: given up", flush=True)
+    _, ctx = system((20, 18, 17))
+    for precond in PRECONDS[:2]:  # (FSAI that ends at a limit goes on with Jacobi)
+        for launch, limit in ((0, 5000), (1, 5000), (3, 5000), (0, 9), (1, 9), (3, 9)):
+            done = 2 * launch
+            kw = dict(precond=precond, rtol=1e-10, raise_on_noconv=False)
+            first, _ = resident(ctx, **kw, maxit=done)
+            ref, s1 = launched(monkeypatch, ctx, **kw, x0=first, maxit=limit - done)
+            with monkeypatch.context() as m:
+                m.setenv("GRIDAP_HIP_RESIDENT_PAUSE", "2")
+                m.setenv("GRIDAP_HIP_RESIDENT_GIVE_UP", str(launch))
+                x, st = ctx.pcg(**kw, maxit=limit)
+            assert ctx.solve_form() == _lib.GH_SOLVE_STENCIL
+            assert st.iterations == done + s1.iterations <= limit
+            assert st.converged == s1.converged == (limit == 5000)
+            np.testing.assert_array_equal(x, ref)
+    # 40 launches of an iteration and a read-back each, then one launched iteration
+    _, s1 = launched(monkeypatch, ctx, rtol=1e-10, maxit=1, raise_on_noconv=False)
+    monkeypatch.setenv("GRIDAP_HIP_RESIDENT_PAUSE", "1")
+    monkeypatch.setenv("GRIDAP_HIP_RESIDENT_GIVE_UP", "40")
+    _, st = ctx.pcg(rtol=1e-10, maxit=41, raise_on_noconv=False)
+    assert st.iterations == 41 and st.device_ms > 3 * s1.device_ms
+
+
 def test_two_threads():
     """Two contexts solve at once: whichever finds the device's turn taken runs the launched
     kernels; both are right."""
