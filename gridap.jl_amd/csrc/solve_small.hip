@@ -5,18 +5,19 @@
 // threads runs the solve: start residual, iterations, restarts and the stopping test, one
 // launch and one read-back.  A thread owns rows t, t + 512, ... (R of them); p, x and D^-1
 // live in LDS, r and the first E entries of every row in registers (R E is what the 256
-// registers of 8 waves hold), so consecutive threads read consecutive entries of p (no bank
-// conflicts for lattice numberings) and a row's sum needs no other thread.  The entries
-// past E of a slice of 64 rows are copied once, lane by lane and column as 16 bits, to a
-// workspace from which the wave streams them every iteration (10 bytes an entry,
-// coalesced).  Bound by the LDS reads of p and the three barriers while the matrix fits the
+// registers of 8 waves hold; with R = 8 the ninth entry, the last of a 2-D Q1 row, is in
+// LDS), so consecutive threads read consecutive entries of p (no bank conflicts for lattice
+// numberings) and a row's sum needs no other thread.  The entries past those of a slice of 64
+// rows are copied once, lane by lane and column as 16 bits, to a workspace from which the
+// wave streams them every iteration (10 bytes an entry, coalesced).  Bound by the LDS reads of p and the three barriers while the matrix fits the
 // registers, else by what one compute unit draws from L2.  Microseconds an iteration, start-up
-// included, here and in the general kernels: 2-D Q1 1024 rows 3.2 and 10.2, 4096 rows 4.4
+// included, here and in the general kernels: 2-D Q1 1024 rows 3.2 and 10.2, 4096 rows 3.9
 // and 9.4; 3-D Q1 729 rows 5.7 and 15.7, 1728 rows 7.5 and 16.2; scalar Q2 729 rows 9.8
 // and 14.2.  (1024 threads and sums through LDS permutes took 6.8 for the first: twice the
 // waves at each barrier, half the registers.)  No form spills registers: gh_pcg_noalloc runs
-// them, and the runtime would back scratch with device memory.  (Nine entries with eight rows
-// a thread, 20 registers spilled: 4.3 µs at 2070 rows for 3.8 now, 4.25 at 4096 for 4.4.)
+// them, and the runtime would back scratch with device memory.  (Eight rows a thread at 2070
+// and 4096 rows: nine entries in registers, 20 of them spilled, 4.3 and 4.2 µs; eight, and the
+// ninth streamed, 3.8 and 4.4; the ninth in LDS 3.9 and 3.9.)
 // Both dot products sum in a fixed order: the result is the same every time.
 // One launch runs at most kPause iterations: past them the state goes to the workspace and
 // the next launch takes it up, so that a solve that never ends on its own does not hold the
@@ -69,7 +70,8 @@ __device__ __forceinline__ void sum2(double &a, double &b, double *sh, int &turn
   b = lane_value(v, 31);
 }
 
-template <int R, int E>
+// X: entry E of every row (one more) in LDS too.
+template <int R, int E, int X>
 __global__ __launch_bounds__(kT) void small_pcg_kernel(const SmallArgs A) {
   extern __shared__ __align__(16) double lds[];
   __shared__ double sh[64];
@@ -78,13 +80,15 @@ __global__ __launch_bounds__(kT) void small_pcg_kernel(const SmallArgs A) {
   const int t = threadIdx.x, lane = t & 63, n = A.n;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform values in scalar registers
   double *pl = lds, *xl = lds + R * kT, *dl = lds + 2 * R * kT;
+  double *vx = lds + 3 * R * kT;
+  uint16_t *cx = reinterpret_cast<uint16_t *>(vx + R * kT);
   // matrix: first E entries of each row here, the rest to the stream
   double v[R][E];
   uint32_t col[R][(E + 1) / 2];
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int i = t + k * kT;
-    int len = i < n ? A.cp[i + 1] - A.cp[i] - E : 0;
+    int len = i < n ? A.cp[i + 1] - A.cp[i] - E - X : 0;
     len = max(len, 0);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) len = max(len, __shfl_xor(len, o));
@@ -129,10 +133,19 @@ __global__ __launch_bounds__(kT) void small_pcg_kernel(const SmallArgs A) {
       diag[k] = in && j[e] == i ? v[k][e] : diag[k];
       col[k][e / 2] = e % 2 ? col[k][e / 2] | ((uint32_t)j[e] << 16) : (uint32_t)j[e];
     }
+    if (X) {
+      __builtin_amdgcn_sched_barrier(0);
+      const bool in = p0 + E < p1;
+      const int p = in ? p0 + E : last, jj = A.rv[p];
+      const double a = A.val[p];
+      vx[i] = in ? a : 0.0;
+      cx[i] = (uint16_t)(in ? jj : 0);
+      diag[k] = in && jj == i ? a : diag[k];
+    }
 #pragma unroll 4
     for (int e = 0; e < wd[k]; ++e) {
-      const int p = min(p0 + E + e, last);
-      const bool in = p0 + E + e < p1;
+      const int p = min(p0 + E + X + e, last);
+      const bool in = p0 + E + X + e < p1;
       const int jj = in ? A.rv[p] : 0;
       const double a = in ? A.val[p] : 0.0;
       diag[k] = in && jj == i ? a : diag[k];
@@ -161,6 +174,11 @@ __global__ __launch_bounds__(kT) void small_pcg_kernel(const SmallArgs A) {
       for (int e = 0; e < (E + 1) / 2; ++e) asm volatile("" : "+v"(col[k][e]));
 #pragma unroll
       for (int e = 0; e < E; ++e) s += v[k][e] * pl[(col[k][e / 2] >> (16 * (e % 2))) & 0xffffu];
+      if (X) {
+        int i = t + k * kT;  // its addresses formed here
+        asm volatile("" : "+v"(i));
+        s += vx[i] * pl[cx[i]];
+      }
       int at = base[k] + lane, left = wd[k];
       asm volatile("" : "+v"(at), "+s"(left));
       constexpr int U = 8;
@@ -292,10 +310,10 @@ __global__ __launch_bounds__(kT) void small_pcg_kernel(const SmallArgs A) {
   }
 }
 
-template <int R, int E>
+template <int R, int E, int X = 0>
 void launch(const SmallArgs &A, hipStream_t s) {
-  auto kern = small_pcg_kernel<R, E>;
-  constexpr size_t bytes = sizeof(double) * 3 * R * kT;
+  auto kern = small_pcg_kernel<R, E, X>;
+  constexpr size_t bytes = (sizeof(double) * (3 + X) + sizeof(uint16_t) * X) * R * kT;
   GH_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)bytes));
   hipLaunchKernelGGL(kern, dim3(1), dim3(kT), bytes, s, A);
@@ -330,7 +348,7 @@ bool pcg_small(Ctx &c, HostCopy &copy, int precond, double rtol, int maxit, doub
     if (n <= kT) launch<1, 60>(A, c.stream);
     else if (n <= 2 * kT) launch<2, 32>(A, c.stream);
     else if (n <= 4 * kT) launch<4, 18>(A, c.stream);
-    else launch<8, 8>(A, c.stream);
+    else launch<8, 8, 1>(A, c.stream);
     copy.down(h, A.out, sizeof(h));
     A.resume = 1;
   } while (h[3] == kPaused);

@@ -63,11 +63,11 @@ def system(D, part, order=1, ncomp=1, tags="boundary", seed=0, spread=0.5):
     return G.assemble_matrix(a, assem, U, V), assem.ctx, assem
 
 
-# 2-D Q1 rows of 9, 3-D Q1 of 27 (past the registers' 18 from 1025 rows), scalar Q2 (to 125),
-# vector Q2; 1, 2, 512, 528, 1024, 1056, 2048, 2070, 4032, 4096 rows and past the rule
+# 2-D Q1 rows of 9, 3-D Q1 of 27 (past the registers' 18 from 1025 rows), scalar Q2 (to 125;
+# 2209 rows of up to 25, past the nine kept there), vector Q2; 1, 2, 512, 528, 1024, 1056, 2048, 2070, 4032, 4096 rows and past the rule
 CASES = [(2, (2, 2)), (2, (3, 2)), (2, (33, 17)), (2, (34, 17)), (2, (33, 33)), (2, (33, 34)),
          (2, (65, 33)), (2, (47, 46)), (2, (65, 64)), (2, (65, 65)), (2, (66, 65)),
-         (3, (11, 11, 11)), (3, (9, 14, 13)), (3, (16, 16, 16)), (3, (4, 4, 4), 2),
+         (3, (11, 11, 11)), (3, (9, 14, 13)), (3, (16, 16, 16)), (3, (4, 4, 4), 2), (2, (24, 24), 2),
          (3, (2, 2, 2), 2, 3, ["tag_25"]), (2, (9, 8), 2, 2)]
 
 
