@@ -401,9 +401,10 @@ struct Ctx {
   bool have_mlp = false;
 };
 
-// hostcopy.hip: copies between pageable host arrays and the device through pinned staging,
-// ordered on the context's stream.  up returns with the host array read (the device copy
-// is enqueued), down with the host array written.  finish waits for the stream; a HostCopy
+// hostcopy.hip: copies between pageable host arrays and the device through pinned staging
+// (direct, and where pinning is refused: the runtime's own copies), ordered on the context's
+// stream.  up returns with the host array read (the device copy is enqueued; without staging
+// the array is read by finish at the latest), down with the host array written.  finish waits for the stream; a HostCopy
 // that ends without it waits before its staging is reused.
 class HostCopy {
  public:
@@ -417,7 +418,7 @@ class HostCopy {
   // 0-based 32-bit ids on the device to 1-based 64-bit ids on the host
   void down_ids(int64_t *host, const int32_t *dev, size_t count);
   void finish();
-  // a word of pinned memory that the device may write; null when direct
+  // a word of pinned memory that the device may write; null without staging
   uint64_t *word() const;
   template <class T>
   void up(DBuf<T> &dev, const T *host, size_t count) {

@@ -11,8 +11,9 @@
 // that a context of a single assembly does not pay for pinning; the list holds no device
 // state, any thread and any device's stream may take from it, and a buffer goes back
 // only after the copies that use it have finished.  Calls beyond kMaxIdle at once pin
-// their own buffer and free it.
+// their own buffer and free it.  Where pinning is refused the runtime's own copies take over.
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -29,21 +30,32 @@ constexpr size_t kMaxIdle = 8, kBytes = kSlots * kChunk + 64;  // the slots, a w
 std::mutex g_mu;
 std::vector<char *> g_idle;  // kBytes each
 
+// An idle buffer or a new one; null when pinning is refused (GRIDAP_HIP_PINNED=0: as if).
+char *take_buffer() {
+  const char *env = std::getenv("GRIDAP_HIP_PINNED");
+  if (env && env[0] == '0') return nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_mu);
+    if (!g_idle.empty()) {
+      char *b = g_idle.back();
+      g_idle.pop_back();
+      return b;
+    }
+  }
+  void *b = nullptr;
+  if (hipHostMalloc(&b, kBytes, hipHostMallocCoherent | hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();  // else the next call would report it
+    return nullptr;
+  }
+  return static_cast<char *>(b);
+}
+
 }  // namespace
 
 HostCopy::HostCopy(Ctx &c, bool direct) : s_(c.stream) {
   if (direct) return;
   ev_ = c.copy_events();
-  {
-    std::lock_guard<std::mutex> lock(g_mu);
-    if (!g_idle.empty()) {
-      buf_ = g_idle.back();
-      g_idle.pop_back();
-    }
-  }
-  if (!buf_)
-    GH_CHECK_HIP(hipHostMalloc((void **)&buf_, kBytes,
-                               hipHostMallocCoherent | hipHostMallocPortable));
+  buf_ = take_buffer();
 }
 
 HostCopy::~HostCopy() {
@@ -127,12 +139,18 @@ void HostCopy::down(void *host, const void *dev, size_t bytes) {
 }
 
 void HostCopy::down_ids(int64_t *host, const int32_t *dev, size_t count) {
-  down_chunks(dev, count * sizeof(int32_t), sizeof(int32_t),
-              [&](const char *src, size_t at, size_t n) {
-                const int32_t *in = (const int32_t *)src;
-                int64_t *out = host + at / sizeof(int32_t);
-                for (size_t k = 0; k < n / sizeof(int32_t); ++k) out[k] = int64_t(in[k]) + 1;
-              });
+  auto widen = [&](const char *src, size_t at, size_t n) {
+    const int32_t *in = (const int32_t *)src;
+    int64_t *out = host + at / sizeof(int32_t);
+    for (size_t k = 0; k < n / sizeof(int32_t); ++k) out[k] = int64_t(in[k]) + 1;
+  };
+  if (!buf_) {
+    std::vector<int32_t> ids(count);
+    down(ids.data(), dev, count * sizeof(int32_t));
+    widen((const char *)ids.data(), 0, count * sizeof(int32_t));
+    return;
+  }
+  down_chunks(dev, count * sizeof(int32_t), sizeof(int32_t), widen);
 }
 
 void HostCopy::finish() {

@@ -1,6 +1,6 @@
 """Host arrays through the library's pinned staging: sizes around a chunk (1 MiB) and the
-four chunks in flight, more calls at once than idle buffers are kept, and threads with
-contexts of their own.  The copies move bytes: the comparison is exact."""
+four chunks in flight, more calls at once than idle buffers are kept, threads with
+contexts of their own, and without pinned memory.  The copies move bytes: the comparison is exact."""
 import threading
 
 import numpy as np
@@ -51,6 +51,28 @@ def test_values_round_trip(n):
     inside[cp[1:-1] - 2] = False
     assert np.all(np.diff(rv)[inside] > 0)
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [12, 131_072 * 4 + 4])
+def test_without_pinned_memory(n, monkeypatch):
+    """Pinning refused (GRIDAP_HIP_PINNED=0 answers for the runtime): the same bytes through
+    direct copies, and the solve that is paced by a pinned word reads back instead."""
+    print("[gpu-case] direct copies, %d dofs" % n, flush=True)
+    monkeypatch.setenv("GRIDAP_HIP_SMALL_PCG", "0")
+    got = []
+    for pinned in ("1", "0"):
+        monkeypatch.setenv("GRIDAP_HIP_PINNED", pinned)
+        ctx = lattice(n, n)
+        nz, b = ctx.values_get()
+        nz = nz.copy()
+        cp, rv = ctx.pattern_get()
+        nz[np.flatnonzero(rv - 1 == np.repeat(np.arange(ctx.nfree), np.diff(cp)))] += 1.0
+        ctx.values_set(nz, np.random.default_rng(n).standard_normal(ctx.nfree))
+        x, st = ctx.pcg(rtol=1e-10)
+        got.append((cp, rv, *ctx.values_get(), x, ctx.spmv(x), st.iterations))
+        ctx.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
 
 
 def test_threads_with_their_own_contexts():
