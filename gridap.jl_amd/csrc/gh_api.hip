@@ -166,6 +166,7 @@ int gh_create(gh_ctx **out, int device) {
     delete ctx;
     return e.code;
   }
+  gh::host_copy_context(true);
   *out = ctx;
   return GH_OK;
 }
@@ -177,6 +178,7 @@ int gh_destroy(gh_ctx *ctx) {
   hipStream_t s = ctx->c.stream;
   delete ctx;  // frees device buffers
   (void)hipStreamDestroy(s);
+  gh::host_copy_context(false);
   return GH_OK;
 }
 

@@ -436,6 +436,9 @@ class HostCopy {
   int next_ = 0;
 };
 
+// A context begins or ends: without any, few idle staging buffers are kept.
+void host_copy_context(bool opened);
+
 // pattern.hip
 // contributions: also keep, per nonzero, the ascending list of the (cell, a, b)
 // element entries that sum into it (cstart, perm)

@@ -7,8 +7,9 @@
 // in flight, and the host side of one chunk runs while the next ones are on the link.
 //
 // A staging buffer belongs to one call at a time (HostCopy acquires and returns it).  Idle
-// buffers are kept in a process-wide list of at most kMaxIdle (kMaxIdle x 4 MB pinned), so
-// that a context of a single assembly does not pay for pinning; the list holds no device
+// buffers are kept in a process-wide list of at most kMaxIdle (kMaxIdle x 4 MB pinned), and
+// of kKeepIdle once no context is left, which is what one call takes at most: so a context of
+// a single assembly does not pay for pinning; the list holds no device
 // state, any thread and any device's stream may take from it, and a buffer goes back
 // only after the copies that use it have finished.  Calls beyond kMaxIdle at once pin
 // their own buffer and free it.  Where pinning is refused the runtime's own copies take over.
@@ -25,10 +26,11 @@ namespace {
 
 constexpr size_t kChunk = size_t(1) << 20;
 constexpr int kSlots = 4;
-constexpr size_t kMaxIdle = 8, kBytes = kSlots * kChunk + 64;  // the slots, a word
+constexpr size_t kMaxIdle = 8, kKeepIdle = 2, kBytes = kSlots * kChunk + 64;  // the slots, a word
 
 std::mutex g_mu;
 std::vector<char *> g_idle;  // kBytes each
+int g_contexts = 0;
 
 // An idle buffer or a new one; null when pinning is refused (GRIDAP_HIP_PINNED=0: as if).
 char *take_buffer() {
@@ -51,6 +53,13 @@ char *take_buffer() {
 }
 
 }  // namespace
+
+void host_copy_context(bool opened) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  g_contexts += opened ? 1 : -1;
+  for (; g_contexts == 0 && g_idle.size() > kKeepIdle; g_idle.pop_back())
+    (void)hipHostFree(g_idle.back());
+}
 
 HostCopy::HostCopy(Ctx &c, bool direct) : s_(c.stream) {
   if (direct) return;
