@@ -1172,6 +1172,9 @@ void fsai_forward_build(Ctx &c, bool inference, bool solver) {
                        c.params_bf16.get(), C, c.yo.get());
   } else {
     const unsigned grid = (unsigned)std::min((C + kTrainCells - 1) / kTrainCells, 2 * kTrainGrid);
+    GH_CHECK_HIP(hipFuncSetAttribute((const void *)mlp_train_fwd,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)sizeof(TrainLds)));  // past 64 KB
     hipLaunchKernelGGL(mlp_train_fwd, dim3(grid), dim3(256), sizeof(TrainLds), s, c.feat.get(),
                        c.params_bf16.get(), C, c.yo.get());
   }
