@@ -373,8 +373,8 @@ struct Ctx {
   // box lattice: the free dofs are all nodes of a box of box_m[0] x box_m[1] x box_m[2]
   // lattice nodes, numbered in node order (Q1, every boundary node outside the box
   // Dirichlet), so A is a 27-point stencil in dof space and PCG runs the stencil
-  // kernels: A as 27 offset arrays of N values (a27, zero outside the box) and G as
-  // 14 offset arrays (g14, lower offsets in ascending order), no column indices
+  // kernels: A (a27: its lower half, zero outside the box) and G (g14) as 14 arrays of N
+  // values, lower offsets in ascending order, no column indices
   bool box = false;
   int64_t box_m[3] = {0, 0, 0};
   DBuf<double> a27;

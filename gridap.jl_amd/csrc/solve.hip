@@ -614,8 +614,8 @@ __global__ void diag_inv_box_kernel(int64_t n, const double *__restrict__ a27,
 // the 14 arrays.  All 27 coefficient loads of a row are independent and issued together,
 // ahead of the reduction that gives β.  A row used to load coefficient and vector inside
 // the branch of each neighbour, 27 round trips one after the other: spmv_dir 22.5 µs at
-// 64³ and 181 µs at 128³ (latency), now 10.2 and 70 µs (bandwidth: 294 MB, 4.2 TB/s; with
-// the mirrored entries that miss L2 490 MB, 7 TB/s);
+// 64³ and 181 µs at 128³ (latency), now 10.2 and 66 µs (bandwidth: 294 MB, 4.5 TB/s; with
+// the mirrored entries that miss L2 380 MB, 5.7 TB/s);
 // update_lower 10.6 -> 7.8 µs, upper_rz 6.5 -> 4.8 µs at 64³.
 // Each XCD sweeps a contiguous slab of the tiles in order, so the mirrored coefficients
 // of the next plane are in its L2 when the plane itself reads them.
@@ -1126,7 +1126,9 @@ void pcg_run(Ctx &c, const PcgBufs &V, int precond, double rtol, int maxit, bool
 }  // namespace
 
 // Systems that the one-workgroup solve takes: at most 4096 rows, 40,960 entries and 64
-// entries a row on average, boxes 1536 rows.  Past the entries one compute unit streams too
+// entries a row on average, boxes 1536 rows.  The rows are what a workgroup holds and not
+// where it stops winning (4096 rows 3.9 µs an iteration and 9.4 in the general kernels: past
+// them an iteration takes more than twice as long).  Past the entries one compute unit streams too
 // much of the matrix (µs an iteration: 3-D Q1 39,304 entries 7.5, 50,653 14.6, 64,000 15.6,
 // where the general kernels take 10 to 12); with longer rows a thread's serial share is too
 // long (one workgroup and general kernels: 3-D Q2 of 41 a row 9.8 and 12.2; vector Q2 of

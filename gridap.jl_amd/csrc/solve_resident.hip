@@ -26,17 +26,21 @@
 // On a (re)start, where there is no E1 between, the vectors are published with a wait
 // and read past the exchange instead.
 //
-// Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.1, 31³
-// 11.9 and 6.8; FSAI 25.3 and 19.3, 17.5 and 12.4; rows past one a thread, in LDS: 65³ 19.6
-// and 16.2, 70³ 20.6 and 17.2.  (Barriers for the published vectors too: 10.7, 7.6, 22.6,
+// Microseconds an iteration, launched kernels and here: Jacobi 63³ rows 17.1 and 10.2, 31³
+// 11.9 and 6.9; FSAI 25.3 and 18.4, 17.5 and 12.0; rows past one a thread, in LDS: 65x64x65
+// 19.6 and 15.8, 70³ 20.6 and 16.8.  (Barriers for the published vectors too: 10.7, 7.6, 22.6,
 // 16.0.)  What bounds it: the trips through the fabric, 3 to 4 µs an exchange or published
 // vector with 245 workgroups, 2 with 14.  Hence the largest workgroups that fit, 512 rows
-// at least (31³ with barriers: 256 rows 8.3, 512 7.1, 1024 7.3).
+// at least (31³ with barriers: 256 rows 8.3, 512 7.1, 1024 7.3).  16 waves leave a thread 128
+// registers, of which the coefficients take 54: 28 values spill (FSAI 42, rows in LDS 88) to 20,
+// 60 and 200 bytes of scratch.
 //
 // Every wait ends: a workgroup that waits longer than kArrive for the first exchange (some
 // workgroups are not on the device: other work holds it) or kLost for a later one sets the
-// abort word, which every waiting workgroup polls, and the general kernels solve the
-// system.  One launch runs at most kPause iterations.
+// abort word, which every waiting workgroup polls, and the launched kernels go on from the
+// last iterate that reached memory.  Those group the dot products differently, so the last
+// bits of a solution depend on which form ended it.  One launch runs at most kPause
+// iterations, and holds the compute units that long (21 ms at 63³, 38 ms with FSAI).
 #include <algorithm>
 #include <atomic>
 #include <cmath>

@@ -321,11 +321,12 @@ int gh_pcg(gh_ctx *ctx, int precond, const double *b, double *x, double rtol, in
 /* gh_pcg without any device allocation.  No counterpart in Gridap: for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Jacobi (GH_PRECOND_JACOBI) or no preconditioner,
- * the general CSR kernels (small systems: one workgroup), nfree <= GH_NOALLOC_MAX_N.  Its vectors live in one fixed
- * device array of the library (9 x GH_NOALLOC_MAX_N doubles plus partial sums, about
- * 19 MB), which every GPU the library runs on holds until the process ends; all calls
- * on one GPU share it, so calls that overlap on one GPU race.  Same results as gh_pcg
- * with the same preconditioner on the CSR kernels (GRIDAP_HIP_STENCIL_PCG=0);
+ * the general CSR kernels (small systems: one workgroup), nfree <= GH_NOALLOC_MAX_N.  Its
+ * vectors live in one fixed device array of the library (9 x GH_NOALLOC_MAX_N doubles plus
+ * partial sums, about 19 MB), which every GPU the library runs on holds until the process
+ * ends; its kernels use no scratch memory; all calls on one GPU share the array, so calls that
+ * overlap on one GPU race.  The same bits as gh_pcg with the same preconditioner where both
+ * take the same form (gh_solve_form_get), as they do with GRIDAP_HIP_STENCIL_PCG=0;
  * stats->device_ms is the host wall time of the call. */
 #define GH_NOALLOC_MAX_N 262144
 int gh_pcg_noalloc(gh_ctx *ctx, int precond, const double *b, double *x, double rtol,

@@ -249,9 +249,9 @@ def test_trained_network_beats_jacobi_on_heldout():
 
 
 def test_stencil_pcg_matches_general_pcg(case, monkeypatch):
-    """On a box lattice PCG runs stencil kernels (A as 27 offset arrays, G as 14, Gᵀ from
-    mirrored offsets); GRIDAP_HIP_STENCIL_PCG=0 runs the general CSR / 16-slot kernels on
-    the same system.  Both must reach the same solution with the same iteration count
+    """On a box lattice PCG runs stencil kernels (A and G as 14 offset arrays, A's upper half
+    and Gᵀ from mirrored offsets); GRIDAP_HIP_STENCIL_PCG=0 runs the general CSR / 16-slot
+    kernels on the same system.  Both must reach the same solution with the same iteration count
     (up to rounding: the sums run in another order)."""
     announce("fsai: stencil PCG vs general PCG (Jacobi and FSAI)")
     ctx = case["ctx"]
