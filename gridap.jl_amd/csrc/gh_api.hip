@@ -2,6 +2,7 @@
 // status-code boundary.  Compute lives in pattern.hip, assemble.hip, solve.hip.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 
 #include "gh_internal.h"
@@ -154,6 +155,8 @@ int gh_create(gh_ctx **out, int device) {
   gh_ctx *ctx = new (std::nothrow) gh_ctx();
   if (!ctx) return GH_ERR_OOM;
   ctx->c.device = device;
+  const char *pinned = std::getenv("GRIDAP_HIP_PINNED");
+  ctx->c.pinned = !(pinned && pinned[0] == '0');
   if (hipSetDevice(device) != hipSuccess ||
       hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking) != hipSuccess) {
     delete ctx;

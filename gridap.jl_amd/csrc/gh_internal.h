@@ -209,6 +209,7 @@ struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
+  bool pinned = true;  // host copies through pinned staging (GRIDAP_HIP_PINNED)
   Events events;
   hipEvent_t *copy_events() { return events.get(0, Events::kCopy, hipEventDisableTiming); }
   hipEvent_t *timing_events() { return events.get(Events::kCopy, 2, hipEventDefault); }

@@ -14,7 +14,6 @@
 // only after the copies that use it have finished.  Calls beyond kMaxIdle at once pin
 // their own buffer and free it.  Where pinning is refused the runtime's own copies take over.
 #include <algorithm>
-#include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -32,10 +31,8 @@ std::mutex g_mu;
 std::vector<char *> g_idle;  // kBytes each
 int g_contexts = 0;
 
-// An idle buffer or a new one; null when pinning is refused (GRIDAP_HIP_PINNED=0: as if).
+// An idle buffer or a new one; null when pinning is refused.
 char *take_buffer() {
-  const char *env = std::getenv("GRIDAP_HIP_PINNED");
-  if (env && env[0] == '0') return nullptr;
   {
     std::lock_guard<std::mutex> lock(g_mu);
     if (!g_idle.empty()) {
@@ -62,7 +59,7 @@ void host_copy_context(bool opened) {
 }
 
 HostCopy::HostCopy(Ctx &c, bool direct) : s_(c.stream) {
-  if (direct) return;
+  if (direct || !c.pinned) return;
   ev_ = c.copy_events();
   buf_ = take_buffer();
 }
